@@ -175,8 +175,10 @@ void decode_chunk_kernel(sisa_decode_args a) {
 }
 
 // out[row] = sum_c exp(m_c - M) o_c / sum_c exp(m_c - M) l_c. One wave per row: chunk c's max and sum are read by
-// lane c mod 64, its output row by lane = feature, chunks in order, 8 row loads issued ahead of their FMAs.
-__global__ __launch_bounds__(64) void decode_combine_kernel(sisa_decode_args a, int nchunk) {
+// lane c mod 64, its output row by lane = feature, chunks in order, 8 row loads issued ahead of their FMAs. The result
+// is rounded to TO (fp32, or the compute dtype for a layer step, whose next product reads it).
+template <class TO>
+__global__ __launch_bounds__(64) void decode_combine_kernel(sisa_decode_args a, TO* out, int nchunk) {
     const int row = blockIdx.x, lane = threadIdx.x;
     const float* part = a.workspace + (int64_t)row * nchunk * PART;
     float M = -__builtin_inff();
@@ -201,17 +203,17 @@ __global__ __launch_bounds__(64) void decode_combine_kernel(sisa_decode_args a, 
         }
     }
     L = wave_sum(L);
-    a.out[(int64_t)row * DH + lane] = o / L;
+    out[(int64_t)row * DH + lane] = cvt<TO>(o / L);
 }
 
-template <class T>
-int launch_decode(const sisa_decode_args* a, hipStream_t st) {
+template <class T, class TO>
+int launch_decode(const sisa_decode_args* a, TO* out, hipStream_t st) {
     const int nchunk = (int)sisa::cdiv(a->N, KCH);
     const int rows = a->B * a->H * a->M;
     decode_chunk_kernel<T><<<dim3((unsigned)nchunk, (unsigned)rows), 64 * DW, 0, st>>>(*a);
     const int rc = sisa::launch_status("sisa_decode_attn");
     if (rc) return rc;
-    decode_combine_kernel<<<(unsigned)rows, 64, 0, st>>>(*a, nchunk);
+    decode_combine_kernel<TO><<<(unsigned)rows, 64, 0, st>>>(*a, out, nchunk);
     return sisa::launch_status("sisa_decode_attn (combine)");
 }
 
@@ -222,6 +224,17 @@ bool rows_ok(const sisa_view& v, int dtype, int width) {
 }
 
 }  // namespace
+
+namespace sisa {
+namespace detail {
+// The decode attention of 16-bit operands with the result rounded to their dtype, (B,H,M,64) contiguous (checked by
+// the caller: sisa_step).
+__attribute__((visibility("hidden"))) int decode_attn_out16(const sisa_decode_args* a, void* out, hipStream_t st) {
+    return a->dtype == SISA_BF16 ? launch_decode<__bf16>(a, (__bf16*)out, st)
+                                 : launch_decode<_Float16>(a, (_Float16*)out, st);
+}
+}  // namespace detail
+}  // namespace sisa
 
 extern "C" int64_t sisa_decode_workspace_bytes(int32_t B, int32_t H, int32_t M, int32_t N) {
     return (int64_t)B * H * M * sisa::cdiv(N, KCH) * PART * (int64_t)sizeof(float);
@@ -244,8 +257,8 @@ extern "C" int sisa_decode_attn(const sisa_decode_args* a, void* stream) {
     SISA_REQUIRE((a->fq.ptr == nullptr) == (a->fk.ptr == nullptr), "sisa_decode_attn: fq and fk given together");
     hipStream_t st = (hipStream_t)stream;
     switch (a->dtype) {
-        case SISA_BF16: return launch_decode<__bf16>(a, st);
-        case SISA_F16: return launch_decode<_Float16>(a, st);
-        default: return launch_decode<float>(a, st);
+        case SISA_BF16: return launch_decode<__bf16>(a, a->out, st);
+        case SISA_F16: return launch_decode<_Float16>(a, a->out, st);
+        default: return launch_decode<float>(a, a->out, st);
     }
 }

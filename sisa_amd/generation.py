@@ -3,7 +3,8 @@
 Per head and cached position a SISA layer keeps, besides ``k`` and ``v``, the rotated state write vector ``b~``
 (``d_state`` values) and the cumulative decay ``g`` and forget ``F`` values; the running phase ``Phi`` is kept for the
 last position only. A new token extends ``g``, ``F`` and ``Phi`` in float32 and attends to the whole cache with the
-exact score (on the GPU through the HIP decode kernel, :mod:`sisa_amd.kernels.decode`).
+exact score (on the GPU through the HIP decode kernel, :mod:`sisa_amd.kernels.decode`, or, for a single new position
+of a 16-bit model, together with the rest of its layer, :mod:`sisa_amd.kernels.step`).
 
 The cache is a set of preallocated slabs per layer, ``(B, H, capacity, .)``, filled front to back: a decode step
 writes its rows in place and the layer state handed to the attention is a view of the filled prefix, so a step costs
@@ -89,20 +90,28 @@ class SISACache:
             bufs = new if old is None else {n: torch.cat([getattr(old, n), t], 2) for n, t in new.items()}
             slab = _Slab(bufs, bufs["k"].shape[2], phi)
         else:
-            filled = 0 if slab is None else slab.filled
-            need = filled + n_new
-            if slab is None or need > slab.capacity:
-                room = max(need, self.capacity or 0, 2 * slab.capacity if slab is not None else 0)
-                grown = {n: t.new_empty(t.shape[:2] + (room,) + t.shape[3:]) for n, t in new.items()}
-                if slab is not None:
-                    for n, t in grown.items():
-                        t[:, :, :filled].copy_(slab.buffers[n][:, :, :filled])
-                slab = _Slab(grown, filled, phi)
+            slab = self.room(layer_idx, n_new, new, phi)
+            filled, need = slab.filled, slab.filled + n_new
             for n, t in new.items():
                 slab.buffers[n][:, :, filled:need].copy_(t)
             slab.filled, slab.phi = need, phi
         self._slabs[layer_idx] = slab
         return slab.state()
+
+    def room(self, layer_idx: int, n_new: int, like: dict[str, Tensor], phi: Tensor) -> _Slab:
+        """The layer's slab with space for ``n_new`` more positions after its filled ones; made, or grown by doubling,
+        where it lacks that. ``like``: tensors with the batch and head sizes, widths and dtypes of new buffers."""
+        slab = self._slabs.get(layer_idx)
+        filled = 0 if slab is None else slab.filled
+        need = filled + n_new
+        if slab is None or need > slab.capacity:
+            room = max(need, self.capacity or 0, 2 * slab.capacity if slab is not None else 0)
+            grown = {n: t.new_empty(t.shape[:2] + (room,) + t.shape[3:]) for n, t in like.items()}
+            if slab is not None:
+                for n, t in grown.items():
+                    t[:, :, :filled].copy_(slab.buffers[n][:, :, :filled])
+            slab = self._slabs[layer_idx] = _Slab(grown, filled, phi)
+        return slab
 
     @property
     def seq_len(self) -> int:

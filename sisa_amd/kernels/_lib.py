@@ -119,6 +119,23 @@ class LmceTrainArgs(Structure):
                 ("dw_accumulate", c_int32), ("dx_splits", c_int32), ("workspace", c_void_p)]
 
 
+class StepArgs(Structure):
+    _fields_ = [("B", c_int32), ("H", c_int32), ("D", c_int32), ("FF", c_int32), ("dtype", c_int32), ("pos", c_int32),
+                ("eps_attn", c_float), ("eps_ffn", c_float), ("x", c_void_p), ("sx", c_int64), ("res", c_void_p),
+                *((n, c_void_p) for n in ("attn_norm", "w_q", "w_k", "w_v", "w_b", "w_c", "w_theta", "w_alpha",
+                                          "b_alpha", "w_forget", "b_forget", "w_o", "ffn_norm", "w_gate", "w_up",
+                                          "w_down", "lambda_raw")),
+                ("k", View), ("v", View), ("b", View), ("g", View), ("f", View), ("phi_in", c_void_p),
+                ("phi_out", c_void_p), ("h", c_void_p), ("ffn", c_void_p), ("workspace", c_void_p)]
+
+
+class CacheFillArgs(Structure):
+    _fields_ = [("B", c_int32), ("H", c_int32), ("L", c_int32), ("dtype", c_int32), ("proj", c_void_p),
+                ("s_b", c_int64), ("s_l", c_int64), ("col_k", c_int32), ("col_v", c_int32), ("br", c_void_p),
+                ("gs", c_void_p), ("fs", c_void_p), ("totals", c_void_p), ("k", View), ("v", View), ("b", View),
+                ("g", View), ("f", View), ("phi", c_void_p)]
+
+
 class Round16Args(Structure):
     _fields_ = [("n", c_int64), ("dtype", c_int32), ("x", c_void_p), ("y", c_void_p), ("back", c_void_p)]
 
@@ -157,6 +174,13 @@ SIGNATURES = {
     "sisa_round16": ([POINTER(Round16Args), c_void_p], c_int),
 }
 
+# the generation entry points (include/sisa_hip_step.h)
+STEP_SIGNATURES = {
+    "sisa_step_workspace_bytes": ([c_int32, c_int32, c_int32, c_int32, c_int32], c_int64),
+    "sisa_step": ([POINTER(StepArgs), c_void_p], c_int),
+    "sisa_cache_fill": ([POINTER(CacheFillArgs), c_void_p], c_int),
+}
+
 _LOCK = threading.Lock()
 _LIB = None
 
@@ -172,7 +196,7 @@ def load() -> ctypes.CDLL:
         if not os.path.exists(LIB_PATH):
             raise RuntimeError(f"SISA HIP library not built: {LIB_PATH} is missing (run sisa_amd.build.build())")
         lib = ctypes.CDLL(LIB_PATH)
-        for name, (argtypes, restype) in SIGNATURES.items():
+        for name, (argtypes, restype) in (*SIGNATURES.items(), *STEP_SIGNATURES.items()):
             fn = getattr(lib, name)
             fn.argtypes = argtypes
             fn.restype = restype

@@ -1,0 +1,95 @@
+"""Generation on the HIP kernels of csrc/step.hip: one new token of every row through a whole decoder layer with a
+filled cache (``sisa_step``, seven launches behind one C call), and the filling of a layer's cache after a prefill on
+the fused route (``sisa_cache_fill``). The module path these stand in for is src/sisa/modeling.py:171-199, 224-238,
+288-291; there a layer's step is about seventy torch kernels, whose launches cost four times what they compute.
+
+Both write into the cache's slabs in place and are for inference: the callers check that no gradient is wanted and
+that nothing observes the modules they pass by (:func:`unobserved`, :func:`step_weights`).
+"""
+from __future__ import annotations
+
+import torch
+from torch import Tensor, nn
+from torch.nn.modules import module as _nn_module
+
+from ..config import HIP_D_HEAD, HIP_D_STATE
+from . import _lib
+from . import attention as A
+from . import fused_prep as P
+
+__all__ = ["unobserved", "plain", "step_weights", "layer_step", "prefill", "MAX_ROWS", "MAX_WIDTH"]
+
+MAX_ROWS, MAX_WIDTH = 64, 1024          # SISA_STEP_MAX_ROWS, SISA_STEP_MAX_D
+
+
+def unobserved(x: Tensor) -> bool:
+    """Whether nothing follows the torch operations on ``x``: a plain tensor, no gradient or forward-mode level, no
+    compile trace, function transform, dispatch or function mode, and no global module hooks."""
+    return (type(x) is Tensor and not torch.is_grad_enabled() and not torch.compiler.is_compiling()
+            and torch.autograd.forward_ad._current_level < 0
+            and torch._C._functorch.peek_interpreter_stack() is None
+            and not torch._C._len_torch_dispatch_stack() and not torch._C._len_torch_function_stack()
+            and not _nn_module._global_forward_hooks and not _nn_module._global_forward_pre_hooks)
+
+
+def plain(module: nn.Module, kind: type) -> bool:
+    """A module of exactly this class whose call is its class's ``forward``: no hooks, no patched method."""
+    return (type(module) is kind and not module._forward_hooks and not module._forward_pre_hooks
+            and "forward" not in module.__dict__)
+
+
+def step_weights(table, x: Tensor) -> list[int] | None:
+    """Addresses of the parameters of ``table``, an iterable of (parameter, shape): each a plain contiguous parameter
+    of ``x``'s dtype on its device with that shape and, when it is a matrix, 16-byte aligned. None otherwise."""
+    dtype, device, out = x.dtype, x.get_device(), []
+    for p, shape in table:
+        if type(p) is not nn.Parameter or p.dtype is not dtype or p.shape != shape or p.get_device() != device \
+                or not p.is_contiguous():
+            return None
+        address = p.data_ptr()
+        if address % 16 and (len(shape) == 2 or shape[0] % 8 == 0):
+            return None
+        out.append(address)
+    return out
+
+
+def layer_step(x: Tensor, res: Tensor | None, weights: list[int], lambda_raw: Tensor, eps: tuple[float, float],
+               d_ff: int, slab, phi: Tensor) -> tuple[Tensor, Tensor, Tensor]:
+    """The new position of ``x`` ``(B, 1, D)`` (plus ``res``, added first) through a layer; ``weights`` in the order of
+    ``sisa_step_args`` (attn_norm .. w_down). Writes the position into ``slab`` (room for it is the caller's care) and
+    returns ``(h, ffn, phi)``: the residual stream after the attention, the FFN output still to be added to it, and
+    the phase at the new position."""
+    B, _, D = x.shape
+    H, pos = D // HIP_D_HEAD, slab.filled
+    h, ffn = torch.empty((2, B, 1, D), device=x.device, dtype=x.dtype).unbind(0)
+    phi_out = torch.empty((B, H, HIP_D_STATE // 2), device=x.device, dtype=torch.float32)
+    lib = _lib.load()
+    ws = torch.empty((lib.sisa_step_workspace_bytes(B, H, D, d_ff, pos + 1),), device=x.device, dtype=torch.uint8)
+    buf = slab.buffers
+    args = _lib.StepArgs(B, H, D, d_ff, _lib.dtype_code(x.dtype), pos, *eps, x.data_ptr(), x.stride(0),
+                         None if res is None else res.data_ptr(), *weights, lambda_raw.data_ptr(),
+                         *(_lib.view(buf[n]) for n in ("k", "v", "b", "g", "fgate")), phi.data_ptr(),
+                         phi_out.data_ptr(), h.data_ptr(), ffn.data_ptr(), ws.data_ptr())
+    _lib.call("sisa_step", args, x)
+    return h, ffn, phi_out
+
+
+def prefill(proj: Tensor, z: Tensor, lam: Tensor, n_head: int, cache, layer_idx: int) -> Tensor:
+    """The fused layer core on a prompt that also fills the layer's (empty) cache: ``proj`` (B, L, NPAD), ``z``
+    (B, L, H) as :func:`sisa_amd.kernels.fused_prep.sisa_fused` takes them. The check of ``g`` is the unfused route's,
+    which a prefill ran before. Returns y (B, L, H*64). Inference only."""
+    B, L, _ = proj.shape
+    lay = P.fused_layout(n_head)
+    pp = P.prep_forward(proj, z, n_head)
+    q, k, v = (P._heads(proj, lay[n], n_head) for n in ("Q", "K", "V"))
+    c, b = pp.state_views()
+    fw = A.attn_forward(q, k, v, c, b, pp.g, lam, pp.f)
+    phi = torch.empty((B, n_head, HIP_D_STATE // 2), device=proj.device, dtype=torch.float32)
+    slab = cache.room(layer_idx, L, dict(k=k, v=v, b=b, g=pp.g, fgate=pp.f), phi)
+    buf = slab.buffers
+    _lib.call("sisa_cache_fill", _lib.CacheFillArgs(
+        B, n_head, L, _lib.dtype_code(proj.dtype), proj.data_ptr(), proj.stride(0), proj.stride(1), lay["K"], lay["V"],
+        pp.br.data_ptr(), pp.g.data_ptr(), pp.f.data_ptr(), pp.totals.data_ptr(),
+        *(_lib.view(buf[n]) for n in ("k", "v", "b", "g", "fgate")), phi.data_ptr()), proj)
+    slab.filled = L
+    return fw.o.transpose(1, 2).flatten(2)

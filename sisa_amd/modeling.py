@@ -28,7 +28,7 @@ from torch import Tensor
 from torch.utils.checkpoint import checkpoint
 
 from . import backends
-from .config import SISAConfig
+from .config import HIP_D_STATE, SISAConfig
 from .functional import attend_block, autocast_disabled, rotate_pairs, sisa_attention, working_dtype
 
 if TYPE_CHECKING:  # pragma: no cover
@@ -227,10 +227,10 @@ class SISAAttention(nn.Module):
                                     self.W_C.weight, self.theta_proj.weight, self.alpha_proj.weight,
                                     self.alpha_proj.bias)
 
-    def _forward_fused(self, x: Tensor, z: Tensor | None = None) -> Tensor:
+    def _forward_fused(self, x: Tensor, z: Tensor | None = None, cache: "SISACache | None" = None) -> Tensor:
         """The fused route. ``z``: forget-gate logits already produced by the decoder block's norm kernel; with it
         the projections use the HIP weight-gradient GEMM path of the block, without it (the sublayer called on its
-        own) plain ``F.linear``."""
+        own) plain ``F.linear``. ``cache`` (with ``z``, inference): also fill this layer's empty entry."""
         from .kernels.fused_prep import fused_layout, sisa_fused
 
         weight, bias = self._fused_weights()
@@ -238,6 +238,11 @@ class SISAAttention(nn.Module):
         if z is None:
             y = sisa_fused(F.linear(x, weight, bias), self._forget_logits(x), self.lam(), n_head)
             return self.W_O(y)                         # y: (B, L, d), heads side by side
+        if cache is not None:
+            from .kernels.step import prefill
+
+            return F.linear(prefill(F.linear(x, weight, bias), z, self.lam(), n_head, cache, self.layer_idx),
+                            self.W_O.weight)
         a0 = fused_layout(n_head)["A"]                 # the bias is a parameter on the alpha columns only
         y = sisa_fused(_linear(x, weight, bias, (a0, a0 + n_head)), z, self.lam(), n_head)
         return _linear(y, self.W_O.weight)
@@ -315,7 +320,62 @@ class SISABlock(nn.Module):
             return False
         return backends.select_impl(self.config.attn_impl, x, self.config) == "hip_fused"
 
-    def _forward_hip(self, x: Tensor, res: Tensor | None = None, defer: bool = False):
+    def _plain(self) -> bool:
+        """Every module a cached HIP route passes by is the class this file builds it from, without hooks."""
+        from .kernels.step import plain
+
+        at, ffn = self.attn, self.ffn
+        return (plain(self, SISABlock) and plain(at, SISAAttention) and plain(ffn, SwiGLU) and plain(self.attn_norm, RMSNorm)
+                and plain(self.ffn_norm, RMSNorm)
+                and all(plain(lin, nn.Linear) for lin in (at.W_Q, at.W_K, at.W_V, at.W_O, at.W_B, at.W_C, at.theta_proj,
+                                                          at.alpha_proj, at.forget_proj, ffn.w_gate, ffn.w_up,
+                                                          ffn.w_down)))
+
+    def _forward_cached_hip(self, x: Tensor, res: Tensor | None, cache: "SISACache"):
+        """Generation on HIP kernels, or None where it does not apply. A prompt (empty cache entry) takes
+        :meth:`_forward_hip` with the cache filled from the fused projections; one new position of at most 64 rows of
+        a 16-bit model takes ``sisa_step``. Both return ``(h, f)`` as :meth:`_forward_hip` with ``defer``. Only for
+        inference with nothing watching the modules in between: other calls take the module path."""
+        from .generation import SISACache
+        from .kernels import step
+
+        if x.device.type != "cuda" or type(cache) is not SISACache or not step.unobserved(x) \
+                or not self._fused_norm_ok(x) or not self._plain():
+            return None
+        at, ffn = self.attn, self.ffn
+        if at.alpha_proj.bias is None or at.forget_proj.bias is None:
+            return None
+        slab = cache._slabs.get(at.layer_idx)
+        if slab is None:
+            return self._forward_hip(x, res, defer=True, cache=cache)
+        B, L, D = x.shape
+        H, d_ff = self.config.n_head, ffn.w_gate.out_features
+        if L != 1 or B > step.MAX_ROWS or D > step.MAX_WIDTH or slab.filled < 1 \
+                or torch.is_autocast_enabled("cuda") or x.dtype not in _LOW_PRECISION or x.stride(-1) != 1 \
+                or x.stride(0) % 8 or x.data_ptr() % 16 or at.lambda_raw.dtype != torch.float32 \
+                or at.lambda_raw.shape != (H,) or at.lambda_raw.get_device() != x.get_device():
+            return None
+        buf = slab.buffers
+        if buf["k"].dtype != x.dtype or buf["k"].shape[:2] != (B, H) or buf["k"].get_device() != x.get_device():
+            return None
+        s = HIP_D_STATE
+        weights = step.step_weights(
+            ((self.attn_norm.weight, (D,)), (at.W_Q.weight, (D, D)), (at.W_K.weight, (D, D)),
+             (at.W_V.weight, (D, D)), (at.W_B.weight, (H * s, D)), (at.W_C.weight, (H * s, D)),
+             (at.theta_proj.weight, (H * s // 2, D)), (at.alpha_proj.weight, (H, D)), (at.alpha_proj.bias, (H,)),
+             (at.forget_proj.weight, (H, D)), (at.forget_proj.bias, (H,)), (at.W_O.weight, (D, D)),
+             (self.ffn_norm.weight, (D,)), (ffn.w_gate.weight, (d_ff, D)), (ffn.w_up.weight, (d_ff, D)),
+             (ffn.w_down.weight, (D, d_ff))), x)
+        if weights is None:
+            return None
+        slab = cache.room(at.layer_idx, 1, buf, slab.phi)
+        h, f, phi = step.layer_step(x, res, weights, at.lambda_raw.detach().contiguous(),
+                                    (self.attn_norm.eps, self.ffn_norm.eps), d_ff, slab, slab.phi.contiguous())
+        slab.filled, slab.phi = slab.filled + 1, phi
+        return h, f
+
+    def _forward_hip(self, x: Tensor, res: Tensor | None = None, defer: bool = False,
+                     cache: "SISACache | None" = None):
         """The block on the HIP kernels: the attention norm and the fp32 forget-gate projection in one pass that
         also emits the normalised rows in the dtype of the projection GEMM (the reference casts them under autocast),
         the fused attention sublayer, the residual add and the FFN norm in one pass, SwiGLU.
@@ -335,7 +395,7 @@ class SISABlock(nn.Module):
             if res is not None:
                 x = x + res
             n, z = rms_norm_forget_hip(x, nw, eps, wf, bf, out_dtype)
-        a = at._forward_fused(n, z)
+        a = at._forward_fused(n, z, cache)
         if a.dtype == out_dtype and a.shape == x.shape:   # residual add fused into the FFN norm
             x, m = rms_norm_add_hip(x, a, self.ffn_norm.weight, self.ffn_norm.eps, out_dtype)
         else:
@@ -349,6 +409,9 @@ class SISABlock(nn.Module):
     def forward(self, x: Tensor, cache: "SISACache | None" = None) -> Tensor:
         if cache is None and self._fused_norm_ok(x):
             return self._forward_hip(x)
+        done = None if cache is None else self._forward_cached_hip(x, None, cache)
+        if done is not None:
+            return done[0] if done[1] is None else done[0] + done[1]
         h = x + self.attn(self.attn_norm(x), cache=cache)
         return h + self.ffn(self.ffn_norm(h))
 
@@ -420,6 +483,10 @@ class SISAModel(nn.Module):
         for block in self.layers:
             if DEFER_RESIDUAL and not recompute and cache is None and block._fused_norm_ok(x):
                 x, pending = block._forward_hip(x, pending, defer=True)
+                continue
+            done = None if cache is None else block._forward_cached_hip(x, pending, cache)
+            if done is not None:
+                x, pending = done
                 continue
             if pending is not None:
                 x, pending = x + pending, None

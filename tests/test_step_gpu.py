@@ -1,0 +1,137 @@
+"""Generation on sisa_step / sisa_cache_fill (csrc/step.hip) against the module path and the dense fp64 model, and the
+calls that must keep the module path."""
+import ctypes
+import os
+import subprocess
+
+import pytest
+import torch
+
+from model_utils import rel_err, tiny_model, token_ids
+from oracle import model64 as M64
+
+DEV = "cuda:0"
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+
+def _decode(model, ids, prompt, capacity=None):
+    from sisa_amd import SISACache
+    cache = SISACache(capacity)
+    with torch.no_grad():
+        parts = [model(ids[:, :prompt], cache=cache).logits]
+        parts += [model(ids[:, t:t + 1], cache=cache).logits for t in range(prompt, ids.shape[1])]
+    return torch.cat(parts, 1).float(), cache
+
+
+def _count(monkeypatch):
+    from sisa_amd.kernels import _lib
+    calls, real = {}, _lib.call
+
+    def call(name, args, t):
+        calls[name] = calls.get(name, 0) + 1
+        return real(name, args, t)
+    monkeypatch.setattr(_lib, "call", call)
+    return calls
+
+
+def _watched(model):
+    """The same model with a hook that does nothing on one projection: the modules are called one by one."""
+    return [blk.attn.W_Q.register_forward_hook(lambda *a: None) for blk in model.layers]
+
+
+# rows: one, two and four column groups of the products and their edges; widths below and above eight 32-element steps,
+# a head count that is not a multiple of the 16-row groups' 16; hidden widths that are no multiple of 32, 16, 8 or 2;
+# prompts of one position, of a chunk's edge and past it
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("B,H,d_ff,prompt,steps", [(1, 2, 256, 1, 3), (4, 12, 2744, 64, 3), (16, 3, 40, 5, 2),
+                                                   (17, 5, 329, 65, 2), (33, 2, 250, 7, 2), (64, 16, 1000, 3, 2)])
+def test_step_matches_modules(B, H, d_ff, prompt, steps, dtype, monkeypatch):
+    model = tiny_model(seed=B, theta_scale=0.25, attn_impl="auto", n_head=H, d_model=64 * H, d_ff=d_ff).to(DEV).to(
+        dtype).eval()
+    ids = token_ids(B, prompt + steps, seed=H).to(DEV)
+    ref = M64.logits64(model, M64.params64(model, requires_grad=False), ids)
+    calls = _count(monkeypatch)
+    got, cache = _decode(model, ids, prompt, None if B % 2 else prompt + steps)
+    assert calls["sisa_step"] == 2 * steps and calls["sisa_cache_fill"] == 2
+    assert "sisa_decode_attn" not in calls
+    hooks = _watched(model)
+    calls.clear()
+    want, kept = _decode(model, ids, prompt)
+    assert "sisa_step" not in calls and "sisa_cache_fill" not in calls and calls["sisa_decode_attn"] == 2 * steps
+    for h in hooks:
+        h.remove()
+    # both round the same quantities to the compute dtype: neither is further from fp64 than the other by more than
+    # the spread of such errors over a few hundred logits
+    assert rel_err(got, ref) <= 1.25 * rel_err(want, ref) + 1e-3
+    eps = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+    for layer in range(2):
+        a, b = cache.get(layer), kept.get(layer)
+        assert a.length == b.length == prompt + steps
+        error = {n: rel_err(getattr(a, n), getattr(b, n)) for n in ("k", "v", "b", "g", "fgate", "phi")}
+        # two roundings to the compute dtype each side; a phase that is off by d radians turns b~ by d more, and the
+        # phases, sums of rounded rates, are largest at the last position
+        turn = 2 * eps * float(b.phi.pow(2).mean().sqrt())
+        bound = dict(k=4 * eps, v=4 * eps, b=4 * eps + turn, g=2 * eps, fgate=2 * eps, phi=2 * eps)
+        assert all(error[n] <= bound[n] for n in error), (error, bound)
+
+
+@pytest.mark.gpu
+def test_calls_that_keep_the_module_path(monkeypatch):
+    """What a step does not stand for: gradients, autocast, fp32, several new positions, more rows than it takes, a
+    forced implementation other than the fused one, a subclass, a patched forward, a cache of another dtype."""
+    from sisa_amd import SISACache
+    calls = _count(monkeypatch)
+
+    def steps_of(model, ids, n=1, **kw):
+        cache = SISACache()
+        calls.clear()
+        with torch.no_grad():
+            model(ids[:, :8], cache=cache)
+        with kw.get("ctx", torch.no_grad)():
+            model(ids[:, 8:8 + n], cache=cache)
+        return calls.get("sisa_step", 0)
+
+    ids = token_ids(3, 12, seed=1).to(DEV)
+    model = tiny_model(seed=1, attn_impl="auto").to(DEV).to(torch.bfloat16).eval()
+    assert steps_of(model, ids) == 2
+    assert steps_of(model, ids, n=2) == 0
+    assert steps_of(model, ids, ctx=torch.enable_grad) == 0
+    assert steps_of(model, ids, ctx=lambda: torch.autocast("cuda", dtype=torch.bfloat16)) == 0
+    assert steps_of(model, token_ids(65, 12, seed=1).to(DEV)) == 0
+    model.set_attn_impl("hip")
+    assert steps_of(model, ids) == 0
+    model.set_attn_impl("auto")
+    model.layers[0].ffn.w_down.forward = model.layers[0].ffn.w_down.forward
+    assert steps_of(model, ids) == 1
+    assert steps_of(tiny_model(seed=1, attn_impl="auto").to(DEV).eval(), ids) == 0
+
+
+@pytest.mark.gpu
+def test_step_refuses_what_it_cannot_run():
+    from sisa_amd.kernels import _lib
+    x = torch.zeros(1, 64, device=DEV, dtype=torch.bfloat16)
+    for bad in (dict(B=0), dict(B=65), dict(D=63), dict(D=64 * 17, H=17), dict(pos=0), dict(dtype=_lib.F32), {}):
+        args = _lib.StepArgs(**{**dict(B=1, H=1, D=64, FF=64, dtype=_lib.BF16, pos=1), **bad})
+        with pytest.raises(RuntimeError):
+            _lib.call("sisa_step", args, x)
+
+
+def test_step_struct_layout_matches_c(tmp_path):
+    from sisa_amd.kernels import _lib
+    pairs = {"StepArgs": "sisa_step_args", "CacheFillArgs": "sisa_cache_fill_args"}
+    lines, expect = ["#include <stdio.h>", "#include <stddef.h>", '#include "sisa_hip_step.h"', "int main(void) {"], []
+    for py, c in pairs.items():
+        cls = getattr(_lib, py)
+        lines.append(f'printf("%zu\\n", sizeof({c}));')
+        expect.append(ctypes.sizeof(cls))
+        for name, _ in cls._fields_:
+            lines.append(f'printf("%zu\\n", offsetof({c}, {name}));')
+            expect.append(getattr(cls, name).offset)
+    lines += ["return 0;", "}"]
+    (tmp_path / "layout.c").write_text("\n".join(lines))
+    exe = tmp_path / "layout"
+    subprocess.run(["gcc", "-std=c99", "-I", os.path.join(ROOT, "include"), str(tmp_path / "layout.c"), "-o", str(exe)],
+                   check=True)
+    got = subprocess.run([str(exe)], capture_output=True, text=True, check=True).stdout.split()
+    assert [int(v) for v in got] == expect
