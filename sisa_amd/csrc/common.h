@@ -283,3 +283,11 @@ SISA_DEV frag8<T> ones_frag() {
     for (int j = 0; j < 8; ++j) r[j] = (T)1.f;
     return r;
 }
+
+// Work item of block i of a part of n items laid over 8 * ceil(n / 8) blocks (block i runs on XCD i % 8): XCD x
+// takes a contiguous range of items. -1 for a spare block.
+SISA_DEV int xcd_item(int i, int n) {
+    const int x = i & 7, k = i >> 3, q = n >> 3, r = n & 7;
+    if (k >= q + (x < r ? 1 : 0)) return -1;
+    return x * q + (x < r ? x : r) + k;
+}

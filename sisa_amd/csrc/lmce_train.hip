@@ -76,14 +76,6 @@ struct GradArgs {
     int accumulate;
 };
 
-// Work item of block i of a part of n items laid over 8 * ceil(n / 8) blocks (block i runs on XCD i % 8): XCD x
-// takes a contiguous range of items. -1 for a spare block.
-SISA_DEV int xcd_item(int i, int n) {
-    const int x = i & 7, k = i >> 3, q = n >> 3, r = n & 7;
-    if (k >= q + (x < r ? 1 : 0)) return -1;
-    return x * q + (x < r ? x : r) + k;
-}
-
 SISA_DEV int64_t clamp_bytes(int64_t b) {
     return b < 0 ? 0 : (b > (int64_t)0x7ffffff0 ? (int64_t)0x7ffffff0 : b);
 }
