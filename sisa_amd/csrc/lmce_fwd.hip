@@ -188,16 +188,28 @@ __global__ __launch_bounds__(64 * NWC) void lmce_fwd_kernel(sisa_lmce_fwd_args a
                 const float mref = mt == -__builtin_inff() ? 0.f : mt;
                 const int64_t n = row0 + wn + 16 * j + lc;
                 float ls = 0.f;
+                u32x2 prev = {0u, 0u};
 #pragma unroll
                 for (int i = 0; i < IB; ++i) {
                     f32x4 e;
 #pragma unroll
                     for (int r = 0; r < 4; ++r) e[r] = fast_exp2(fmaf(acc[i][j][r], LOG2E, -mref));
                     ls += (e[0] + e[1]) + (e[2] + e[3]);
-                    if constexpr (STORE) {   // unconditional: positions past the data go past the resource
-                        const int64_t v = (int64_t)vt * TV + wv + 16 * i + 4 * grp;
-                        const int off = (n < N && v < a.Vp) ? (int)((n * a.Vp + v) * (int64_t)sizeof(T)) : 0x7ffffff8;
-                        __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, to_vec4<T>(e)), prs, off, 0, 0);
+                    if constexpr (STORE) {
+                        // Blocks i - 1 and i trade places between neighbouring lane groups: a lane then holds 8
+                        // consecutive columns, 8 (grp / 2) .. + 7 of block i - 1 + grp % 2, and a store covers 64
+                        // consecutive bytes of each of its 16 rows (32 without the trade, for twice the stores).
+                        // Stores are unconditional: positions past the data go past the resource.
+                        const u32x2 cur = __builtin_bit_cast(u32x2, to_vec4<T>(e));
+                        if (i & 1) {
+                            const auto lo = __builtin_amdgcn_permlane16_swap(prev[0], cur[0], false, false);
+                            const auto hi = __builtin_amdgcn_permlane16_swap(prev[1], cur[1], false, false);
+                            const u32x4 q = {lo[0], hi[0], lo[1], hi[1]};
+                            const int64_t v = (int64_t)vt * TV + wv + 16 * (i - 1 + (grp & 1)) + 8 * (grp >> 1);
+                            const int off = (n < N && v < a.Vp) ? (int)((n * a.Vp + v) * (int64_t)sizeof(T)) : 0x7ffffff0;
+                            __builtin_amdgcn_raw_buffer_store_b128(q, prs, off, 0, 0);
+                        }
+                        prev = cur;
                     }
                 }
                 if constexpr (STORE) {
@@ -225,11 +237,11 @@ __global__ __launch_bounds__(64 * NWC) void lmce_fwd_kernel(sisa_lmce_fwd_args a
                 for (int j = 0; j < JB; ++j) acc[i][j] = zero4();
             if constexpr (STORE) {
                 // The barrier after a tile's stores waits only until the next stage's DMA (issued before them) has
-                // landed: vector memory operations complete in issue order, and at least the 32 exponential stores
-                // (unconditional instructions) follow it, so vmcnt <= 32 implies the DMA is done; the stores
+                // landed: vector memory operations complete in issue order, and at least the 16 exponential stores
+                // (unconditional instructions) follow it, so vmcnt <= 16 implies the DMA is done; the stores
                 // themselves complete under the next stage (its barrier waits for everything).
                 __builtin_amdgcn_sched_barrier(0);
-                __builtin_amdgcn_s_waitcnt(0x8070);   // vmcnt(32) expcnt(7) lgkmcnt(0)
+                __builtin_amdgcn_s_waitcnt(0x4070);   // vmcnt(16) expcnt(7) lgkmcnt(0)
                 __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
                 __builtin_amdgcn_s_barrier();
                 __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
