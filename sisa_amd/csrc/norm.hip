@@ -14,7 +14,7 @@
 //
 // Work decomposition: a wave holds RB = 64 / HP rows (HP = the projection width padded to 16, 32 or 64) with NVL =
 // HP / 8 eight-element vectors per lane (lane l holds elements 8 c .. 8 c + 7, c = l + 64 i), so RB * NVL = 8 and
-// the row length is at most 512 NVL. For up to 16 outputs and rows of at most 768 (a multiple of 64) the projection
+// the row length is at most 512 NVL. For up to 16 outputs and rows of at most 1024 (a multiple of 64) the projection
 // and its adjoint run on the matrix cores: the workgroup's sixteen rows of n (of dz W_f) pass through LDS and each
 // wave forms a quarter of the columns with v_mfma_f32_16x16x4_f32 (norm_fwd_mfma_kernel, norm_bwd_mfma_kernel).
 // Otherwise a lane's RB * HP projection partial sums are reduced over the 64 lanes with a halving exchange (63
@@ -191,10 +191,16 @@ __global__ __launch_bounds__(64 * NORM_WAVES) void norm_fwd_kernel(sisa_norm_arg
 // holds row l % 16 and reads four consecutive columns with one 16-byte LDS read, one per MFMA of the step; B = W_f:
 // the same four columns of row l % 16 of W_f), and the four partial tiles are summed in wave order (in the LDS
 // space of n once every wave is done with it).
-constexpr int MFMA_DMAX = 768;                  // W_f operand of at most 12 steps in registers
+// NQ: 16-column steps of a wave's quarter of the columns whose W_f operand fits its registers, 12 (D <= 768) or 16
+// (D <= 1024; a kernel of its own, so that narrower rows keep the smaller register set). At rows of 1,024
+// with 16 outputs the forward launch takes 10.0 us for 500 rows and 19.1 for 5,000 this way, 12.0 and 19.8 with the
+// projection on the vector units (one memory round trip and an MFMA chain set the short ones); the backward of 5,000
+// 42 us, 55 before this and the batched tails of the reductions.
+constexpr int MFMA_DMAX = 1024;
+constexpr int NQ_SMALL = 12, NQ_LARGE = MFMA_DMAX / 64;
 constexpr int NL_PAD = 4;                       // row padding of the staged n: conflict-free 16-byte reads
 inline int64_t norm_mfma_lds_bytes(int D) { return (int64_t)16 * (D + NL_PAD) * (int64_t)sizeof(float); }
-template <class TX, class TY>
+template <class TX, class TY, int NQ>
 __global__ __launch_bounds__(64 * NORM_WAVES) void norm_fwd_mfma_kernel(sisa_norm_args a) {
     constexpr int RB = 4, NVL = 2;
     extern __shared__ __attribute__((aligned(16))) float dyn_lds[];
@@ -223,9 +229,9 @@ __global__ __launch_bounds__(64 * NORM_WAVES) void norm_fwd_mfma_kernel(sisa_nor
     const int hq = lane & 15, kg = lane >> 4;
     const int nq = D / 64;                                 // 16-column steps per wave
     const int cw = w * (D / 4) + 4 * kg;
-    f32x4 wb[MFMA_DMAX / 64];
+    f32x4 wb[NQ];
 #pragma unroll
-    for (int q = 0; q < MFMA_DMAX / 64; ++q)
+    for (int q = 0; q < NQ; ++q)
         wb[q] = (q < nq && hq < a.H) ? *reinterpret_cast<const f32x4*>(a.wf + (int64_t)hq * D + cw + 16 * q)
                                      : f32x4{0.f, 0.f, 0.f, 0.f};
     if (a.res) {   // h = x + res, rounded to x's dtype as the residual add, normalised in place of x
@@ -281,7 +287,7 @@ __global__ __launch_bounds__(64 * NORM_WAVES) void norm_fwd_mfma_kernel(sisa_nor
     f32x4 acc = {0.f, 0.f, 0.f, 0.f};
     const float* arow = nl + hq * ld + cw;
 #pragma unroll
-    for (int q = 0; q < MFMA_DMAX / 64; ++q) {
+    for (int q = 0; q < NQ; ++q) {
         if (q < nq) {
             const f32x4 av = *reinterpret_cast<const f32x4*>(arow + 16 * q);
 #pragma unroll
@@ -441,7 +447,7 @@ __global__ __launch_bounds__(64 * NORM_WAVES) void norm_bwd_kernel(sisa_norm_arg
 // 4 s + l / 16 of K-step s; B = dz^T of tile row l % 16), so that a lane ends with four consecutive columns of one row,
 // stored to LDS as one 16-byte write; the row pass then reads its rows' products from there. Every wave takes part
 // in both steps (its rows past the end contribute zeros), so the barriers see the whole workgroup.
-template <class TX, class TY>
+template <class TX, class TY, int NQ>
 __global__ __launch_bounds__(64 * NORM_WAVES) void norm_bwd_mfma_kernel(sisa_norm_args a, float* __restrict__ dw_part) {
     constexpr int RB = 4, NVL = 2;
     extern __shared__ __attribute__((aligned(16))) float dyn_lds[];   // [16][D + NL_PAD]: dz W_f of the step's rows
@@ -471,9 +477,9 @@ __global__ __launch_bounds__(64 * NORM_WAVES) void norm_bwd_mfma_kernel(sisa_nor
     const int jq = lane & 15, kg = lane >> 4;
     const int nq = D / 64;
     const int cw = w * (D / 4) + jq;
-    f32x4 wa[MFMA_DMAX / 64];
+    f32x4 wa[NQ];
 #pragma unroll
-    for (int q = 0; q < MFMA_DMAX / 64; ++q)
+    for (int q = 0; q < NQ; ++q)
 #pragma unroll
         for (int s2 = 0; s2 < 4; ++s2) {
             const int h = 4 * s2 + kg;
@@ -504,7 +510,7 @@ __global__ __launch_bounds__(64 * NORM_WAVES) void norm_bwd_mfma_kernel(sisa_nor
         }
         if (it > 0) __syncthreads();                   // every wave is done reading the previous products
 #pragma unroll
-        for (int q = 0; q < MFMA_DMAX / 64; ++q) {
+        for (int q = 0; q < NQ; ++q) {
             if (q < nq) {
                 f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -632,7 +638,9 @@ SISA_DEV void forget_dw_block(const sisa_norm_args& a, float* __restrict__ part,
 }
 
 // s + p[0] + p[stride] + ... + p[(n-1) stride], added in that order; the loads go out BATCH at a time ahead of their
-// adds (a load-add chain would wait for every load in turn).
+// adds, those of a last, shorter batch too (a load-add chain waits for every load in turn: at 5,000 rows, whose 40
+// dW_f partials are less than one batch, that made the totals launch 17 us; the tail in batches
+// of 8, since 64 clamped loads for one partial cost 5 us).
 template <int BATCH = 16>
 SISA_DEV float ordered_sum(const float* __restrict__ p, int64_t stride, int64_t n, float s) {
     int64_t k = 0;
@@ -643,7 +651,14 @@ SISA_DEV float ordered_sum(const float* __restrict__ p, int64_t stride, int64_t 
 #pragma unroll
         for (int e = 0; e < BATCH; ++e) s += t[e];
     }
-    for (; k < n; ++k) s += p[k * stride];
+    constexpr int TAIL = BATCH < 8 ? BATCH : 8;
+    for (; k < n; k += TAIL) {         // the rest 8 at a time: loads past it repeat the last row, unused
+        float t[TAIL];
+#pragma unroll
+        for (int e = 0; e < TAIL; ++e) t[e] = p[(k + e < n ? k + e : n - 1) * stride];
+#pragma unroll
+        for (int e = 0; e < TAIL; ++e) s = k + e < n ? s + t[e] : s;
+    }
     return s;
 }
 
@@ -740,8 +755,10 @@ int launch_norm_hp(const sisa_norm_args* a, int bwd, hipStream_t st) {
     constexpr int RB = 64 / HP;
     if (!bwd) {
         if (HP == 16 && a->H > 0 && a->D % 64 == 0 && a->D <= MFMA_DMAX) {
-            norm_fwd_mfma_kernel<TX, TY><<<(unsigned)sisa::cdiv(a->N, 16), 64 * NORM_WAVES,
-                                           (size_t)norm_mfma_lds_bytes(a->D), st>>>(*a);
+            const unsigned grid = (unsigned)sisa::cdiv(a->N, 16);
+            const size_t lds = (size_t)norm_mfma_lds_bytes(a->D);
+            if (a->D <= 64 * NQ_SMALL) norm_fwd_mfma_kernel<TX, TY, NQ_SMALL><<<grid, 64 * NORM_WAVES, lds, st>>>(*a);
+            else norm_fwd_mfma_kernel<TX, TY, NQ_LARGE><<<grid, 64 * NORM_WAVES, lds, st>>>(*a);
             return sisa::launch_status("sisa_norm_fwd");
         }
         const int64_t waves = sisa::cdiv(a->N, RB);
@@ -750,11 +767,15 @@ int launch_norm_hp(const sisa_norm_args* a, int bwd, hipStream_t st) {
     }
     const NormWs ws = norm_ws(a);
     const int64_t np = sisa::cdiv(a->N, NORM_RPW);
-    if (HP == 16 && a->H > 0 && a->D % 64 == 0 && a->D <= MFMA_DMAX)
-        norm_bwd_mfma_kernel<TX, TY><<<(unsigned)sisa::cdiv(np, NORM_WAVES), 64 * NORM_WAVES,
-                                       (size_t)norm_mfma_lds_bytes(a->D), st>>>(*a, ws.dw_part);
+    const unsigned grid = (unsigned)sisa::cdiv(np, NORM_WAVES);
+    const size_t lds = (size_t)norm_mfma_lds_bytes(a->D);
+    const bool mfma = HP == 16 && a->H > 0 && a->D % 64 == 0 && a->D <= MFMA_DMAX;
+    if (mfma && a->D <= 64 * NQ_SMALL)
+        norm_bwd_mfma_kernel<TX, TY, NQ_SMALL><<<grid, 64 * NORM_WAVES, lds, st>>>(*a, ws.dw_part);
+    else if (mfma)
+        norm_bwd_mfma_kernel<TX, TY, NQ_LARGE><<<grid, 64 * NORM_WAVES, lds, st>>>(*a, ws.dw_part);
     else
-        norm_bwd_kernel<TX, TY, HP><<<(unsigned)sisa::cdiv(np, NORM_WAVES), 64 * NORM_WAVES, 0, st>>>(*a, ws.dw_part);
+        norm_bwd_kernel<TX, TY, HP><<<grid, 64 * NORM_WAVES, 0, st>>>(*a, ws.dw_part);
     int rc = sisa::launch_status("sisa_norm_bwd");
     if (rc) return rc;
     const int nrb = (int)norm_nrb(a->N);
