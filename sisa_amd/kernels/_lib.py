@@ -215,9 +215,7 @@ def dtype_code(dt: torch.dtype) -> int:
 
 def view(t: torch.Tensor | None) -> View:
     """(B,H,L,.) or (B,H,L) tensor -> View (pointer + batch/head/sequence strides). None -> null view."""
-    if t is None:
-        return View(None, 0, 0, 0)
-    return View(t.data_ptr(), t.stride(0), t.stride(1), t.stride(2))
+    return View(None, 0, 0, 0) if t is None else View(t.data_ptr(), *t.stride()[:3])
 
 
 def ptr(t: torch.Tensor | None):
@@ -225,13 +223,23 @@ def ptr(t: torch.Tensor | None):
 
 
 def stream_of(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
+    """The raw handle of the current stream on ``t``'s device."""
+    return torch._C._cuda_getCurrentRawStream(t.get_device())
+
+
+def launch(fn, tensor: torch.Tensor, *args) -> int:
+    """``fn(*args, stream)`` on ``tensor``'s device and its current stream. The device is entered only when it is not
+    the current one: the context manager and a Stream object cost as much host time as the launch itself."""
+    index = tensor.get_device()
+    if index == torch._C._cuda_getDevice():
+        return fn(*args, torch._C._cuda_getCurrentRawStream(index))
+    with torch.cuda.device(index):
+        return fn(*args, torch._C._cuda_getCurrentRawStream(index))
 
 
 def call(name: str, args, dev_tensor: torch.Tensor) -> None:
     lib = load()
-    with torch.cuda.device(dev_tensor.device):
-        rc = getattr(lib, name)(ctypes.byref(args), stream_of(dev_tensor))
+    rc = launch(getattr(lib, name), dev_tensor, ctypes.byref(args))
     if rc != 0:
         msg = lib.sisa_last_error().decode(errors="replace")
         raise RuntimeError(f"{name} failed (code {rc}): {msg}")

@@ -17,7 +17,7 @@ from . import _lib
 from . import attention as A
 from . import fused_prep as P
 
-__all__ = ["unobserved", "plain", "step_weights", "layer_step", "prefill", "MAX_ROWS", "MAX_WIDTH"]
+__all__ = ["unobserved", "plain", "plain_linears", "rows_ok", "step_weights", "layer_step", "prefill", "MAX_ROWS", "MAX_WIDTH"]
 
 MAX_ROWS, MAX_WIDTH = 64, 1024          # SISA_STEP_MAX_ROWS, SISA_STEP_MAX_D
 
@@ -38,23 +38,55 @@ def plain(module: nn.Module, kind: type) -> bool:
             and "forward" not in module.__dict__)
 
 
-def step_weights(table, x: Tensor) -> list[int] | None:
-    """Addresses of the parameters of ``table``, an iterable of (parameter, shape): each a plain contiguous parameter
-    of ``x``'s dtype on its device with that shape and, when it is a matrix, 16-byte aligned. None otherwise."""
-    dtype, device, out = x.dtype, x.get_device(), []
-    for p, shape in table:
+_ATTN_LINEARS = ("W_Q", "W_K", "W_V", "W_B", "W_C", "theta_proj", "alpha_proj", "forget_proj", "W_O")
+_FFN_LINEARS = ("w_gate", "w_up", "w_down")
+
+
+def plain_linears(attn: dict, ffn: dict) -> list[dict] | None:
+    """The parameter dicts of a block's twelve linear modules (attention in the order of ``sisa_step_args`` with W_O
+    last, then gate, up, down), or None unless every one is a :func:`plain` ``nn.Linear``."""
+    out = []
+    for mods, names in ((attn, _ATTN_LINEARS), (ffn, _FFN_LINEARS)):
+        for name in names:
+            m = mods.get(name)
+            if type(m) is not nn.Linear or m._forward_hooks or m._forward_pre_hooks or "forward" in m.__dict__:
+                return None
+            out.append(m._parameters)
+    return out
+
+
+def rows_ok(x: Tensor) -> bool:
+    """``x`` (B, 1, D) has rows that 16-byte loads can read."""
+    sb, _, sd = x.stride()
+    return sd == 1 and sb % 8 == 0 and x.data_ptr() % 16 == 0
+
+
+def step_weights(linears: list[dict], attn_norm, ffn_norm, H: int, x: Tensor) -> tuple[list[int], int] | None:
+    """Addresses of the parameters in the order of ``sisa_step_args`` (attn_norm .. w_down) and the FFN's width, or
+    None unless each is a plain contiguous parameter of the block's shape in ``x``'s dtype on its device, 16-byte
+    aligned where the kernels load it in vectors, with biases on the two gates only."""
+    D, s, dtype, device = x.shape[-1], HIP_D_STATE, x.dtype, x.get_device()
+    q, k, v, b, c, theta, alpha, forget, o, gate, up, down = (p["weight"] for p in linears)
+    biases = [p["bias"] for p in linears]
+    if gate is None or any(t is not None for i, t in enumerate(biases) if i not in (6, 7)):
+        return None
+    ff = gate.shape[0]
+    out = []
+    for p, shape in ((attn_norm, (D,)), (q, (D, D)), (k, (D, D)), (v, (D, D)), (b, (H * s, D)), (c, (H * s, D)),
+                     (theta, (H * s // 2, D)), (alpha, (H, D)), (biases[6], (H,)), (forget, (H, D)), (biases[7], (H,)),
+                     (o, (D, D)), (ffn_norm, (D,)), (gate, (ff, D)), (up, (ff, D)), (down, (D, ff))):
         if type(p) is not nn.Parameter or p.dtype is not dtype or p.shape != shape or p.get_device() != device \
                 or not p.is_contiguous():
             return None
         address = p.data_ptr()
-        if address % 16 and (len(shape) == 2 or shape[0] % 8 == 0):
+        if address % 16 and shape != (H,):
             return None
         out.append(address)
-    return out
+    return out, ff
 
 
-def layer_step(x: Tensor, res: Tensor | None, weights: list[int], lambda_raw: Tensor, eps: tuple[float, float],
-               d_ff: int, slab, phi: Tensor) -> tuple[Tensor, Tensor, Tensor]:
+def layer_step(x: Tensor, res: Tensor | None, weights: list[int], d_ff: int, lambda_raw: Tensor,
+               eps: tuple[float, float], slab, phi: Tensor) -> tuple[Tensor, Tensor, Tensor]:
     """The new position of ``x`` ``(B, 1, D)`` (plus ``res``, added first) through a layer; ``weights`` in the order of
     ``sisa_step_args`` (attn_norm .. w_down). Writes the position into ``slab`` (room for it is the caller's care) and
     returns ``(h, ffn, phi)``: the residual stream after the attention, the FFN output still to be added to it, and

@@ -28,7 +28,7 @@ from torch import Tensor
 from torch.utils.checkpoint import checkpoint
 
 from . import backends
-from .config import HIP_D_STATE, SISAConfig
+from .config import SISAConfig
 from .functional import attend_block, autocast_disabled, rotate_pairs, sisa_attention, working_dtype
 
 if TYPE_CHECKING:  # pragma: no cover
@@ -320,17 +320,6 @@ class SISABlock(nn.Module):
             return False
         return backends.select_impl(self.config.attn_impl, x, self.config) == "hip_fused"
 
-    def _plain(self) -> bool:
-        """Every module a cached HIP route passes by is the class this file builds it from, without hooks."""
-        from .kernels.step import plain
-
-        at, ffn = self.attn, self.ffn
-        return (plain(self, SISABlock) and plain(at, SISAAttention) and plain(ffn, SwiGLU) and plain(self.attn_norm, RMSNorm)
-                and plain(self.ffn_norm, RMSNorm)
-                and all(plain(lin, nn.Linear) for lin in (at.W_Q, at.W_K, at.W_V, at.W_O, at.W_B, at.W_C, at.theta_proj,
-                                                          at.alpha_proj, at.forget_proj, ffn.w_gate, ffn.w_up,
-                                                          ffn.w_down)))
-
     def _forward_cached_hip(self, x: Tensor, res: Tensor | None, cache: "SISACache"):
         """Generation on HIP kernels, or None where it does not apply. A prompt (empty cache entry) takes
         :meth:`_forward_hip` with the cache filled from the fused projections; one new position of at most 64 rows of
@@ -340,37 +329,32 @@ class SISABlock(nn.Module):
         from .kernels import step
 
         if x.device.type != "cuda" or type(cache) is not SISACache or not step.unobserved(x) \
-                or not self._fused_norm_ok(x) or not self._plain():
+                or not self._fused_norm_ok(x) or not step.plain(self, SISABlock):
             return None
-        at, ffn = self.attn, self.ffn
-        if at.alpha_proj.bias is None or at.forget_proj.bias is None:
+        mods = self._modules
+        at, ffn, n1, n2 = mods["attn"], mods["ffn"], mods["attn_norm"], mods["ffn_norm"]
+        if not (step.plain(at, SISAAttention) and step.plain(ffn, SwiGLU) and step.plain(n1, RMSNorm)
+                and step.plain(n2, RMSNorm)):
+            return None
+        linears = step.plain_linears(at._modules, ffn._modules)
+        if linears is None:
             return None
         slab = cache._slabs.get(at.layer_idx)
         if slab is None:
             return self._forward_hip(x, res, defer=True, cache=cache)
         B, L, D = x.shape
-        H, d_ff = self.config.n_head, ffn.w_gate.out_features
-        if L != 1 or B > step.MAX_ROWS or D > step.MAX_WIDTH or slab.filled < 1 \
-                or torch.is_autocast_enabled("cuda") or x.dtype not in _LOW_PRECISION or x.stride(-1) != 1 \
-                or x.stride(0) % 8 or x.data_ptr() % 16 or at.lambda_raw.dtype != torch.float32 \
-                or at.lambda_raw.shape != (H,) or at.lambda_raw.get_device() != x.get_device():
+        H, lam, buf = self.config.n_head, at.lambda_raw, slab.buffers
+        if L != 1 or B > step.MAX_ROWS or D > step.MAX_WIDTH or slab.filled < 1 or x.dtype not in _LOW_PRECISION \
+                or torch.is_autocast_enabled("cuda") or not step.rows_ok(x) or lam.dtype != torch.float32 \
+                or lam.shape != (H,) or lam.get_device() != x.get_device() or not lam.is_contiguous():
             return None
-        buf = slab.buffers
         if buf["k"].dtype != x.dtype or buf["k"].shape[:2] != (B, H) or buf["k"].get_device() != x.get_device():
             return None
-        s = HIP_D_STATE
-        weights = step.step_weights(
-            ((self.attn_norm.weight, (D,)), (at.W_Q.weight, (D, D)), (at.W_K.weight, (D, D)),
-             (at.W_V.weight, (D, D)), (at.W_B.weight, (H * s, D)), (at.W_C.weight, (H * s, D)),
-             (at.theta_proj.weight, (H * s // 2, D)), (at.alpha_proj.weight, (H, D)), (at.alpha_proj.bias, (H,)),
-             (at.forget_proj.weight, (H, D)), (at.forget_proj.bias, (H,)), (at.W_O.weight, (D, D)),
-             (self.ffn_norm.weight, (D,)), (ffn.w_gate.weight, (d_ff, D)), (ffn.w_up.weight, (d_ff, D)),
-             (ffn.w_down.weight, (D, d_ff))), x)
+        weights = step.step_weights(linears, n1._parameters["weight"], n2._parameters["weight"], H, x)
         if weights is None:
             return None
         slab = cache.room(at.layer_idx, 1, buf, slab.phi)
-        h, f, phi = step.layer_step(x, res, weights, at.lambda_raw.detach().contiguous(),
-                                    (self.attn_norm.eps, self.ffn_norm.eps), d_ff, slab, slab.phi.contiguous())
+        h, f, phi = step.layer_step(x, res, *weights, lam, (n1.eps, n2.eps), slab, slab.phi.contiguous())
         slab.filled, slab.phi = slab.filled + 1, phi
         return h, f
 
