@@ -112,92 +112,128 @@ SISA_DEV void fwd_tile(const FwdLds<T>& sm, int qblk, int lane, int n0, int q0, 
                        const frag8<T>& cx0, const frag8<T>& cx1, const frag8<T>& onesf, float fq, float rs, float gq,
                        float lam, float& m, float& l, f32x4 (&acc)[5], int nkb = 4) {
     constexpr bool ANCH = Anchor<T>::on && !DIAG;
+    constexpr int SB = DIAG ? 2 : 1;       // 32-key halves whose scores are held at once
     const int grp = lane >> 4, lc = lane & 15;
     const int qq = q0 + lc;
     const float* cfm = sm.cfm[qblk];
-    f32x4 sc[4], cb[4];
-#pragma unroll
-    for (int kb = 0; kb < 4; ++kb) {
-        if (DIAG && kb >= nkb) continue;
-        const frag8<T> k0 = frag_rows<T, DH>(sm.ks, kb * 16, 0, lane);
-        const frag8<T> k1 = frag_rows<T, DH>(sm.ks, kb * 16, 1, lane);
-        const frag8<T> bf = frag_rows<T, DS>(sm.bs, kb * 16, 0, lane);
-        if constexpr (ANCH) sc[kb] = mma(k1, qf[1], mma(k0, qf[0], lds4f(&sm.nfe[kb * 16 + 4 * grp])));
-        else sc[kb] = mma(k1, qf[1], mma(k0, qf[0], zero4()));
-        if constexpr (!DIAG && SplitC<T>::on) cb[kb] = mma(bf, cx1, mma(bf, cx0, zero4()));
-        else cb[kb] = mma(bf, cx0, zero4());
-    }
-    float mloc = -__builtin_inff();
-#pragma unroll
-    for (int kb = 0; kb < 4; ++kb) {
-        if (DIAG && kb >= nkb) continue;
-        const int j0 = kb * 16 + 4 * grp;
-        if constexpr (!ANCH) {   // the reference's difference F_i - F_j per element
-            const f32x4 fk = lds4f(&sm.fk[j0]);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) sc[kb][i] = sc[kb][i] + (fq - fk[i]);
-        }
-        if (DIAG) {
-            const f32x4 gk = lds4f(&sm.gk[j0]);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int jj = n0 + j0 + i;
-                const bool valid = jj <= qq && jj < L;
-                const float dec = valid ? exp2_le0((gq - gk[i]) * LOG2E) : 0.f;
-                float s = sc[kb][i] + lam * (dec * cb[kb][i]);
-                s = valid ? s : -__builtin_inff();
-                sc[kb][i] = s;
-                mloc = fmaxf(mloc, s);
-            }
-        } else {
-            const f32x4 cf = lds4f(&cfm[j0]);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                float s;
-                if constexpr (FoldC<T>::on) s = fmaf(cb[kb][i], cf[i], sc[kb][i]);
-                else s = sc[kb][i] + rs * (cb[kb][i] * cf[i]);
-                sc[kb][i] = s;
-                mloc = fmaxf(mloc, s);
-            }
-        }
-    }
-    // anchored tiles: sc holds s'' = s - (F_i - F_e); ft = (F_i - F_e) * log2e restores s in the exponent and max
     const float ft = ANCH ? (fq - sm.fk[63]) * LOG2E : 0.f;
-    // Online softmax in log2 units with lazy rescaling: a query's running offset m moves (and its l, acc are
-    // rescaled) only when its tile maximum exceeds m by more than RESCALE_LOG2, so the exponentials stay below
-    // 2^RESCALE_LOG2. The decision is per query (a query's results never depend on its neighbours); the wave skips
-    // the rescale when no query needs it, and queries that do not need it multiply by exactly 1. m starts at a
-    // finite floor, so fully masked rows give exp2(-inf) = 0. A NaN score reaches l through its exponential.
-    const float mt = ANCH ? fmaf(group_max(mloc), LOG2E, ft) : group_max(mloc) * LOG2E;
-    const bool need = mt > m + RESCALE_LOG2;
-    if (__builtin_amdgcn_ballot_w64(need) != 0) {
-        const float mn = need ? fmaxf(m, mt) : m;
+    f32x4 sc[SB][2], cb[SB][2];
+    // scores of the 32 keys of K-step st: sc holds s (anchored tiles: s'' = s - (F_i - F_e), restored by ft)
+    auto scores = [&](int st, f32x4 (&sc)[2], f32x4 (&cb)[2]) {
+#pragma unroll
+        for (int hb = 0; hb < 2; ++hb) {
+            const int kb = 2 * st + hb;
+            if (DIAG && kb >= nkb) continue;
+            const frag8<T> k0 = frag_rows<T, DH>(sm.ks, kb * 16, 0, lane);
+            const frag8<T> k1 = frag_rows<T, DH>(sm.ks, kb * 16, 1, lane);
+            const frag8<T> bf = frag_rows<T, DS>(sm.bs, kb * 16, 0, lane);
+            if constexpr (ANCH) sc[hb] = mma(k1, qf[1], mma(k0, qf[0], lds4f(&sm.nfe[kb * 16 + 4 * grp])));
+            else sc[hb] = mma(k1, qf[1], mma(k0, qf[0], zero4()));
+            if constexpr (!DIAG && SplitC<T>::on) cb[hb] = mma(bf, cx1, mma(bf, cx0, zero4()));
+            else cb[hb] = mma(bf, cx0, zero4());
+        }
+    };
+    auto finish = [&](int st, f32x4 (&sc)[2], f32x4 (&cb)[2]) {   // side term, decay, mask
+#pragma unroll
+        for (int hb = 0; hb < 2; ++hb) {
+            const int kb = 2 * st + hb;
+            if (DIAG && kb >= nkb) {
+                sc[hb] = f32x4{-__builtin_inff(), -__builtin_inff(), -__builtin_inff(), -__builtin_inff()};
+                continue;
+            }
+            const int j0 = kb * 16 + 4 * grp;
+            if constexpr (!ANCH) {   // the reference's difference F_i - F_j per element
+                const f32x4 fk = lds4f(&sm.fk[j0]);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) sc[hb][i] = sc[hb][i] + (fq - fk[i]);
+            }
+            if (DIAG) {
+                const f32x4 gk = lds4f(&sm.gk[j0]);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int jj = n0 + j0 + i;
+                    const bool valid = jj <= qq && jj < L;
+                    const float dec = valid ? exp2_le0((gq - gk[i]) * LOG2E) : 0.f;
+                    const float s = sc[hb][i] + lam * (dec * cb[hb][i]);
+                    sc[hb][i] = valid ? s : -__builtin_inff();
+                }
+            } else {
+                const f32x4 cf = lds4f(&cfm[j0]);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    if constexpr (FoldC<T>::on) sc[hb][i] = fmaf(cb[hb][i], cf[i], sc[hb][i]);
+                    else sc[hb][i] = sc[hb][i] + rs * (cb[hb][i] * cf[i]);
+                }
+            }
+        }
+    };
+    // Online softmax in log2 units with lazy rescaling: a query's running offset m moves (and its l, acc are rescaled)
+    // only when its weights would exceed 2^RESCALE_LOG2. The decision is per query (a query's results never depend on
+    // its neighbours); the wave skips the rescale when no query needs it, and queries that do not need it keep exactly
+    // what they have. m starts at a finite floor, so fully masked rows give exp2(-inf) = 0. A NaN score reaches l
+    // through its exponential.
+    float ls = 0.f;
+    auto weights = [&](const f32x4 (&sc)[2], f32x4 (&p)[2]) {   // p = exp2(s - m), ls = the lane's sum of them
+        const float off = ANCH ? ft - m : -m;
+        ls = 0.f;
+#pragma unroll
+        for (int hb = 0; hb < 2; ++hb)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                p[hb][i] = fast_exp2(fmaf(sc[hb][i], LOG2E, off));
+                ls += p[hb][i];
+            }
+    };
+    auto rescale = [&](float mloc, bool over) {   // the offset of the queries with `over` moved up to the maximum
+        const float mt = ANCH ? fmaf(group_max(mloc), LOG2E, ft) : group_max(mloc) * LOG2E;
+        const float mn = over ? fmaxf(m, mt) : m;
         const float corr = fast_exp2(m - mn);
         m = mn;
         l *= corr;
 #pragma unroll
         for (int db = 0; db < 5; ++db) acc[db] *= corr;
-    }
-    float ls = 0.f;
-    const float off = ANCH ? ft - m : -m;
+    };
+    auto max8 = [&](const f32x4 (&sc)[2], float x) {
 #pragma unroll
-    for (int kb = 0; kb < 4; ++kb) {
-        if (DIAG && kb >= nkb) {
-            sc[kb] = zero4();
-            continue;
-        }
+        for (int hb = 0; hb < 2; ++hb)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const float pe = fast_exp2(fmaf(sc[kb][i], LOG2E, off));
-            sc[kb][i] = pe;
-            ls += pe;
+            for (int i = 0; i < 4; ++i) x = fmaxf(x, sc[hb][i]);
+        return x;
+    };
+    if constexpr (DIAG) {                 // a wave's first tile: the offset from the whole tile's maximum
+        float mloc = -__builtin_inff();
+#pragma unroll
+        for (int st = 0; st < 2; ++st) {
+            scores(st, sc[st % SB], cb[st % SB]);
+            finish(st, sc[st % SB], cb[st % SB]);
+            mloc = max8(sc[st % SB], mloc);
         }
+        rescale(mloc, true);
     }
-    l += ls;
 #pragma unroll
     for (int st = 0; st < 2; ++st) {
         if (DIAG && 2 * st >= nkb) break;
-        const frag8<T> pf = pack8<T>(sc[2 * st], sc[2 * st + 1]);
+        f32x4 (&s2)[2] = sc[st % SB], (&p2)[2] = cb[st % SB];
+        if constexpr (!DIAG) {
+            __builtin_amdgcn_sched_barrier(0);
+            scores(st, s2, p2);
+            finish(st, s2, p2);
+        }
+        weights(s2, p2);
+        if constexpr (!DIAG) {
+            // The weights first, under the offset at hand: a lane's sum of 8 of them at most 2^RESCALE_LOG2 bounds
+            // each. With the tile's maximum formed before them (16 max, a reduction over the lane groups and a ballot
+            // between the scores and the first exponential) all 64 keys' scores had to be held at once; 32 keys at a
+            // time leave registers for the scheduler. 4 x 4096 x 8 heads 174 -> 170 us, 1 x 16384 x 16 heads
+            // 1082 -> 991, 2 x 3001 x 12 heads 81 -> 77.
+            const bool over = ls > __builtin_exp2f(RESCALE_LOG2);
+            if (__builtin_amdgcn_ballot_w64(over) != 0) {
+                rescale(max8(s2, -__builtin_inff()), group_max(over ? 1.f : 0.f) > 0.f);
+                weights(s2, p2);
+            }
+        }
+        l += ls;
+        const frag8<T> pf = pack8<T>(p2[0], p2[1]);
 #pragma unroll
         for (int db = 0; db < 4; ++db) acc[db] = mma(frag_tr<T, DH>(sm.vs, db * 16, st, lane), pf, acc[db]);
         acc[4] = mma(onesf, pf, acc[4]);   // block 4: every row holds the sum of the rounded weights
