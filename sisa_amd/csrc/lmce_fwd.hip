@@ -32,6 +32,7 @@ namespace {
 constexpr int NWC = 8;            // waves per workgroup: 2 along the vocabulary x 4 along the rows
 constexpr int TR = 256;           // rows of x per workgroup
 constexpr int TV = 256;           // vocabulary columns per tile
+constexpr int RGRP = 4;           // row blocks that walk the same vocabulary tiles side by side
 constexpr int WV = 128;           // vocabulary columns of a wave (8 MFMA blocks)
 constexpr int WR = 64;            // rows of a wave (4 MFMA blocks)
 constexpr int IB = WV / 16, JB = WR / 16;
@@ -73,7 +74,12 @@ __global__ __launch_bounds__(64 * NWC) void lmce_fwd_kernel(sisa_lmce_fwd_args a
     const int nrb = (int)((N + TR - 1) / TR);
     const int item = xcd_item(blockIdx.x, nrb * S);
     if (item < 0) return;
-    const int split = item % S, rb = item / S;
+    // Items (row block, split) in groups of RGRP row blocks, row blocks fastest: the 32 workgroups an XCD runs at a time
+    // are then 4 row blocks x 8 splits, which read 12 tiles of x and W per tile time through its L2; one row block with 32
+    // splits reads 33.
+    const int grp_items = RGRP * S, g0 = item / grp_items * RGRP, in_grp = item % grp_items;
+    const int rg = nrb - g0 < RGRP ? nrb - g0 : RGRP;
+    const int split = in_grp / rg, rb = g0 + in_grp % rg;
     const int tiles = (int)((a.Vp + TV - 1) / TV);
     const int t_begin = split * per;
     const int t_end = t_begin + per < tiles ? t_begin + per : tiles;
