@@ -17,10 +17,13 @@
 // when the tile holds a row's label it keeps that logit. At the end the lane groups and the two waves sharing rows
 // combine their partials; a second launch combines the S splits of each row in a fixed order.
 //
-// The training pass (sisa_lmce_train, lmce_train.hip) runs the same kernel with STORE: each exponential
-// p~ = exp2(logit*log2e - m_t), m_t the row's maximum over the wave's half of the tile, is also stored in the compute
-// dtype into a (N, Vp) buffer, and m_t into a (2 * tiles, N) table; the gradient GEMMs later form
-// G = p~ * exp2(m_t - lse) * scale - onehot from them. Both passes therefore give bitwise the same loss rows.
+// bf16 takes the exponentials against one reference per row, its label's logit (REF; lmce_ref_kernel), and falls back,
+// for a call with a row that reference does not suit, to the maxima described above; see launch_logits. At 4,094 rows of
+// 1,024 (V 50,277) the launch takes 427 us with REF, 458 without.
+//
+// The training pass (sisa_lmce_train, lmce_train.hip) runs the same kernel with STORE: each exponential is also stored in
+// the compute dtype into a (N, Vp) buffer, and without REF the maxima m_t it is relative to into a (2 * tiles, N) table.
+// Both passes give bitwise the same loss rows.
 // Deterministic: no atomics. Workgroup i runs on XCD i % 8; each XCD takes an equal, contiguous range of (row block,
 // split) items, whole row blocks with all their splits where there are enough, so that its L2 keeps those rows of x for
 // every vocabulary tile and fewer than eight row blocks still fill all XCDs.
@@ -47,11 +50,16 @@ struct __attribute__((aligned(16))) CeLds {
     float red_m[TR], red_s[TR];   // the second wave of each row pair hands over its row partials
 };
 
-// Outputs of the training pass (STORE): exponentials relative to the tile-half maxima and those maxima.
+// What a launch stores and against what it takes its exponentials.
+//   STORE: the exponentials go to probs. REF: they are relative to one given reference per row (ref, log2 units)
+//   instead of the row's maxima over the tile halves, which go to mtab.
+//   gate: run only if *gate is nonzero (null: always).
 template <class T>
 struct CeStore {
     T* probs;                     // (N, Vp) in the compute dtype, row stride Vp; columns >= V hold 0
     float* mtab;                  // (2 * tiles, N): m_t of (tile t, half h) at row (2 t + h) * N + n, log2 units
+    const float* ref;             // (N,)
+    const int* gate;
 };
 
 // The vocabulary splits of one problem: S splits of `per` consecutive tiles (the last ones may be shorter or empty).
@@ -65,9 +73,10 @@ inline Split ce_split(int64_t N, int64_t Vp) {
     return {tiles, S, sisa::cdiv(tiles, S)};
 }
 
-template <class T, bool STORE>
+template <class T, bool STORE, bool REF>
 __global__ __launch_bounds__(64 * NWC) void lmce_fwd_kernel(sisa_lmce_fwd_args a, int S, int per, CeStore<T> out) {
     __shared__ CeLds<T> sm;
+    if (out.gate && *out.gate == 0) return;
     const int tid = threadIdx.x, lane = tid & 63, grp = lane >> 4, lc = lane & 15;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int64_t N = a.N, V = a.V;
@@ -101,9 +110,9 @@ __global__ __launch_bounds__(64 * NWC) void lmce_fwd_kernel(sisa_lmce_fwd_args a
         const int k0 = (g % nks) * TK;
 #pragma unroll
         for (int h = 0; h < 4; ++h) {
-            dma_issue<STORE ? 8 : 4>(sx, X, xbytes, (int)(((row0 + 64 * h) * a.ldx + k0) * (int64_t)sizeof(T)),
+            dma_issue<(STORE ? 8 : 4) + (REF ? 16 : 0)>(sx, X, xbytes, (int)(((row0 + 64 * h) * a.ldx + k0) * (int64_t)sizeof(T)),
                          sm.x[buf] + 64 * h * TK, w);
-            dma_issue<STORE ? 9 : 5>(sw, W, wbytes, (int)(((v0 + 64 * h) * a.ldw + k0) * (int64_t)sizeof(T)),
+            dma_issue<(STORE ? 9 : 5) + (REF ? 16 : 0)>(sw, W, wbytes, (int)(((v0 + 64 * h) * a.ldw + k0) * (int64_t)sizeof(T)),
                          sm.w[buf] + 64 * h * TK, w);
         }
     };
@@ -125,10 +134,11 @@ __global__ __launch_bounds__(64 * NWC) void lmce_fwd_kernel(sisa_lmce_fwd_args a
             }
         }
     }
-    float m[JB], s[JB], zlab[JB];
+    float m[JB], s[JB], zlab[JB];   // REF: m is the rows' reference
 #pragma unroll
     for (int j = 0; j < JB; ++j) {
-        m[j] = M_FLOOR_CE;
+        const int64_t n = row0 + wn + 16 * j + lc;
+        m[j] = REF ? (n < N ? out.ref[n] : 0.f) : M_FLOOR_CE;
         s[j] = 0.f;
         zlab[j] = 0.f;
     }
@@ -185,13 +195,15 @@ __global__ __launch_bounds__(64 * NWC) void lmce_fwd_kernel(sisa_lmce_fwd_args a
 #pragma unroll
             for (int j = 0; j < JB; ++j) {
                 float mt = -__builtin_inff();   // the row's maximum over the wave's 128 columns, in log2 units
+                if constexpr (!REF) {
 #pragma unroll
-                for (int i = 0; i < IB; ++i)
+                    for (int i = 0; i < IB; ++i)
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) mt = fmaxf(mt, acc[i][j][r]);
-                mt = group_max(mt) * LOG2E;
+                        for (int r = 0; r < 4; ++r) mt = fmaxf(mt, acc[i][j][r]);
+                    mt = group_max(mt) * LOG2E;
+                }
                 // a half made only of padding columns (-inf) takes the reference 0: its exponentials are 0
-                const float mref = mt == -__builtin_inff() ? 0.f : mt;
+                const float mref = REF ? m[j] : (mt == -__builtin_inff() ? 0.f : mt);
                 const int64_t n = row0 + wn + 16 * j + lc;
                 float ls = 0.f;
                 u32x2 prev = {0u, 0u};
@@ -218,10 +230,12 @@ __global__ __launch_bounds__(64 * NWC) void lmce_fwd_kernel(sisa_lmce_fwd_args a
                         prev = cur;
                     }
                 }
-                if constexpr (STORE) {
+                if constexpr (STORE && !REF) {
                     if (grp == 0 && n < N) out.mtab[(int64_t)(2 * vt + (w & 1)) * N + n] = mref;
                 }
-                if (mt > m[j]) {
+                if constexpr (REF) {
+                    s[j] += ls;
+                } else if (mt > m[j]) {
                     s[j] = fmaf(s[j], fast_exp2(m[j] - mt), ls);
                     m[j] = mt;
                 } else {
@@ -261,8 +275,8 @@ __global__ __launch_bounds__(64 * NWC) void lmce_fwd_kernel(sisa_lmce_fwd_args a
     float rm[JB], rsum[JB];
 #pragma unroll
     for (int j = 0; j < JB; ++j) {
-        rm[j] = group_max(m[j]);
-        rsum[j] = group_sum(s[j] * fast_exp2(m[j] - rm[j]));
+        rm[j] = REF ? m[j] : group_max(m[j]);
+        rsum[j] = group_sum(REF ? s[j] : s[j] * fast_exp2(m[j] - rm[j]));
         if (got[j]) a.workspace[2 * (int64_t)S * N + row0 + wn + 16 * j + lc] = zlab[j];
     }
     if ((w & 1) && grp == 0) {
@@ -279,6 +293,10 @@ __global__ __launch_bounds__(64 * NWC) void lmce_fwd_kernel(sisa_lmce_fwd_args a
             const int64_t n = row0 + wn + 16 * j + lc;
             if (n >= N) continue;
             const float m2 = sm.red_m[wn + 16 * j + lc], s2 = sm.red_s[wn + 16 * j + lc];
+            if constexpr (REF) {
+                a.workspace[(int64_t)(S + split) * N + n] = rsum[j] + s2;
+                continue;
+            }
             const float mm = fmaxf(rm[j], m2);
             a.workspace[(int64_t)split * N + n] = mm;
             a.workspace[(int64_t)(S + split) * N + n] = rsum[j] * fast_exp2(rm[j] - mm) + s2 * fast_exp2(m2 - mm);
@@ -293,34 +311,55 @@ struct CeTrainRows {
     float2* rinfo;                // (N,): s_n, and the label as the bit pattern of an int (-1 outside [0, V))
     const float* inv_n;           // device scalar 1 / N_valid
     float gscale;
+    const float* ref;             // REF: (N,) the reference of the row's exponentials, log2 units
+    float* cn;                    // REF: (N,) s_n / Z_n, or nullptr
+    int* flag;                    // REF: set when a row's sum is not one the reference was good for
+    const int* gate;              // run only if *gate is nonzero (null: always)
 };
 
 // 16 rows per workgroup, 16 threads per row: each folds every sixteenth split, and the row's first thread the sixteen
 // partial results in order. (One thread per row walks S splits in dependent loads: with the 128 splits of 1,023 rows
 // that took 66 us.)
 constexpr int CRW = 16, CSP = 16;
+constexpr float Z_MAX = 0x1p60f, Z_MIN = 0x1p-20f;   // sums whose exponentials and products stay far inside fp32 / bf16
+
+template <bool REF>
 __global__ __launch_bounds__(CRW * CSP) void lmce_combine_kernel(sisa_lmce_fwd_args a, int S, CeTrainRows tr) {
     __shared__ float pm[CSP][CRW], ps[CSP][CRW];
+    if (tr.gate && *tr.gate == 0) return;
     const int lr = threadIdx.x % CRW, part = threadIdx.x / CRW;
     const int64_t n = (int64_t)blockIdx.x * CRW + lr, N = a.N;
     float mm = M_FLOOR_CE, ss = 0.f;
     if (n < N) {
         for (int sp = part; sp < S; sp += CSP) {
-            const float m = a.workspace[(int64_t)sp * N + n], s = a.workspace[(int64_t)(S + sp) * N + n];
-            const float mn = fmaxf(mm, m);
-            ss = fmaf(ss, fast_exp2(mm - mn), s * fast_exp2(m - mn));
-            mm = mn;
+            const float s = a.workspace[(int64_t)(S + sp) * N + n];
+            if constexpr (REF) {
+                ss += s;
+            } else {
+                const float m = a.workspace[(int64_t)sp * N + n];
+                const float mn = fmaxf(mm, m);
+                ss = fmaf(ss, fast_exp2(mm - mn), s * fast_exp2(m - mn));
+                mm = mn;
+            }
         }
     }
     pm[part][lr] = mm;
     ps[part][lr] = ss;
     __syncthreads();
     if (part != 0 || n >= N) return;
+    if constexpr (REF) {
+        mm = tr.ref[n];
+        ss = 0.f;
 #pragma unroll
-    for (int p = 1; p < CSP; ++p) mm = fmaxf(mm, pm[p][lr]);
-    ss = 0.f;
+        for (int p = 0; p < CSP; ++p) ss += ps[p][lr];
+        if (!(ss >= Z_MIN && ss <= Z_MAX)) *tr.flag = 1;   // NaN too; every writer stores the same value
+    } else {
 #pragma unroll
-    for (int p = 0; p < CSP; ++p) ss = fmaf(ps[p][lr], fast_exp2(pm[p][lr] - mm), ss);
+        for (int p = 1; p < CSP; ++p) mm = fmaxf(mm, pm[p][lr]);
+        ss = 0.f;
+#pragma unroll
+        for (int p = 0; p < CSP; ++p) ss = fmaf(ps[p][lr], fast_exp2(pm[p][lr] - mm), ss);
+    }
     const float l2 = mm + __builtin_amdgcn_logf(ss);
     const float lse = l2 * LN2;
     const int64_t y = a.labels[n];
@@ -333,20 +372,76 @@ __global__ __launch_bounds__(CRW * CSP) void lmce_combine_kernel(sisa_lmce_fwd_a
     if (tr.lse2) {
         tr.lse2[n] = l2;
         const int lab = (y >= 0 && y < a.V) ? (int)y : -1;
-        tr.rinfo[n] = float2{y == a.ignore_index ? 0.f : tr.inv_n[0] * tr.gscale, __int_as_float(lab)};
+        const float sn = y == a.ignore_index ? 0.f : tr.inv_n[0] * tr.gscale;
+        tr.rinfo[n] = float2{sn, __int_as_float(lab)};
+        if (REF && tr.cn) tr.cn[n] = sn / ss;
     }
 }
 
+// The reference of a row's exponentials: the logit of its label (of column 0 without a valid one), in log2 units. Any
+// column's logit bounds the row's sum below by 1; the label's is near the largest wherever the loss is small. One wave
+// per row; also clears the flag.
 template <class T>
-int launch_lmce_fwd(const sisa_lmce_fwd_args* a, hipStream_t st) {
+__global__ __launch_bounds__(256) void lmce_ref_kernel(sisa_lmce_fwd_args a, float* ref, int* flag) {
+    const int64_t n = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    const int lane = threadIdx.x & 63;
+    if (blockIdx.x == 0 && threadIdx.x == 0) *flag = 0;
+    if (n >= a.N) return;
+    const int64_t y = a.labels[n];
+    const T* x = (const T*)a.x + n * a.ldx;
+    const T* w = (const T*)a.w + (y >= 0 && y < a.V ? y : 0) * a.ldw;
+    float d = 0.f;
+    for (int c = 8 * lane; c < a.D; c += 512) {
+        const f32x8 xv = load_f32x8<T>(x + c), wv = load_f32x8<T>(w + c);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) d = fmaf(xv[e], wv[e], d);
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) d += __shfl_xor(d, o);
+    if (lane == 0) ref[n] = d * LOG2E;
+}
+
+// Logits GEMM and combine. bf16: against the label logits (REF), then, gated on the flag of a row whose sum left
+// [Z_MIN, Z_MAX] (its label's logit more than 41 below the row's largest, or non-finite values), again against the
+// tile-half maxima; the gated launches of an unflagged call end at once. That spares each logit the running maximum,
+// and lets the gradient products of the training pass take the stored exponentials as they are. fp16 has too little
+// exponent range for a reference per row and always takes the maxima.
+template <class T, bool STORE>
+int launch_logits(const sisa_lmce_fwd_args* a, T* probs, float* mtab, const CeTrainRows& rows, float* ref, int* flag,
+                  hipStream_t st) {
     const Split sp = ce_split(a->N, a->Vp);
     const unsigned grid = (unsigned)(8 * sisa::cdiv(sisa::cdiv(a->N, TR) * sp.S, 8));
-    lmce_fwd_kernel<T, false><<<grid, 64 * NWC, 0, st>>>(*a, (int)sp.S, (int)sp.per, CeStore<T>{nullptr, nullptr});
-    const int rc = sisa::launch_status("sisa_lmce_fwd");
+    const unsigned cgrid = (unsigned)sisa::cdiv(a->N, CRW);
+    const int S = (int)sp.S, per = (int)sp.per;
+    CeTrainRows r = rows;
+    if constexpr (__is_same(T, __bf16)) {
+        lmce_ref_kernel<T><<<(unsigned)sisa::cdiv(a->N, 4), 256, 0, st>>>(*a, ref, flag);
+        int rc = sisa::launch_status("linear CE (reference)");
+        if (rc) return rc;
+        lmce_fwd_kernel<T, STORE, true><<<grid, 64 * NWC, 0, st>>>(*a, S, per, CeStore<T>{probs, nullptr, ref, nullptr});
+        rc = sisa::launch_status("linear CE (logits)");
+        if (rc) return rc;
+        r.ref = ref;
+        r.flag = flag;
+        lmce_combine_kernel<true><<<cgrid, CRW * CSP, 0, st>>>(*a, S, r);
+        rc = sisa::launch_status("linear CE (combine)");
+        if (rc) return rc;
+        r.gate = flag;
+    }
+    lmce_fwd_kernel<T, STORE, false><<<grid, 64 * NWC, 0, st>>>(*a, S, per, CeStore<T>{probs, mtab, nullptr, r.gate});
+    const int rc = sisa::launch_status("linear CE (logits)");
     if (rc) return rc;
-    lmce_combine_kernel<<<(unsigned)sisa::cdiv(a->N, CRW), CRW * CSP, 0, st>>>(*a, (int)sp.S,
-                                                                        CeTrainRows{nullptr, nullptr, nullptr, 0.f});
-    return sisa::launch_status("sisa_lmce_fwd (combine)");
+    lmce_combine_kernel<false><<<cgrid, CRW * CSP, 0, st>>>(*a, S, r);
+    return sisa::launch_status("linear CE (combine)");
+}
+
+// The split partials (max and sum rows, label logits), then the rows' references and the flag.
+float* ws_ref(const sisa_lmce_fwd_args* a) { return a->workspace + (2 * ce_split(a->N, a->Vp).S + 1) * a->N; }
+int* ws_flag(const sisa_lmce_fwd_args* a) { return (int*)(ws_ref(a) + a->N); }
+
+template <class T>
+int launch_lmce_fwd(const sisa_lmce_fwd_args* a, hipStream_t st) {
+    return launch_logits<T, false>(a, nullptr, nullptr, CeTrainRows{}, ws_ref(a), ws_flag(a), st);
 }
 
 }  // namespace
@@ -354,26 +449,28 @@ int launch_lmce_fwd(const sisa_lmce_fwd_args* a, hipStream_t st) {
 namespace sisa {
 namespace detail {
 
-int64_t lmce_fwd_splits(int64_t N, int64_t Vp) { return ce_split(N, Vp).S; }
+// Bytes of the logits pass's workspace (partials, references, flag).
+int64_t lmce_fwd_ws_bytes(int64_t N, int64_t Vp) {
+    return (2 * ce_split(N, Vp).S + 2) * N * (int64_t)sizeof(float) + 16;
+}
 
-// The training pass's forward: the logits GEMM storing the exponentials and tile-half maxima (probs: (N, Vp) in the
-// compute dtype; mtab: (2 * ceil(Vp / 256), N) fp32), then the split combine writing the loss rows, lse in log2 units
-// and each row's gradient scale. a->workspace holds the (2 S + 1) N split partials.
-int lmce_train_forward(const sisa_lmce_fwd_args* a, void* probs, float* mtab, float* lse2, float2* rinfo,
-                       const float* inv_n, float gscale, hipStream_t st) {
-    const Split sp = ce_split(a->N, a->Vp);
-    const unsigned grid = (unsigned)(8 * sisa::cdiv(sisa::cdiv(a->N, TR) * sp.S, 8));
+// The training pass's forward: the logits GEMM storing the exponentials (probs: (N, Vp) in the compute dtype), then the
+// split combine writing the loss rows, lse in log2 units and each row's gradient scale, for bf16 also s_n / Z_n (cn).
+// Afterwards *flag (returned; null for fp16) tells on the device which exponentials probs holds: zero, those against
+// one reference per row, G = probs * cn - s_n [label]; nonzero or null, those against the tile-half maxima in mtab
+// ((2 * ceil(Vp / 256), N) fp32). a->workspace: lmce_fwd_ws_bytes.
+int lmce_train_forward(const sisa_lmce_fwd_args* a, void* probs, float* mtab, float* lse2, float2* rinfo, float* cn,
+                       const float* inv_n, float gscale, const int** flag, hipStream_t st) {
+    CeTrainRows r{};
+    r.lse2 = lse2;
+    r.rinfo = rinfo;
+    r.inv_n = inv_n;
+    r.gscale = gscale;
+    r.cn = cn;
+    *flag = a->dtype == SISA_BF16 ? ws_flag(a) : nullptr;
     if (a->dtype == SISA_BF16)
-        lmce_fwd_kernel<__bf16, true><<<grid, 64 * NWC, 0, st>>>(*a, (int)sp.S, (int)sp.per,
-                                                                  CeStore<__bf16>{(__bf16*)probs, mtab});
-    else
-        lmce_fwd_kernel<_Float16, true><<<grid, 64 * NWC, 0, st>>>(*a, (int)sp.S, (int)sp.per,
-                                                                    CeStore<_Float16>{(_Float16*)probs, mtab});
-    const int rc = sisa::launch_status("sisa_lmce_train (logits)");
-    if (rc) return rc;
-    lmce_combine_kernel<<<(unsigned)sisa::cdiv(a->N, CRW), CRW * CSP, 0, st>>>(*a, (int)sp.S,
-                                                                        CeTrainRows{lse2, rinfo, inv_n, gscale});
-    return sisa::launch_status("sisa_lmce_train (combine)");
+        return launch_logits<__bf16, true>(a, (__bf16*)probs, mtab, r, ws_ref(a), ws_flag(a), st);
+    return launch_logits<_Float16, true>(a, (_Float16*)probs, mtab, r, nullptr, nullptr, st);
 }
 
 }  // namespace detail
@@ -381,7 +478,7 @@ int lmce_train_forward(const sisa_lmce_fwd_args* a, void* probs, float* mtab, fl
 
 extern "C" int64_t sisa_lmce_fwd_workspace_bytes(int64_t N, int64_t Vp) {
     if (N < 1 || Vp < 1) return 0;
-    return (2 * ce_split(N, Vp).S + 1) * N * (int64_t)sizeof(float);
+    return sisa::detail::lmce_fwd_ws_bytes(N, Vp);
 }
 
 extern "C" int sisa_lmce_fwd(const sisa_lmce_fwd_args* a, void* stream) {

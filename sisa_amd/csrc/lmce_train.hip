@@ -6,27 +6,33 @@
 // dW += G^T x (library GEMMs, fp32 results). The contract (loss rows, fp32 dx and dW of a G rounded once to the
 // compute dtype, ignored rows contributing nothing) is the reference's; the arrangement is this library's own:
 //
-//   1. the logits GEMM of sisa_lmce_fwd (lmce_fwd.hip) with its STORE epilogue: each exponential
-//      p~ = exp2(logit * log2e - m_t), m_t the row's maximum over one 128-column half of a 256-column vocabulary
-//      tile, goes to a (N, Vp) buffer in the compute dtype and m_t to a (2 * tiles, N) table; the split partials
-//      are combined into the loss rows (bitwise those of sisa_lmce_fwd), lse2 = lse / ln 2 and, per row, the scale
-//      s_n = inv_n * gscale (0 for ignored rows) with the label (-1 when outside [0, V));
-//   2. lmce_scale_kernel turns the m_t table into c = exp2(m_t - lse2) * s_n in place, so that
-//      G[n, v] = p~[n, v] * c[n, tile half of v] - s_n [v == label_n], and writes each row's label entry of G;
-//   3. one launch of lmce_grad_kernel runs two kinds of output tiles: dW tiles (256 vocabulary x 256 hidden, all
-//      rows of the chunk as K) first, then dx tiles (256 rows x 256 hidden, K = a range of the vocabulary: dx is
-//      split over the vocabulary so that both kinds of workgroup run about equally long and the last round of the
-//      grid is short). Both form G from p~ and c while staging it into LDS (16-byte loads, 8 multiplies, the rare
-//      label subtraction, one rounding to the compute dtype, one 16-byte LDS store per 8 values); the dense operand
-//      (W_pad rows for dx, x rows for dW) is staged by buffer loads straight into LDS; both are double-buffered;
+//   1. the logits GEMM of sisa_lmce_fwd (lmce_fwd.hip) with its STORE epilogue: each row's exponentials go to a (N, Vp)
+//      buffer in the compute dtype. bf16: p~ = exp2(logit * log2e - r_n) against one reference per row, its label's
+//      logit, so that G = p~ s_n / Z_n - s_n [v == label_n] with Z_n = sum_v p~ and the row's scale s_n = inv_n * gscale
+//      (0 for ignored rows). A row whose Z_n leaves [2^-20, 2^60] raises the chunk's flag, and launches gated on it redo
+//      the chunk the second way (also fp16's, whose exponent range is too small for the first): against m_t, the row's
+//      maximum over one 128-column half of a vocabulary tile, kept in a (2 * tiles, N) table. The loss rows are bitwise
+//      those of sisa_lmce_fwd either way;
+//   2. first way: lmce_xscale_kernel writes x s_n / Z_n, rounded; one launch of lmce_grad_kernel runs plain products of
+//      the stored exponentials, dW tiles (256 vocabulary x 256 hidden, all rows of the chunk as K) first, then dx tiles
+//      (256 rows x 256 hidden, K = a range of the vocabulary: dx is split so that both kinds of workgroup run about
+//      equally long), both operands by buffer loads straight into LDS (plain_tile); lmce_label_dw_kernel and the dx
+//      reduction subtract the label terms in fp32 and the latter applies s_n / Z_n;
+//   3. second way: lmce_scale_kernel turns the m_t table into c = exp2(m_t - lse2) * s_n in place, so that
+//      G[n, v] = p~[n, v] * c[n, tile half of v] - s_n [v == label_n], and writes each row's label entry of G; the same
+//      launch of lmce_grad_kernel then forms G from p~ and c while staging it into LDS (grad_tile: 16-byte loads, 8
+//      multiplies, the rare label subtraction, one rounding and one 16-byte LDS store per 8 values);
 //   4. lmce_dx_reduce_kernel adds the dx splits in split order.
+// Rounding: p~ once; then x s_n / Z_n (dW) or nothing (dx) the first way, G the second; the label terms are exact to fp32
+// the first way. At 16,384 rows of 768 (V 50,277) the gradient launch takes 2,399 us the first way (1.06 PFLOP/s) and
+// 3,209 the second; 157 and 204 us at 1,023 rows of 512.
 // G and the logits are never written to memory; the only large buffer is the chunk's exponentials (read once per
 // output column tile). Deterministic: no atomics.
 //
-// Tile arithmetic: a workgroup of 2 x 4 waves, two waves per SIMD (247 VGPRs); a wave owns 128 hidden x 64 rows
+// Tile arithmetic: a workgroup of 2 x 4 waves, two waves per SIMD (249 VGPRs); a wave owns 128 hidden x 64 rows
 // (dx) or 128 hidden x 64 vocabulary (dW) as 8 x 4 blocks of v_mfma_f32_16x16x32 (128 accumulators; all 12 operand
 // fragments of a 32-deep step are read before its 32 MFMAs), hidden on the A side so that a lane's 4 results are 4
-// consecutive hidden values (16-byte stores). The next stage's exponentials are loaded into registers before a
+// consecutive hidden values (16-byte stores). The second way's next exponentials are loaded into registers before a
 // stage's MFMAs and formed into G in LDS after them. dx reads W_pad as A with the feature-map transpose read (K = vocabulary, W_pad
 // rows) and G as B with direct 16-byte fragment reads (K = vocabulary along G rows); dW reads x and G both with the
 // sequence-map transpose read (K = rows). Workgroup i runs on XCD i % 8; each XCD takes consecutive work items, so
@@ -36,9 +42,9 @@
 
 namespace sisa {
 namespace detail {
-int64_t lmce_fwd_splits(int64_t N, int64_t Vp);
-int lmce_train_forward(const sisa_lmce_fwd_args* a, void* probs, float* mtab, float* lse2, float2* rinfo,
-                       const float* inv_n, float gscale, hipStream_t st);
+int64_t lmce_fwd_ws_bytes(int64_t N, int64_t Vp);
+int lmce_train_forward(const sisa_lmce_fwd_args* a, void* probs, float* mtab, float* lse2, float2* rinfo, float* cn,
+                       const float* inv_n, float gscale, const int** flag, hipStream_t st);
 }  // namespace detail
 }  // namespace sisa
 
@@ -53,6 +59,7 @@ constexpr int WD = 128, WO = 64;    // wave tile: hidden x rows / vocabulary (tw
 constexpr int IB = WD / 16, JB = WO / 16;
 constexpr int GL = TO * TK / 8 / (64 * NWG);   // 16-byte G loads per thread and stage (4)
 
+// Both forms of the gradient tiles stage the same amounts.
 template <class T>
 struct __attribute__((aligned(16))) GradLds {
     T dense[2][TK * TD];            // W_pad rows (dx) or x rows (dW): 64 K-rows x 256 hidden, toff<T, 256>
@@ -74,6 +81,8 @@ struct GradArgs {
     int dx_splits, dx_per;          // vocabulary splits of dx, 64-column stages per split
     int n_dw, n_dw_pad, n_dx;       // dW items (blocks padded to a multiple of 8), dx items
     int accumulate;
+    const int* flag;                // device: nonzero = exponentials against tile-half maxima (null: always so)
+    const void* xs;                 // (N, D) x * s_n / Z_n in the compute dtype, row stride D (per-row references)
 };
 
 SISA_DEV int64_t clamp_bytes(int64_t b) {
@@ -95,6 +104,39 @@ SISA_DEV void g_store(T* dst, const frag8<T>& raw, float c, int rel, float gl) {
 template <class T>
 SISA_DEV frag8<T> load16(__amdgpu_buffer_rsrc_t r, int voff) {
     return __builtin_bit_cast(frag8<T>, __builtin_amdgcn_raw_buffer_load_b128(r, voff, 0, 0));
+}
+
+// An output tile from the accumulators: dW (added to what is there with accumulate), or a dx partial.
+template <bool DW>
+SISA_DEV void store_tile(const GradArgs& a, f32x4 (&acc)[IB][JB], int vt, int sp, int64_t n0, int d0, int wd, int wo,
+                         int grp, int lc) {
+    const int64_t N = a.N, Vp = a.Vp;
+    // lane l, register r of block (i, j): hidden d0 + wd + 16 i + 4 (l / 16) + r, row / vocabulary wo + 16 j + l % 16
+    if constexpr (DW) {
+        if (a.accumulate) {   // all of the lane's earlier partial sums in flight at once, then the sums
+#pragma unroll
+            for (int j = 0; j < JB; ++j) {
+                const int64_t o = (int64_t)vt * TO + wo + 16 * j + lc;
+#pragma unroll
+                for (int i = 0; i < IB; ++i) {
+                    const int d = d0 + wd + 16 * i + 4 * grp;
+                    if (o < Vp && d < a.D) acc[i][j] += *reinterpret_cast<const f32x4*>(a.dw + o * a.lddw + d);
+                }
+            }
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < JB; ++j) {
+        const int64_t o = (DW ? (int64_t)vt * TO : n0) + wo + 16 * j + lc;
+        if (o >= (DW ? Vp : N)) continue;
+#pragma unroll
+        for (int i = 0; i < IB; ++i) {
+            const int d = d0 + wd + 16 * i + 4 * grp;
+            if (d >= a.D) continue;
+            if constexpr (DW) *reinterpret_cast<f32x4*>(a.dw + o * a.lddw + d) = acc[i][j];
+            else *reinterpret_cast<f32x4*>(a.dxo + (int64_t)sp * a.split_stride + o * a.lddxo + d) = acc[i][j];
+        }
+    }
 }
 
 // One output tile: DW (dW tile u = vocabulary tile * dts + hidden tile) or dx (u = (row block * dx_splits + split)
@@ -231,53 +273,191 @@ SISA_DEV void grad_tile(const GradArgs& a, GradLds<T>& sm, int u) {
         __syncthreads();
     }
 
-    // lane l, register r of block (i, j): hidden d0 + wd + 16 i + 4 (l / 16) + r, row / vocabulary wo + 16 j + l % 16
-    if constexpr (DW) {
-        if (a.accumulate) {   // all of the lane's earlier partial sums in flight at once, then the sums
+    store_tile<DW>(a, acc, vt, sp, n0, d0, wd, wo, grp, lc);
+}
+
+// One output tile when the exponentials are relative to one reference per row, G = p~ cn - s_n [label]: plain products of
+// the stored exponentials, dW = p~^T (x cn) and dx / cn = p~ W (the scale and the label terms are applied where dx is
+// reduced and by lmce_label_dw_kernel). Both operands go straight into LDS, so a stage's MFMAs have nothing beside them
+// but their fragment reads: forming G while staging it (16-byte loads to registers, 32 multiplies, packing and label
+// checks a thread and stage) kept the matrix pipe idle for a third of the launch.
+template <class T, bool DW>
+SISA_DEV void plain_tile(const GradArgs& a, GradLds<T>& sm, int u) {
+    const int lane = threadIdx.x & 63, grp = lane >> 4, lc = lane & 15;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int64_t N = a.N, Vp = a.Vp;
+    const int dt = u % a.dts, rest = u / a.dts;
+    const int d0 = dt * TD;
+    const int vt = rest, sp = rest % a.dx_splits, rb = rest / a.dx_splits;
+    const int64_t n0 = DW ? 0 : (int64_t)rb * TO;
+    const int k0 = DW ? 0 : sp * a.dx_per;
+    const int kstages = DW ? (int)((N + TK - 1) / TK) : (int)(Vp / TK);
+    const int k1 = DW ? kstages : (k0 + a.dx_per < kstages ? k0 + a.dx_per : kstages);
+    const int total = k1 > k0 ? k1 - k0 : 0;
+    const int wd = WD * (w & 1), wo = WO * (w >> 1);
+
+    DmaStage<T, TD, NWG> dma;                        // dense: 64 K-rows x 256 hidden columns
+    const T* dsrc = DW ? (const T*)a.xs + d0 : (const T*)a.w + d0;
+    const int64_t dld = DW ? a.D : a.ldw;
+    const int64_t drows = DW ? N : Vp;
+    const int64_t dbytes = ((drows - 1) * dld + a.D - d0) * (int64_t)sizeof(T);
+    dma.init(dld, w, lane);
+    // exponentials: 64 rows x 256 vocabulary columns (dW), 256 rows x 64 columns as four groups of 64 rows (dx); rows past
+    // the data read as zero, columns past Vp belong to outputs that are not stored
+    constexpr int GC = DW ? TO : TK, GG = DW ? 1 : TO / 64;
+    DmaStage<T, GC, NWG> dmg;
+    dmg.init(Vp, w, lane);
+    const T* P = (const T*)a.probs;
+    auto issue = [&](int g, int buf) {
+        const int64_t k = (int64_t)(k0 + g) * TK;
+        dma_issue<DW ? 10 : 11>(dma, dsrc, dbytes, (int)(k * dld * (int64_t)sizeof(T)), sm.dense[buf], w);
 #pragma unroll
-            for (int j = 0; j < JB; ++j) {
-                const int64_t o = (int64_t)vt * TO + wo + 16 * j + lc;
-#pragma unroll
-                for (int i = 0; i < IB; ++i) {
-                    const int d = d0 + wd + 16 * i + 4 * grp;
-                    if (o < Vp && d < a.D) acc[i][j] += *reinterpret_cast<const f32x4*>(a.dw + o * a.lddw + d);
-                }
-            }
+        for (int h = 0; h < GG; ++h) {
+            const int64_t row = DW ? k : n0 + 64 * h, col = DW ? (int64_t)vt * TV : k;
+            dma_issue<DW ? 12 : 13>(dmg, P + row * Vp + col, clamp_bytes(((N - row) * Vp - col) * (int64_t)sizeof(T)), 0,
+                                    sm.g[buf] + 64 * h * GC, w);
         }
-    }
+    };
+
+    f32x4 acc[IB][JB];
 #pragma unroll
-    for (int j = 0; j < JB; ++j) {
-        const int64_t o = (DW ? (int64_t)vt * TO : n0) + wo + 16 * j + lc;
-        if (o >= (DW ? Vp : N)) continue;
+    for (int i = 0; i < IB; ++i)
 #pragma unroll
-        for (int i = 0; i < IB; ++i) {
-            const int d = d0 + wd + 16 * i + 4 * grp;
-            if (d >= a.D) continue;
-            if constexpr (DW) *reinterpret_cast<f32x4*>(a.dw + o * a.lddw + d) = acc[i][j];
-            else *reinterpret_cast<f32x4*>(a.dxo + (int64_t)sp * a.split_stride + o * a.lddxo + d) = acc[i][j];
+        for (int j = 0; j < JB; ++j) acc[i][j] = zero4();
+    if (total > 0) issue(0, 0);
+    __syncthreads();
+    for (int g = 0; g < total; ++g) {
+        const int buf = g & 1;
+        if (g + 1 < total) issue(g + 1, buf ^ 1);
+        __builtin_amdgcn_sched_barrier(0);           // the next stage's loads go out before this stage's MFMAs
+#pragma unroll
+        for (int step = 0; step < TK / 32; ++step) {
+            frag8<T> af[IB], bf[JB];
+#pragma unroll
+            for (int j = 0; j < JB; ++j)
+                bf[j] = DW ? frag_tr<T, TO>(sm.g[buf], wo + 16 * j, step, lane)
+                           : frag_rows<T, TK>(sm.g[buf], wo + 16 * j, step, lane);
+#pragma unroll
+            for (int i = 0; i < IB; ++i)
+                af[i] = DW ? frag_tr<T, TD>(sm.dense[buf], wd + 16 * i, step, lane)
+                           : frag_trf<T, TD>(sm.dense[buf], wd + 16 * i, step, lane);
+#pragma unroll
+            for (int i = 0; i < IB; ++i)
+#pragma unroll
+                for (int j = 0; j < JB; ++j) acc[i][j] = mma(af[i], bf[j], acc[i][j]);
         }
+        __syncthreads();
     }
+    store_tile<DW>(a, acc, vt, sp, n0, d0, wd, wo, grp, lc);
 }
 
 template <class T>
 __global__ __launch_bounds__(64 * NWG) void lmce_grad_kernel(GradArgs a) {
     __shared__ GradLds<T> sm;
     const int i = blockIdx.x;
-    if (i < a.n_dw_pad) {
-        const int u = xcd_item(i, a.n_dw);
-        if (u >= 0) grad_tile<T, true>(a, sm, u);
-    } else {
-        const int u = xcd_item(i - a.n_dw_pad, a.n_dx);
-        if (u >= 0) grad_tile<T, false>(a, sm, u);
+    const bool dw = i < a.n_dw_pad;
+    const int u = dw ? xcd_item(i, a.n_dw) : xcd_item(i - a.n_dw_pad, a.n_dx);
+    if (u < 0) return;
+    if constexpr (__is_same(T, __bf16)) {
+        if (a.flag && *a.flag == 0) {
+            if (dw) plain_tile<T, true>(a, sm, u);
+            else plain_tile<T, false>(a, sm, u);
+            return;
+        }
+    }
+    if (dw) grad_tile<T, true>(a, sm, u);
+    else grad_tile<T, false>(a, sm, u);
+}
+
+// xs[n, :] = x[n, :] * cn[n], rounded once (the dense operand of dW; the other one is the rounded exponential, as G was
+// the rounded product of the two)
+template <class T>
+__global__ __launch_bounds__(256) void lmce_xscale_kernel(const T* x, int64_t ldx, const float* cn, T* xs, int64_t N,
+                                                          int D, const int* flag) {
+    if (*flag) return;
+    const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    const int q = D / 8;
+    if (idx >= N * q) return;
+    const int64_t n = idx / q;
+    const int d = 8 * (int)(idx % q);
+    const f32x8 v = load_f32x8<T>(x + n * ldx + d) * cn[n];
+    store_f32x8<T>(xs + n * D + d, v);
+}
+
+// dW[label_n, :] -= s_n x[n, :] in row order, for rows with a valid label. A workgroup owns 64 vocabulary rows and
+// collects, LBATCH rows of the chunk at a time, the rows whose label is among them (in order, by ballots); wave w then adds
+// those of vocabulary rows 16 w .. 16 w + 15, each lane always the same columns, so that sums run in row order without
+// atomics. 16,384 labels over 50,304 vocabulary rows: 66 us (32 and 128 rows a workgroup: 82, 78).
+constexpr int LROWS = 64, LBATCH = 4096;
+template <class T>
+__global__ __launch_bounds__(256) void lmce_label_dw_kernel(const float2* rinfo, const T* x, int64_t ldx, float* dw,
+                                                            int64_t lddw, int64_t N, int D, const int* flag) {
+    if (*flag) return;
+    __shared__ int list[LBATCH], lrow[LBATCH];
+    __shared__ int count[4], base[4];
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    const int v0 = blockIdx.x * LROWS;
+    constexpr int PW = LBATCH / 4;                   // consecutive rows scanned by a wave
+    for (int64_t b0 = 0; b0 < N; b0 += LBATCH) {
+        const int64_t n0 = b0 + w * PW;
+        int lab[PW / 64];
+        int cnt = 0;
+#pragma unroll
+        for (int k = 0; k < PW / 64; ++k) {
+            const int64_t n = n0 + 64 * k + lane;
+            lab[k] = n < N ? __float_as_int(rinfo[n].y) - v0 : -1;
+        }
+#pragma unroll
+        for (int k = 0; k < PW / 64; ++k) cnt += __popcll(__builtin_amdgcn_ballot_w64((unsigned)lab[k] < (unsigned)LROWS));
+        if (lane == 0) count[w] = cnt;
+        __syncthreads();
+        if (tid == 0) {
+            int s = 0;
+            for (int k = 0; k < 4; ++k) {
+                base[k] = s;
+                s += count[k];
+            }
+        }
+        __syncthreads();
+        const int total = base[3] + count[3];
+        int at = base[w];
+#pragma unroll
+        for (int k = 0; k < PW / 64; ++k) {
+            const bool hit = (unsigned)lab[k] < (unsigned)LROWS;
+            const uint64_t m = __builtin_amdgcn_ballot_w64(hit);
+            if (hit) {
+                const int p = at + __popcll(m & (((uint64_t)1 << lane) - 1));
+                list[p] = (int)(n0 - b0) + 64 * k + lane;
+                lrow[p] = lab[k];
+            }
+            at += __popcll(m);
+        }
+        __syncthreads();
+        for (int e = 0; e < total; ++e) {
+            const int r = lrow[e];
+            if (r / (LROWS / 4) != w) continue;      // wave-uniform
+            const int64_t n = b0 + list[e];
+            const float sn = rinfo[n].x;
+            float* out = dw + (int64_t)(v0 + r) * lddw;
+            for (int d = 4 * lane; d < D; d += 256) {
+                const vec4<T> xv = load4<T>(x + n * ldx + d);
+                f32x4 o = lds4f(out + d);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) o[i] = fmaf(-sn, (float)xv[i], o[i]);
+                *reinterpret_cast<f32x4*>(out + d) = o;
+            }
+        }
+        __syncthreads();
     }
 }
 
-// c[k, n] = exp2(m_t[k, n] - lse2[n]) * s_n, in place over the (2 * tiles, N) table
 // c[k, n] = exp2(m_t[k, n] - lse2[n]) * s_n, in place over the (2 * tiles, N) table; the entry k that holds the
 // row's label also writes G at the label, p~ * c - s_n, rounded once to T (glab, kept in fp32)
 template <class T>
 __global__ __launch_bounds__(256) void lmce_scale_kernel(float* cs, const float* lse2, const float2* rinfo,
-                                                         const T* probs, int64_t Vp, float* glab, int64_t N) {
+                                                         const T* probs, int64_t Vp, float* glab, int64_t N,
+                                                         const int* gate) {
+    if (gate && *gate == 0) return;
     const int64_t n = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (n >= N) return;
     const int k = blockIdx.y;
@@ -290,20 +470,33 @@ __global__ __launch_bounds__(256) void lmce_scale_kernel(float* cs, const float*
         glab[n] = (float)cvt<T>(fmaf((float)probs[n * Vp + lab], c, -ri.x));
 }
 
-// dx[n, :] = sum over the splits, in split order, of the partial rows
+// dx[n, :] = sum over the splits, in split order, of the partial rows; with per-row references (flag given and zero) that
+// sum is scaled by cn[n], and the label's term s_n W[label_n] subtracted
+template <class T>
 __global__ __launch_bounds__(256) void lmce_dx_reduce_kernel(const float* part, float* dx, int64_t N, int D, int S,
-                                                             int64_t lddx) {
+                                                             int64_t lddx, const int* flag, const float* cn,
+                                                             const float2* rinfo, const T* w, int64_t ldw) {
     const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
     const int q = D / 4;
     if (idx >= N * q) return;
     const int64_t n = idx / q, d = 4 * (idx % q);
     f32x4 s = lds4f(part + n * D + d);
     for (int sp = 1; sp < S; ++sp) s += lds4f(part + ((int64_t)sp * N + n) * D + d);
+    if (flag && *flag == 0) {
+        s *= cn[n];
+        const float2 ri = rinfo[n];
+        const int lab = __float_as_int(ri.y);
+        if (lab >= 0) {
+            const vec4<T> wv = load4<T>(w + (int64_t)lab * ldw + d);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) s[i] = fmaf(-ri.x, (float)wv[i], s[i]);
+        }
+    }
     *reinterpret_cast<f32x4*>(dx + n * lddx + d) = s;
 }
 
 struct Layout {
-    int64_t probs, cs, part, lse2, srow, glab, dxp, total;
+    int64_t probs, cs, part, lse2, srow, glab, cn, xs, dxp, total;
 };
 
 int64_t align256(int64_t b) { return (b + 255) / 256 * 256; }
@@ -321,11 +514,13 @@ Layout layout(int64_t N, int64_t Vp, int D, int dx_splits) {
     l.probs = 0;
     l.cs = align256(N * Vp * 2);
     l.part = l.cs + align256(2 * tiles * N * 4);
-    l.lse2 = l.part + align256((2 * sisa::detail::lmce_fwd_splits(N, Vp) + 1) * N * 4);
+    l.lse2 = l.part + align256(sisa::detail::lmce_fwd_ws_bytes(N, Vp));
     l.srow = l.lse2 + align256(N * 4);
     l.glab = l.srow + align256(N * 8);
-    l.dxp = l.glab + align256(N * 4);
-    l.total = l.dxp + (dx_splits > 1 ? align256((int64_t)dx_splits * N * D * 4) : 0);
+    l.cn = l.glab + align256(N * 4);
+    l.xs = l.cn + align256(N * 4);
+    l.dxp = l.xs + align256(N * D * 2);
+    l.total = l.dxp + align256((int64_t)dx_splits * N * D * 4);
     return l;
 }
 
@@ -371,18 +566,27 @@ extern "C" int sisa_lmce_train(const sisa_lmce_train_args* a, void* stream) {
     float* glab = (float*)(ws + l.glab);
     sisa_lmce_fwd_args f{a->N, a->V, a->Vp, a->D, a->dtype, a->x, a->ldx, a->w, a->ldw, a->labels, a->ignore_index,
                          a->lse, a->loss_rows, (float*)(ws + l.part)};
-    int rc = sisa::detail::lmce_train_forward(&f, ws + l.probs, cs, lse2, rinfo, a->inv_n, a->gscale, st);
+    float* cn = (float*)(ws + l.cn);
+    const int* flag = nullptr;       // bf16: which exponentials the logits pass left (lmce_train_forward)
+    int rc = sisa::detail::lmce_train_forward(&f, ws + l.probs, cs, lse2, rinfo, cn, a->inv_n, a->gscale, &flag, st);
     if (rc || (a->dx == nullptr && a->dw == nullptr)) return rc;
 
     const int64_t tiles = sisa::cdiv(a->Vp, TV);
     const dim3 sgrid((unsigned)sisa::cdiv(a->N, 256), (unsigned)(2 * tiles));
     if (a->dtype == SISA_BF16)
-        lmce_scale_kernel<__bf16><<<sgrid, 256, 0, st>>>(cs, lse2, rinfo, (const __bf16*)(ws + l.probs), a->Vp, glab, a->N);
+        lmce_scale_kernel<__bf16><<<sgrid, 256, 0, st>>>(cs, lse2, rinfo, (const __bf16*)(ws + l.probs), a->Vp, glab, a->N,
+                                                         flag);
     else
         lmce_scale_kernel<_Float16><<<sgrid, 256, 0, st>>>(cs, lse2, rinfo, (const _Float16*)(ws + l.probs), a->Vp, glab,
-                                                           a->N);
+                                                           a->N, flag);
     rc = sisa::launch_status("sisa_lmce_train (scale)");
     if (rc) return rc;
+    if (flag && a->dw) {
+        lmce_xscale_kernel<__bf16><<<(unsigned)sisa::cdiv(a->N * (a->D / 8), 256), 256, 0, st>>>(
+            (const __bf16*)a->x, a->ldx, cn, (__bf16*)(ws + l.xs), a->N, a->D, flag);
+        rc = sisa::launch_status("sisa_lmce_train (scaled rows)");
+        if (rc) return rc;
+    }
 
     GradArgs g{};
     g.probs = ws + l.probs;
@@ -407,7 +611,10 @@ extern "C" int sisa_lmce_train(const sisa_lmce_train_args* a, void* stream) {
     g.dw = a->dw;
     g.lddw = a->lddw;
     g.accumulate = a->dw_accumulate != 0;
-    if (S > 1) {
+    g.flag = flag;
+    g.xs = ws + l.xs;
+    const bool reduce = S > 1 || flag;
+    if (reduce) {
         g.dxo = (float*)(ws + l.dxp);
         g.lddxo = a->D;
         g.split_stride = a->N * a->D;
@@ -420,8 +627,20 @@ extern "C" int sisa_lmce_train(const sisa_lmce_train_args* a, void* stream) {
     if (a->dtype == SISA_BF16) lmce_grad_kernel<__bf16><<<grid, 64 * NWG, 0, st>>>(g);
     else lmce_grad_kernel<_Float16><<<grid, 64 * NWG, 0, st>>>(g);
     rc = sisa::launch_status("sisa_lmce_train (gradients)");
-    if (rc || a->dx == nullptr || S == 1) return rc;
-    lmce_dx_reduce_kernel<<<(unsigned)sisa::cdiv(a->N * (a->D / 4), 256), 256, 0, st>>>(g.dxo, a->dx, a->N, a->D, S,
-                                                                                       a->lddx);
+    if (rc) return rc;
+    if (flag && a->dw) {
+        lmce_label_dw_kernel<__bf16><<<(unsigned)(a->Vp / LROWS), 256, 0, st>>>(rinfo, (const __bf16*)a->x, a->ldx, a->dw,
+                                                                              a->lddw, a->N, a->D, flag);
+        rc = sisa::launch_status("sisa_lmce_train (label rows)");
+        if (rc) return rc;
+    }
+    if (a->dx == nullptr || !reduce) return SISA_OK;
+    const unsigned rgrid = (unsigned)sisa::cdiv(a->N * (a->D / 4), 256);
+    if (a->dtype == SISA_BF16)
+        lmce_dx_reduce_kernel<__bf16><<<rgrid, 256, 0, st>>>(g.dxo, a->dx, a->N, a->D, S, a->lddx, flag, cn, rinfo,
+                                                             (const __bf16*)a->w, a->ldw);
+    else
+        lmce_dx_reduce_kernel<_Float16><<<rgrid, 256, 0, st>>>(g.dxo, a->dx, a->N, a->D, S, a->lddx, flag, cn, rinfo,
+                                                               (const _Float16*)a->w, a->ldw);
     return sisa::launch_status("sisa_lmce_train (dx splits)");
 }

@@ -1,0 +1,89 @@
+"""The linear cross-entropy's two ways of keeping a row's exponentials: against one reference per row (its label's
+logit; plain gradient products) and, where a row's sum leaves that reference's range, against the maxima over half
+vocabulary tiles. A chunk takes the second way as soon as one of its rows needs it."""
+import pytest
+import torch
+
+DEV = "cuda:0"
+
+
+def _case(N, D, V, seed, one_label=False):
+    gen = torch.Generator().manual_seed(seed)
+    x = torch.randn(N, D, generator=gen).to(torch.bfloat16).to(DEV)
+    w = (0.7 / D ** 0.5 * torch.randn(V, D, generator=gen)).to(torch.bfloat16).to(DEV)
+    lab = torch.full((N,), V - 1) if one_label else torch.randint(0, V, (N,), generator=gen)
+    lab[0], lab[N // 2], lab[N // 3] = 0, V - 1, -100
+    return x, w, lab.to(DEV)
+
+
+def _poison(x, w, lab):
+    """One more row, ignored, that no single reference of column 0 fits: its logits spread over hundreds."""
+    row = (w[1] - w[0]).float()
+    row = (row * (300.0 / row.norm() ** 2)).to(torch.bfloat16)
+    return torch.cat([x, row[None]]), w, torch.cat([lab, lab.new_tensor([-100])])
+
+
+def _run(x, w, lab, **kw):
+    from sisa_amd.kernels.linear_ce import linear_cross_entropy
+    x, w = x.clone().requires_grad_(True), w.float().requires_grad_(True)
+    loss = linear_cross_entropy(x, w, lab, **kw)
+    dx, dw = torch.autograd.grad(loss, (x, w))
+    return loss.detach(), dx, dw
+
+
+def _truth(x, w, lab):
+    x, w = x.double().requires_grad_(True), w.double().requires_grad_(True)
+    loss = torch.nn.functional.cross_entropy(x @ w.t(), lab, ignore_index=-100)
+    return (loss.detach(), *torch.autograd.grad(loss, (x, w)))
+
+
+def _rel(a, b):
+    return float((a.double() - b.double()).norm() / b.double().norm())
+
+
+# ragged rows and vocabularies; the hidden sizes' tile remainders (64, 768, 1024 of 256-wide tiles); one, several and many
+# vocabulary splits of dx; 5,000 rows with one label (a label list longer than the kernel's batch)
+@pytest.mark.gpu
+@pytest.mark.parametrize("N,D,V,one_label", [(1, 64, 65, False), (300, 512, 1003, False), (257, 768, 50277, False),
+                                             (5000, 64, 130, True), (4500, 320, 1000, False), (70, 1024, 8191, False)])
+def test_row_references_match_tile_maxima(N, D, V, one_label):
+    x, w, lab = _case(N, D, V, N + D, one_label)
+    if N == 1:
+        lab[0] = 3
+    ref = _truth(x, w, lab)
+    fast = _run(x, w, lab)
+    loss, dx, dw = _run(*_poison(x, w, lab))
+    slow = (loss, dx[:N], dw)
+    assert torch.equal(dx[N], torch.zeros_like(dx[N]))
+    assert N == 1 or not torch.equal(fast[1], slow[1])      # two computations, not one
+    for got in (fast, slow):
+        # logits rounded to 8 bits shift the loss by the mean of their errors; gradients: three 8-bit roundings
+        assert abs(float(got[0] - ref[0])) <= 2 ** -8 * (1 + abs(float(ref[0])))
+        assert _rel(got[1], ref[1]) <= 3 * 2 ** -8 and _rel(got[2], ref[2]) <= 3 * 2 ** -8
+    assert abs(float(fast[0] - slow[0])) <= 1e-5 * abs(float(slow[0]))
+    again = _run(x, w, lab)
+    assert all(torch.equal(a, b) for a, b in zip(fast, again))
+    with torch.no_grad():
+        from sisa_amd.kernels.linear_ce import linear_cross_entropy
+        assert torch.equal(linear_cross_entropy(x, w.float(), lab), fast[0])
+        assert torch.equal(linear_cross_entropy(*_poison(x, w, lab)[:2], _poison(x, w, lab)[2]), slow[0])
+
+
+@pytest.mark.gpu
+def test_chunks_of_both_kinds_and_a_hopeless_label():
+    """Chunks decide for themselves (dW accumulates over both kinds); a valid row whose label lies 200 below its
+    largest logit is exact in the second way."""
+    x, w, lab = _poison(*_case(500, 256, 2000, 9))
+    order = torch.randperm(501, generator=torch.Generator().manual_seed(1)).to(DEV)
+    x, lab = x[order], lab[order]
+    ref = _truth(x, w, lab)
+    got = _run(x, w, lab, chunk_tokens=128)
+    assert _rel(got[1], ref[1]) <= 3 * 2 ** -8 and _rel(got[2], ref[2]) <= 3 * 2 ** -8
+    hard = lab.clone()
+    hard[int((order == 500).nonzero())] = 0                 # the poison row's lowest logit as its label
+    ref, got = _truth(x, w, hard), _run(x, w, hard)
+    assert float(ref[0]) > 0.25 and abs(float(got[0] - ref[0])) <= 2 ** -8 * float(ref[0])
+    assert _rel(got[1], ref[1]) <= 3 * 2 ** -8 and _rel(got[2], ref[2]) <= 3 * 2 ** -8
+    bad = lab.clone()
+    bad[7] = 2000                                           # outside the vocabulary: NaN loss, as without it
+    assert not bool(torch.isfinite(_run(x, w, bad)[0]))
