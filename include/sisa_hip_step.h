@@ -57,6 +57,31 @@ typedef struct {
 
 int sisa_cache_fill(const sisa_cache_fill_args* a, void* stream);
 
+/* A prompt of B rows of L positions through a decoder layer with an empty cache, all tensors in one 16-bit dtype: the
+ * layer as above for every position (attention among the prompt's own), its cache filled. Outputs: h, the residual
+ * stream after the attention; act, silu(w_gate m) * (w_up m), zero in columns FF .. act_ld - 1; and, unless ffn is
+ * NULL, ffn = w_down act. rise_ok (or NULL): one byte, whether the cumulative log-decay g nowhere rises by more than
+ * rise_tol between neighbours (left alone for L = 1). */
+#define SISA_PREFILL_MAX_ROWS 8192
+typedef struct {
+    int32_t B, L, H, FF;
+    int32_t dtype;             /* SISA_BF16 or SISA_F16 */
+    float eps_attn, eps_ffn, rise_tol;
+    const void *x, *res;               /* (B*L, D) contiguous; res added to x first, or NULL */
+    const void *attn_norm, *w_q, *w_k, *w_v, *w_b, *w_c, *w_theta, *w_alpha, *b_alpha, *w_forget, *b_forget, *w_o;
+    const void *ffn_norm, *w_gate, *w_up, *w_down;     /* all contiguous, (outputs, inputs) */
+    const float* lambda_raw;           /* (H) */
+    sisa_view k, v, b, g, f;           /* cache slabs (B,H,capacity,64|64|32) in dtype, (B,H,capacity) fp32 */
+    float* phi;                        /* (B,H,16) contiguous: phase at position L - 1 */
+    void *h, *act, *ffn;               /* (B*L, D), (B*L, act_ld), (B*L, D) */
+    int64_t act_ld;                    /* FF rounded up to a multiple of 64 */
+    unsigned char* rise_ok;
+    void* workspace;                   /* sisa_prefill_workspace_bytes(B,L,H), 256-byte aligned */
+} sisa_prefill_args;
+
+int64_t sisa_prefill_workspace_bytes(int32_t B, int32_t L, int32_t H);
+int sisa_prefill(const sisa_prefill_args* a, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -129,6 +129,17 @@ class StepArgs(Structure):
                 ("phi_out", c_void_p), ("h", c_void_p), ("ffn", c_void_p), ("workspace", c_void_p)]
 
 
+class PrefillArgs(Structure):
+    _fields_ = [("B", c_int32), ("L", c_int32), ("H", c_int32), ("FF", c_int32), ("dtype", c_int32),
+                ("eps_attn", c_float), ("eps_ffn", c_float), ("rise_tol", c_float), ("x", c_void_p), ("res", c_void_p),
+                *((n, c_void_p) for n in ("attn_norm", "w_q", "w_k", "w_v", "w_b", "w_c", "w_theta", "w_alpha",
+                                          "b_alpha", "w_forget", "b_forget", "w_o", "ffn_norm", "w_gate", "w_up",
+                                          "w_down", "lambda_raw")),
+                ("k", View), ("v", View), ("b", View), ("g", View), ("f", View), ("phi", c_void_p), ("h", c_void_p),
+                ("act", c_void_p), ("ffn", c_void_p), ("act_ld", c_int64), ("rise_ok", c_void_p),
+                ("workspace", c_void_p)]
+
+
 class CacheFillArgs(Structure):
     _fields_ = [("B", c_int32), ("H", c_int32), ("L", c_int32), ("dtype", c_int32), ("proj", c_void_p),
                 ("s_b", c_int64), ("s_l", c_int64), ("col_k", c_int32), ("col_v", c_int32), ("br", c_void_p),
@@ -178,6 +189,8 @@ SIGNATURES = {
 STEP_SIGNATURES = {
     "sisa_step_workspace_bytes": ([c_int32, c_int32, c_int32, c_int32, c_int32], c_int64),
     "sisa_step": ([POINTER(StepArgs), c_void_p], c_int),
+    "sisa_prefill_workspace_bytes": ([c_int32, c_int32, c_int32], c_int64),
+    "sisa_prefill": ([POINTER(PrefillArgs), c_void_p], c_int),
     "sisa_cache_fill": ([POINTER(CacheFillArgs), c_void_p], c_int),
 }
 

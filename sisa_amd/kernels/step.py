@@ -1,6 +1,7 @@
-"""Generation on the HIP kernels of csrc/step.hip: one new token of every row through a whole decoder layer with a
-filled cache (``sisa_step``, seven launches behind one C call), and the filling of a layer's cache after a prefill on
-the fused route (``sisa_cache_fill``). The module path these stand in for is src/sisa/modeling.py:171-199, 224-238,
+"""Generation on the HIP kernels of csrc/step.hip and csrc/prefill.hip: one new token of every row through a whole
+decoder layer with a filled cache (``sisa_step``, seven launches behind one C call), a prompt through a layer with an empty
+one (``sisa_prefill``, thirteen), and the filling of a layer's cache after a prefill on the fused route
+(``sisa_cache_fill``). The module path these stand in for is src/sisa/modeling.py:171-199, 224-238,
 288-291; there a layer's step is about seventy torch kernels, whose launches cost four times what they compute.
 
 Both write into the cache's slabs in place and are for inference: the callers check that no gradient is wanted and
@@ -9,6 +10,7 @@ that nothing observes the modules they pass by (:func:`unobserved`, :func:`step_
 from __future__ import annotations
 
 import torch
+import torch.nn.functional as F
 from torch import Tensor, nn
 from torch.nn.modules import module as _nn_module
 
@@ -17,9 +19,13 @@ from . import _lib
 from . import attention as A
 from . import fused_prep as P
 
-__all__ = ["unobserved", "plain", "plain_linears", "rows_ok", "step_weights", "layer_step", "prefill", "MAX_ROWS", "MAX_WIDTH"]
+__all__ = ["unobserved", "plain", "plain_linears", "rows_ok", "whole", "step_weights", "layer_step", "layer_prefill", "prefill", "MAX_ROWS", "MAX_WIDTH", "PREFILL_ROWS"]
 
 MAX_ROWS, MAX_WIDTH = 64, 1024          # SISA_STEP_MAX_ROWS, SISA_STEP_MAX_D
+#: Prompts of at most this many tokens (all rows together) take ``sisa_prefill``: as far as it was measured ahead of the
+#: launch-by-launch route, whose library GEMMs gain on it with size (whole model, ms: 800 tokens at width 768 2.0 against
+#: 5.1, 8,192 tokens as 8 x 1,024 4.6 against 5.5; width 1,024 3.6 against 10.3 and 10.3 against 12.9).
+PREFILL_ROWS = 8192
 
 
 def unobserved(x: Tensor) -> bool:
@@ -53,6 +59,11 @@ def plain_linears(attn: dict, ffn: dict) -> list[dict] | None:
                 return None
             out.append(m._parameters)
     return out
+
+
+def whole(x: Tensor | None) -> bool:
+    """``x`` is contiguous and 16-byte aligned (or None)."""
+    return x is None or (x.is_contiguous() and x.data_ptr() % 16 == 0)
 
 
 def rows_ok(x: Tensor) -> bool:
@@ -104,6 +115,40 @@ def layer_step(x: Tensor, res: Tensor | None, weights: list[int], d_ff: int, lam
                          phi_out.data_ptr(), h.data_ptr(), ffn.data_ptr(), ws.data_ptr())
     _lib.call("sisa_step", args, x)
     return h, ffn, phi_out
+
+
+def layer_prefill(x: Tensor, res: Tensor | None, weights: list[int], d_ff: int, lambda_raw: Tensor, w_down: Tensor,
+                  eps: tuple[float, float], cache, layer_idx: int, checked: bool) -> tuple[Tensor, Tensor]:
+    """A prompt ``x`` ``(B, L, D)`` (contiguous; plus ``res``, added first) through a layer whose cache entry is empty,
+    filling it; ``weights`` as for :func:`layer_step`. Returns ``(h, f)``: the residual stream after the attention and the
+    FFN output still to be added to it. ``checked``: assert on the device that ``g`` does not rise."""
+    B, L, D = x.shape
+    H, dev = D // HIP_D_HEAD, x.device
+    ld = -(-d_ff // 64) * 64
+    h = torch.empty_like(x)
+    f = torch.empty_like(x) if d_ff % 8 == 0 else None
+    act = torch.empty((B, L, ld), device=dev, dtype=x.dtype)
+    phi = torch.empty((B, H, HIP_D_STATE // 2), device=dev, dtype=torch.float32)
+    ok = torch.empty((1,), device=dev, dtype=torch.bool) if checked and L > 1 else None
+    ws = torch.empty((_lib.load().sisa_prefill_workspace_bytes(B, L, H),), device=dev, dtype=torch.uint8)
+    like = x.new_empty((B, H, 0, HIP_D_HEAD))
+    gates = torch.empty((B, H, 0), device=dev, dtype=torch.float32)
+    slab = cache.room(layer_idx, L, dict(k=like, v=like, b=x.new_empty((B, H, 0, HIP_D_STATE)), g=gates, fgate=gates),
+                      phi)
+    buf = slab.buffers
+    args = _lib.PrefillArgs(B, L, H, d_ff, _lib.dtype_code(x.dtype), *eps, A.MONOTONE_TOL, x.data_ptr(), _lib.ptr(res),
+                            *weights, lambda_raw.data_ptr(),
+                            *(_lib.view(buf[n]) for n in ("k", "v", "b", "g", "fgate")), phi.data_ptr(), h.data_ptr(),
+                            act.data_ptr(), _lib.ptr(f), ld, _lib.ptr(ok), ws.data_ptr())
+    try:
+        _lib.call("sisa_prefill", args, x)
+    except RuntimeError:
+        cache._slabs.pop(layer_idx, None)          # still an empty entry
+        raise
+    if ok is not None:
+        torch._assert_async(ok, "sisa_attention_hip: the cumulative log-decay g increases along the sequence")
+    slab.filled = L
+    return h, F.linear(act[..., :d_ff], w_down) if f is None else f
 
 
 def prefill(proj: Tensor, z: Tensor, lam: Tensor, n_head: int, cache, layer_idx: int) -> Tensor:

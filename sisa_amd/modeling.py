@@ -322,9 +322,10 @@ class SISABlock(nn.Module):
 
     def _forward_cached_hip(self, x: Tensor, res: Tensor | None, cache: "SISACache"):
         """Generation on HIP kernels, or None where it does not apply. A prompt (empty cache entry) takes
-        :meth:`_forward_hip` with the cache filled from the fused projections; one new position of at most 64 rows of
-        a 16-bit model takes ``sisa_step``. Both return ``(h, f)`` as :meth:`_forward_hip` with ``defer``. Only for
-        inference with nothing watching the modules in between: other calls take the module path."""
+        ``sisa_prefill`` in a 16-bit model while it is short, else :meth:`_forward_hip` with the cache filled from the
+        fused projections; one new position of at most 64 rows of a 16-bit model takes ``sisa_step``. All return
+        ``(h, f)`` as :meth:`_forward_hip` with ``defer``. Only for inference with nothing watching the modules in
+        between: other calls take the module path."""
         from .generation import SISACache
         from .kernels import step
 
@@ -339,14 +340,21 @@ class SISABlock(nn.Module):
         linears = step.plain_linears(at._modules, ffn._modules)
         if linears is None:
             return None
-        slab = cache._slabs.get(at.layer_idx)
-        if slab is None:
-            return self._forward_hip(x, res, defer=True, cache=cache)
+        slab, mode = cache._slabs.get(at.layer_idx), backends.get_check_mode()
         B, L, D = x.shape
-        H, lam, buf = self.config.n_head, at.lambda_raw, slab.buffers
-        if L != 1 or B > step.MAX_ROWS or D > step.MAX_WIDTH or slab.filled < 1 or x.dtype not in _LOW_PRECISION \
-                or torch.is_autocast_enabled("cuda") or not step.rows_ok(x) or lam.dtype != torch.float32 \
-                or lam.shape != (H,) or lam.get_device() != x.get_device() or not lam.is_contiguous():
+        H, lam = self.config.n_head, at.lambda_raw
+        native = (x.dtype in _LOW_PRECISION and not torch.is_autocast_enabled("cuda") and lam.dtype == torch.float32
+                  and lam.shape == (H,) and lam.get_device() == x.get_device() and lam.is_contiguous())
+        if slab is None:
+            native = native and B * L <= step.PREFILL_ROWS and mode != "sync" and step.whole(x) and step.whole(res)
+            weights = native and step.step_weights(linears, n1._parameters["weight"], n2._parameters["weight"], H, x)
+            if not weights:
+                return self._forward_hip(x, res, defer=True, cache=cache)
+            return step.layer_prefill(x, res, *weights, lam, ffn.w_down.weight, (n1.eps, n2.eps), cache, at.layer_idx,
+                                      mode == "async")
+        buf = slab.buffers
+        if not native or L != 1 or B > step.MAX_ROWS or D > step.MAX_WIDTH or slab.filled < 1 or not step.rows_ok(x) \
+                or not step.whole(res):
             return None
         if buf["k"].dtype != x.dtype or buf["k"].shape[:2] != (B, H) or buf["k"].get_device() != x.get_device():
             return None

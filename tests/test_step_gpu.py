@@ -39,7 +39,7 @@ def _watched(model):
     return [blk.attn.W_Q.register_forward_hook(lambda *a: None) for blk in model.layers]
 
 
-# rows: one, two and four column groups of the products and their edges; widths below and above eight 32-element steps,
+# prompts of 1 to 1,105 rows (tiles of 128, remainders of 1 to 127); rows: one, two and four column groups of the products and their edges; widths below and above eight 32-element steps,
 # a head count that is not a multiple of the 16-row groups' 16; hidden widths that are no multiple of 32, 16, 8 or 2;
 # prompts of one position, of a chunk's edge and past it
 @pytest.mark.gpu
@@ -53,20 +53,24 @@ def test_step_matches_modules(B, H, d_ff, prompt, steps, dtype, monkeypatch):
     ref = M64.logits64(model, M64.params64(model, requires_grad=False), ids)
     calls = _count(monkeypatch)
     got, cache = _decode(model, ids, prompt, None if B % 2 else prompt + steps)
-    assert calls["sisa_step"] == 2 * steps and calls["sisa_cache_fill"] == 2
-    assert "sisa_decode_attn" not in calls
+    assert calls["sisa_step"] == 2 * steps and calls["sisa_prefill"] == 2
+    assert "sisa_decode_attn" not in calls and "sisa_attn_fwd" not in calls
+    monkeypatch.setattr("sisa_amd.kernels.step.PREFILL_ROWS", 0)       # the long prompts' route: fused, launch by launch
+    calls.clear()
+    long, held = _decode(model, ids, prompt)
+    assert calls["sisa_step"] == 2 * steps and calls["sisa_cache_fill"] == 2 and "sisa_prefill" not in calls
     hooks = _watched(model)
     calls.clear()
     want, kept = _decode(model, ids, prompt)
-    assert "sisa_step" not in calls and "sisa_cache_fill" not in calls and calls["sisa_decode_attn"] == 2 * steps
+    assert not {"sisa_step", "sisa_cache_fill", "sisa_prefill"} & set(calls) and calls["sisa_decode_attn"] == 2 * steps
     for h in hooks:
         h.remove()
     # both round the same quantities to the compute dtype: neither is further from fp64 than the other by more than
     # the spread of such errors over a few hundred logits
     assert rel_err(got, ref) <= 1.25 * rel_err(want, ref) + 1e-3
+    assert rel_err(long, ref) <= 1.25 * rel_err(want, ref) + 1e-3
     eps = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
-    for layer in range(2):
-        a, b = cache.get(layer), kept.get(layer)
+    for a, b in ((c.get(layer), kept.get(layer)) for layer in range(2) for c in (cache, held)):
         assert a.length == b.length == prompt + steps
         error = {n: rel_err(getattr(a, n), getattr(b, n)) for n in ("k", "v", "b", "g", "fgate", "phi")}
         # two roundings to the compute dtype each side; a phase that is off by d radians turns b~ by d more, and the
@@ -111,6 +115,10 @@ def test_calls_that_keep_the_module_path(monkeypatch):
 def test_step_refuses_what_it_cannot_run():
     from sisa_amd.kernels import _lib
     x = torch.zeros(1, 64, device=DEV, dtype=torch.bfloat16)
+    for bad in (dict(B=0), dict(L=0), dict(B=100, L=100), dict(dtype=_lib.F32), dict(H=65), {}):
+        args = _lib.PrefillArgs(**{**dict(B=1, L=4, H=1, FF=64, dtype=_lib.BF16, act_ld=64), **bad})
+        with pytest.raises(RuntimeError):
+            _lib.call("sisa_prefill", args, x)
     for bad in (dict(B=0), dict(B=65), dict(D=63), dict(D=64 * 17, H=17), dict(pos=0), dict(dtype=_lib.F32), {}):
         args = _lib.StepArgs(**{**dict(B=1, H=1, D=64, FF=64, dtype=_lib.BF16, pos=1), **bad})
         with pytest.raises(RuntimeError):
@@ -119,7 +127,8 @@ def test_step_refuses_what_it_cannot_run():
 
 def test_step_struct_layout_matches_c(tmp_path):
     from sisa_amd.kernels import _lib
-    pairs = {"StepArgs": "sisa_step_args", "CacheFillArgs": "sisa_cache_fill_args"}
+    pairs = {"StepArgs": "sisa_step_args", "CacheFillArgs": "sisa_cache_fill_args",
+             "PrefillArgs": "sisa_prefill_args"}
     lines, expect = ["#include <stdio.h>", "#include <stddef.h>", '#include "sisa_hip_step.h"', "int main(void) {"], []
     for py, c in pairs.items():
         cls = getattr(_lib, py)
