@@ -194,6 +194,12 @@ STEP_SIGNATURES = {
     "sisa_cache_fill": ([POINTER(CacheFillArgs), c_void_p], c_int),
 }
 
+# the cross-entropy's scalars (include/sisa_hip_ce.h)
+CE_SIGNATURES = {
+    "sisa_ce_count": ([c_void_p, c_int64, c_int64, c_void_p, c_void_p, c_void_p], c_int),
+    "sisa_ce_mean": ([c_void_p, c_int64, c_void_p, c_void_p, c_void_p], c_int),
+}
+
 _LOCK = threading.Lock()
 _LIB = None
 
@@ -209,7 +215,8 @@ def load() -> ctypes.CDLL:
         if not os.path.exists(LIB_PATH):
             raise RuntimeError(f"SISA HIP library not built: {LIB_PATH} is missing (run sisa_amd.build.build())")
         lib = ctypes.CDLL(LIB_PATH)
-        for name, (argtypes, restype) in (*SIGNATURES.items(), *STEP_SIGNATURES.items()):
+        for name, (argtypes, restype) in (*SIGNATURES.items(), *STEP_SIGNATURES.items(),
+                                           *CE_SIGNATURES.items()):
             fn = getattr(lib, name)
             fn.argtypes = argtypes
             fn.restype = restype
@@ -251,8 +258,13 @@ def launch(fn, tensor: torch.Tensor, *args) -> int:
 
 
 def call(name: str, args, dev_tensor: torch.Tensor) -> None:
+    call_values(name, dev_tensor, ctypes.byref(args))
+
+
+def call_values(name: str, dev_tensor: torch.Tensor, *values) -> None:
+    """An entry point that takes its arguments one by one."""
     lib = load()
-    rc = launch(getattr(lib, name), dev_tensor, ctypes.byref(args))
+    rc = launch(getattr(lib, name), dev_tensor, *values)
     if rc != 0:
         msg = lib.sisa_last_error().decode(errors="replace")
         raise RuntimeError(f"{name} failed (code {rc}): {msg}")

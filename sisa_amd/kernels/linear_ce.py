@@ -45,6 +45,8 @@ __all__ = ["linear_cross_entropy", "reference_linear_cross_entropy", "lmce_rows"
 VOCAB_MULTIPLE = 128
 HIDDEN_MULTIPLE = 64             # the CE kernels stream the hidden size in 64-wide stages
 PROBS_BUDGET = 2 << 30           # bytes of one chunk of stored exponentials
+SCALAR_ROWS = 1 << 17            # rows up to which one workgroup counts the valid ones and averages the loss: 16 and
+                                 # 8 loads a thread deep there, still less than the launches of the general sums
 
 
 # ------------------------------------------------------------------------------------------------ pieces
@@ -140,7 +142,7 @@ def train_workspace(chunk_sizes, Vp: int, D: int, device, dx_splits: int = 0) ->
 
 class _Problem:
     """One call's operands in the compute dtype: x (N, D) contiguous, the padded weight, int64 labels, and the
-    device scalars N_valid and 1/N_valid."""
+    device scalars N_valid and 1/N_valid (fp32)."""
 
     def __init__(self, hidden: torch.Tensor, weight: torch.Tensor, labels: torch.Tensor, ignore_index: int,
                  cdtype: torch.dtype):
@@ -154,11 +156,27 @@ class _Problem:
         self.labels = labels.reshape(-1).to(torch.int64).contiguous()
         self.V, self.ignore_index = weight.shape[0], int(ignore_index)
         self.N, self.D = self.x.shape[0], D
-        self.n_valid = (self.labels != self.ignore_index).sum()
+        self.n_valid, self.inv_n = self._count()
+
+    def _count(self) -> tuple[torch.Tensor, torch.Tensor]:
+        """The number of valid rows and its reciprocal, fp32 device scalars of one element."""
+        if self.N > SCALAR_ROWS:
+            n_valid = (self.labels != self.ignore_index).sum().to(torch.float32).reshape(1)
+            return n_valid, torch.reciprocal(n_valid)
+        n_valid, inv_n = torch.empty(2, dtype=torch.float32, device=self.x.device).split(1)
+        _lib.call_values("sisa_ce_count", self.labels, self.labels.data_ptr(), self.N, self.ignore_index,
+                         n_valid.data_ptr(), inv_n.data_ptr())
+        return n_valid, inv_n
+
+    def _mean(self, rows: torch.Tensor) -> torch.Tensor:
+        if self.N > SCALAR_ROWS:
+            return rows.sum() / self.n_valid[0]
+        mean = torch.empty((), dtype=torch.float32, device=rows.device)
+        _lib.call_values("sisa_ce_mean", rows, rows.data_ptr(), self.N, self.n_valid.data_ptr(), mean.data_ptr())
+        return mean
 
     def loss_without_grad(self) -> torch.Tensor:
-        rows = lmce_fused_loss_rows(self.x, self.wpad, self.labels, self.V, self.ignore_index)
-        return rows.sum() / self.n_valid
+        return self._mean(lmce_fused_loss_rows(self.x, self.wpad, self.labels, self.V, self.ignore_index))
 
     def loss_and_grads(self, want_dx: bool, want_dw: bool, gscale: float, chunk_tokens: int | None):
         """The chunk loop: loss and, as requested, dL/dx (N, D) and dL/dW_pad (Vp, D) in fp32 for a unit seed
@@ -168,19 +186,18 @@ class _Problem:
         rows = torch.empty(N, dtype=torch.float32, device=dev)
         dx = torch.empty((N, Dp), dtype=torch.float32, device=dev) if want_dx else None
         dw = (torch.zeros if N == 0 else torch.empty)((Vp, Dp), dtype=torch.float32, device=dev) if want_dw else None
-        inv_n = torch.reciprocal(self.n_valid.to(torch.float32)).reshape(1)
         step = chunk_rows(N, Vp, chunk_tokens, self.wpad.element_size())
         if N:
             ws = train_workspace({min(step, N), N - (N - 1) // step * step}, Vp, Dp, dev)   # this loop's chunk sizes
             for r0 in range(0, N, step):
                 r1 = min(N, r0 + step)
-                lmce_train_chunk(self.x[r0:r1], self.wpad, self.labels[r0:r1], self.V, self.ignore_index, inv_n,
+                lmce_train_chunk(self.x[r0:r1], self.wpad, self.labels[r0:r1], self.V, self.ignore_index, self.inv_n,
                                  gscale, rows[r0:r1], None if dx is None else dx[r0:r1], dw, r0 > 0, ws)
         if dx is not None and Dp != self.D:
             dx = dx[:, :self.D]
         if dw is not None and Dp != self.D:
             dw = dw[:, :self.D]
-        return rows.sum() / self.n_valid, dx, dw
+        return self._mean(rows), dx, dw
 
 
 class _LinearCE(torch.autograd.Function):

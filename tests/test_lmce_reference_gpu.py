@@ -87,3 +87,23 @@ def test_chunks_of_both_kinds_and_a_hopeless_label():
     bad = lab.clone()
     bad[7] = 2000                                           # outside the vocabulary: NaN loss, as without it
     assert not bool(torch.isfinite(_run(x, w, bad)[0]))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("N", [0, 1, 63, 1024, 8191, 8193, 100001])
+def test_scalars(N):
+    """The valid-row count, its reciprocal and the mean loss over remainders of the workgroup's 1,024 and 8,192."""
+    from sisa_amd.kernels import _lib
+    gen = torch.Generator().manual_seed(N)
+    lab = torch.randint(-1, 3, (N,), generator=gen).to(DEV)
+    rows = (10 + torch.randn(N, generator=gen)).to(DEV)
+    n, inv, mean = torch.empty(3, device=DEV).split(1)
+    _lib.call_values("sisa_ce_count", n, lab.data_ptr(), N, -1, n.data_ptr(), inv.data_ptr())
+    _lib.call_values("sisa_ce_mean", n, rows.data_ptr(), N, n.data_ptr(), mean.data_ptr())
+    count = int((lab != -1).sum())
+    assert float(n) == count and torch.equal(inv, torch.reciprocal(n))
+    want = rows.double().sum() / count
+    if count:       # one rounding of the sum, one of the quotient
+        assert abs(float(mean) - float(want)) <= 2 * 2.0 ** -24 * abs(float(want))
+    else:
+        assert not bool(torch.isfinite(mean))
