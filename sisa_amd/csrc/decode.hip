@@ -37,10 +37,21 @@ SISA_DEV float wave_sum(float x) {
     return x;
 }
 
+// The cached rows are read once per step. A cache larger than the 256 MB last-level cache cannot be found there at the
+// next step, so from that size its rows are loaded with the non-temporal hint and displace nothing on their way.
+// Measured with 8 x 12 heads in bf16: 516 MB 108.9 -> 99.0 us (4.7 -> 5.2 TB/s), and 108.6 -> 100.5 with several such
+// caches in turn. Below the line it depends on the caller: 258 MB read again and again 51.1 -> 53.2, in turn with
+// others 58.6 -> 54.2; 16 MB 9.3 -> 10.3 and 11.2 -> 11.2.
+constexpr int64_t STREAM_BYTES = (int64_t)256 << 20;
+template <class T, bool STREAM> SISA_DEV frag8<T> row8(const T* p) {
+    if constexpr (STREAM) return __builtin_nontemporal_load(reinterpret_cast<const frag8<T>*>(p));
+    else return load8<T>(p);
+}
+
 // Occupancy hint 3 (the 132 registers allow three waves per SIMD either way): the schedule made for that register
-// target runs the config-4 decode step 2-4 % faster than the one made without the hint; forcing four waves (128
-// registers) makes it 15 % slower.
-template <class T>
+// target runs a decode step of 8 x 12 heads at 16,384 positions 2-4 % faster than the one made without the hint; forcing
+// four waves (128 registers) makes it 15 % slower.
+template <class T, bool STREAM>
 __global__ __launch_bounds__(64 * DW) __attribute__((amdgpu_waves_per_eu(3)))
 void decode_chunk_kernel(sisa_decode_args a) {
     __shared__ float wm[DW], wl[DW], wo[DW][DH];
@@ -70,9 +81,9 @@ void decode_chunk_kernel(sisa_decode_args a) {
     for (int i = 0; i < 8; ++i) {
         const int jj = jw + kq + 8 * i;
         if (jj < a.N && jj <= last) {
-            kr[i] = load8<T>(kbase + (int64_t)jj * a.k.sl + 8 * fg);
-            vr[i] = load8<T>(vbase + (int64_t)jj * a.v.sl + 8 * fg);
-            if (fg < DS / 8) br[i] = load8<T>(bbase + (int64_t)jj * a.b.sl + 8 * fg);
+            kr[i] = row8<T, STREAM>(kbase + (int64_t)jj * a.k.sl + 8 * fg);
+            vr[i] = row8<T, STREAM>(vbase + (int64_t)jj * a.v.sl + 8 * fg);
+            if (fg < DS / 8) br[i] = row8<T, STREAM>(bbase + (int64_t)jj * a.b.sl + 8 * fg);
         }
     }
     // per-key scalars with lane = key: lam * exp(g_m - g_j) and F_m - F_j
@@ -210,7 +221,11 @@ template <class T, class TO>
 int launch_decode(const sisa_decode_args* a, TO* out, hipStream_t st) {
     const int nchunk = (int)sisa::cdiv(a->N, KCH);
     const int rows = a->B * a->H * a->M;
-    decode_chunk_kernel<T><<<dim3((unsigned)nchunk, (unsigned)rows), 64 * DW, 0, st>>>(*a);
+    const dim3 grid((unsigned)nchunk, (unsigned)rows);
+    // M > 1: the rows of a head share its cache, which the caches then serve
+    const int64_t bytes = (int64_t)a->B * a->H * a->N * ((2 * DH + DS) * (int64_t)sizeof(T) + 8);
+    if (a->M == 1 && bytes >= STREAM_BYTES) decode_chunk_kernel<T, true><<<grid, 64 * DW, 0, st>>>(*a);
+    else decode_chunk_kernel<T, false><<<grid, 64 * DW, 0, st>>>(*a);
     const int rc = sisa::launch_status("sisa_decode_attn");
     if (rc) return rc;
     decode_combine_kernel<TO><<<(unsigned)rows, 64, 0, st>>>(*a, out, nchunk);

@@ -112,6 +112,28 @@ def test_calls_that_keep_the_module_path(monkeypatch):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("dtype,N", [(torch.bfloat16, 54560), (torch.bfloat16, 54561), (torch.float32, 27617)])
+def test_decode_at_the_streaming_line(dtype, N):
+    """Caches just below and above 256 MiB (15 heads: 4,920 or 9,720 bytes a position) give each row what its head alone,
+    far below it, gives: the loads' cache policy is all that changes."""
+    from sisa_amd.kernels.decode import sisa_decode_hip
+    gen = torch.Generator(device=DEV).manual_seed(3)
+
+    def draw(*shape, dt=dtype):
+        return torch.randn(shape, generator=gen, device=DEV).to(dt)
+    H = 15
+    k, v, b = draw(1, H, N, 64), draw(1, H, N, 64), draw(1, H, N, 32)
+    q, c, lam = draw(1, H, 1, 64), draw(1, H, 1, 32), draw(H, dt=torch.float32).abs()
+    g, f = (-0.01 * draw(1, H, N, dt=torch.float32).abs().cumsum(2) for _ in range(2))
+    out = sisa_decode_hip(q, k, v, c, b, g[:, :, -1:], g, lam, f[:, :, -1:], f, N - 1)
+    for h in (0, 7, 14):
+        s = slice(h, h + 1)
+        one = sisa_decode_hip(q[:, s], k[:, s], v[:, s], c[:, s], b[:, s], g[:, s, -1:], g[:, s], lam[s], f[:, s, -1:],
+                              f[:, s], N - 1)
+        assert torch.equal(out[:, s], one)
+
+
+@pytest.mark.gpu
 def test_step_refuses_what_it_cannot_run():
     from sisa_amd.kernels import _lib
     x = torch.zeros(1, 64, device=DEV, dtype=torch.bfloat16)
