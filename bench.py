@@ -212,7 +212,7 @@ def bench_ce(steps: int, warmup: int) -> dict:
 
     train: the loss with both gradients as linear_cross_entropy runs it -- sisa_lmce_train over the chunk(s) of at
     most 2 GiB of stored exponentials (one chunk here): the logits GEMM storing the exponentials, the split combine,
-    the scale pass, the dW + dx MFMA launch forming G in operand staging, the dx split sum. Each call queued behind a
+    the row-scaled copy of x, the dW + dx MFMA launch over the exponentials, the label terms, the dx split sum. Each call queued behind a
     GPU spin (HIP events). phases_ms: the forward part (the same call without dx and dW) and the rest. Beside it the
     reference's arrangement on this GPU (library_chunk_loop_ms: hipBLASLt logits GEMM, the HIP row pass writing G over
     the logits, hipBLASLt dx and dW GEMMs; chunks of 1 GiB of logits), the design this pass replaces.
@@ -278,7 +278,7 @@ def bench_ce(steps: int, warmup: int) -> dict:
     return {"workload": "linear cross-entropy (config 3): N=16384, d=768, V=50277, bf16", "N": N, "d": D, "V": V,
             "Vp": Vp,
             "train": {"what": "loss, dx, dW: sisa_lmce_train (MFMA logits GEMM storing exponentials; one launch of "
-                              "dW and dx MFMA tiles forming G in operand staging; no library GEMM)",
+                              "dW and dx MFMA tiles over them; no library GEMM)",
                       "chunk_rows": rows, "ms_per_step": round(ms, 4), "tflops": round(tr_tf, 2),
                       "tokens_per_s": round(N / train_s, 1),
                       "phases_ms": {"forward": round(fwd_s * 1e3, 4), "gradients": round((train_s - fwd_s) * 1e3, 4)},
