@@ -308,11 +308,13 @@ __global__ __launch_bounds__(64 * NWC) void lmce_fwd_kernel(sisa_lmce_fwd_args a
 // keeps lse in log2 units and the row's gradient scale (0 for an ignored row, else inv_n * gscale).
 struct CeTrainRows {
     float* lse2;                  // (N,) or nullptr (the no-gradient pass)
-    float2* rinfo;                // (N,): s_n, and the label as the bit pattern of an int (-1 outside [0, V))
+    float2* rinfo;                // (N,): s_n (REF with cn: s_n (1 - p_label), what G holds at the label, negated), and
+                                  // the label as the bit pattern of an int (-1 outside [0, V))
     const float* inv_n;           // device scalar 1 / N_valid
     float gscale;
     const float* ref;             // REF: (N,) the reference of the row's exponentials, log2 units
     float* cn;                    // REF: (N,) s_n / Z_n, or nullptr
+    __bf16* probs;                // REF with cn: the stored exponentials (N, Vp); the label's is zeroed here
     int* flag;                    // REF: set when a row's sum is not one the reference was good for
     const int* gate;              // run only if *gate is nonzero (null: always)
 };
@@ -373,8 +375,15 @@ __global__ __launch_bounds__(CRW * CSP) void lmce_combine_kernel(sisa_lmce_fwd_a
         tr.lse2[n] = l2;
         const int lab = (y >= 0 && y < a.V) ? (int)y : -1;
         const float sn = y == a.ignore_index ? 0.f : tr.inv_n[0] * tr.gscale;
-        tr.rinfo[n] = float2{sn, __int_as_float(lab)};
-        if (REF && tr.cn) tr.cn[n] = sn / ss;
+        float gl = sn;
+        if (REF && tr.cn) {
+            tr.cn[n] = sn / ss;
+            if (lab >= 0) {   // p - 1 is formed here in fp32: taken apart, the two roundings of p would outweigh it near p = 1
+                gl = sn * (1.f - fast_exp2(fmaf(a.workspace[2 * (int64_t)S * N + n], LOG2E, -mm)) / ss);
+                tr.probs[n * a.Vp + lab] = (__bf16)0.f;
+            }
+        }
+        tr.rinfo[n] = float2{gl, __int_as_float(lab)};
     }
 }
 
@@ -457,8 +466,8 @@ int64_t lmce_fwd_ws_bytes(int64_t N, int64_t Vp) {
 // The training pass's forward: the logits GEMM storing the exponentials (probs: (N, Vp) in the compute dtype), then the
 // split combine writing the loss rows, lse in log2 units and each row's gradient scale, for bf16 also s_n / Z_n (cn).
 // Afterwards *flag (returned; null for fp16) tells on the device which exponentials probs holds: zero, those against
-// one reference per row, G = probs * cn - s_n [label]; nonzero or null, those against the tile-half maxima in mtab
-// ((2 * ceil(Vp / 256), N) fp32). a->workspace: lmce_fwd_ws_bytes.
+// one reference per row, G = probs * cn off the label, whose entry of probs is zero, and -rinfo.x at it; nonzero or null,
+// those against the tile-half maxima in mtab ((2 * ceil(Vp / 256), N) fp32). a->workspace: lmce_fwd_ws_bytes.
 int lmce_train_forward(const sisa_lmce_fwd_args* a, void* probs, float* mtab, float* lse2, float2* rinfo, float* cn,
                        const float* inv_n, float gscale, const int** flag, hipStream_t st) {
     CeTrainRows r{};
@@ -467,6 +476,7 @@ int lmce_train_forward(const sisa_lmce_fwd_args* a, void* probs, float* mtab, fl
     r.inv_n = inv_n;
     r.gscale = gscale;
     r.cn = cn;
+    r.probs = (__bf16*)probs;
     *flag = a->dtype == SISA_BF16 ? ws_flag(a) : nullptr;
     if (a->dtype == SISA_BF16)
         return launch_logits<__bf16, true>(a, (__bf16*)probs, mtab, r, ws_ref(a), ws_flag(a), st);

@@ -17,14 +17,15 @@
 //      the stored exponentials, dW tiles (256 vocabulary x 256 hidden, all rows of the chunk as K) first, then dx tiles
 //      (256 rows x 256 hidden, K = a range of the vocabulary: dx is split so that both kinds of workgroup run about
 //      equally long), both operands by buffer loads straight into LDS (plain_tile); lmce_label_dw_kernel and the dx
-//      reduction subtract the label terms in fp32 and the latter applies s_n / Z_n;
+//      reduction add the label terms s_n (p - 1) in fp32 (the combine took the label's p~ out of the buffer and formed
+//      p - 1 there) and the latter applies s_n / Z_n;
 //   3. second way: lmce_scale_kernel turns the m_t table into c = exp2(m_t - lse2) * s_n in place, so that
 //      G[n, v] = p~[n, v] * c[n, tile half of v] - s_n [v == label_n], and writes each row's label entry of G; the same
 //      launch of lmce_grad_kernel then forms G from p~ and c while staging it into LDS (grad_tile: 16-byte loads, 8
 //      multiplies, the rare label subtraction, one rounding and one 16-byte LDS store per 8 values);
 //   4. lmce_dx_reduce_kernel adds the dx splits in split order.
 // Rounding: p~ once; then x s_n / Z_n (dW) or nothing (dx) the first way, G the second; the label terms are exact to fp32
-// the first way. At 16,384 rows of 768 (V 50,277) the gradient launch takes 2,399 us the first way (1.06 PFLOP/s) and
+// the first way (rows with 1 - p near 0.008: dW off by 1e-4 of its norm; 0.29 with the label's p~ left in the products). At 16,384 rows of 768 (V 50,277) the gradient launch takes 2,399 us the first way (1.06 PFLOP/s) and
 // 3,209 the second; 157 and 204 us at 1,023 rows of 512.
 // G and the logits are never written to memory; the only large buffer is the chunk's exponentials (read once per
 // output column tile). Deterministic: no atomics.
@@ -69,7 +70,7 @@ struct __attribute__((aligned(16))) GradLds {
 struct GradArgs {
     const void* probs;              // (N, Vp) exponentials p~ in the compute dtype, row stride Vp
     const float* cs;                // (2 * tiles, N): c = exp2(m_t - lse2) * s_n
-    const float2* rinfo;            // (N,) per row: s_n, and the label (bit pattern of an int; -1 if none)
+    const float2* rinfo;            // (N,) per row: s_n (first way: s_n (1 - p_label)), and the label (bit pattern of an int; -1 if none)
     const float* glab;              // (N,) per row: G at the label, p~ * c - s_n rounded once to the compute dtype
     const int64_t* labels;
     const void* x;
@@ -384,7 +385,7 @@ __global__ __launch_bounds__(256) void lmce_xscale_kernel(const T* x, int64_t ld
     store_f32x8<T>(xs + n * D + d, v);
 }
 
-// dW[label_n, :] -= s_n x[n, :] in row order, for rows with a valid label. A workgroup owns 64 vocabulary rows and
+// dW[label_n, :] -= s_n (1 - p_n) x[n, :] (rinfo's first value) in row order, for rows with a valid label. A workgroup owns 64 vocabulary rows and
 // collects, LBATCH rows of the chunk at a time, the rows whose label is among them (in order, by ballots); wave w then adds
 // those of vocabulary rows 16 w .. 16 w + 15, each lane always the same columns, so that sums run in row order without
 // atomics. 16,384 labels over 50,304 vocabulary rows: 66 us (32 and 128 rows a workgroup: 82, 78).
@@ -471,7 +472,7 @@ __global__ __launch_bounds__(256) void lmce_scale_kernel(float* cs, const float*
 }
 
 // dx[n, :] = sum over the splits, in split order, of the partial rows; with per-row references (flag given and zero) that
-// sum is scaled by cn[n], and the label's term s_n W[label_n] subtracted
+// sum is scaled by cn[n], and the label's term s_n (1 - p_n) W[label_n] subtracted
 template <class T>
 __global__ __launch_bounds__(256) void lmce_dx_reduce_kernel(const float* part, float* dx, int64_t N, int D, int S,
                                                              int64_t lddx, const int* flag, const float* cn,

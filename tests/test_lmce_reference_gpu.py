@@ -70,6 +70,25 @@ def test_row_references_match_tile_maxima(N, D, V, one_label):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("top", [6.0, 12.0])
+def test_confident_rows(top):
+    """Rows whose label holds nearly all the probability: G at the label is p - 1, far below p, and keeps its relative
+    precision. The truth takes the logits as the kernels round them; then three 8-bit roundings, as above."""
+    _, w, lab = _case(300, 256, 1003, 5)
+    lab = lab.clamp_min(0)
+    wl = w[lab].double()
+    x = (top * wl / (wl * wl).sum(1, keepdim=True)).to(torch.bfloat16)
+    logits = (x.double() @ w.double().t()).to(torch.bfloat16).double()
+    G = torch.softmax(logits, 1)
+    rest = G.scatter(1, lab[:, None], 0.0)
+    G = rest.scatter(1, lab[:, None], -rest.sum(1, keepdim=True)) / len(lab)
+    for args in ((x, w, lab), _poison(x, w, lab)):
+        _, dx, dw = _run(*args)
+        assert _rel(dx[:300], G @ w.double()) <= 3 * 2 ** -8
+        assert _rel(dw, G.t() @ x.double()) <= 3 * 2 ** -8
+
+
+@pytest.mark.gpu
 def test_chunks_of_both_kinds_and_a_hopeless_label():
     """Chunks decide for themselves (dW accumulates over both kinds); a valid row whose label lies 200 below its
     largest logit is exact in the second way."""
