@@ -212,7 +212,7 @@ def bench_ce(steps: int, warmup: int) -> dict:
 
     train: the loss with both gradients as linear_cross_entropy runs it -- sisa_lmce_train over the chunk(s) of at
     most 2 GiB of stored exponentials (one chunk here): the logits GEMM storing the exponentials, the split combine,
-    the row-scaled copy of x, the dW + dx MFMA launch over them, the label terms, the dx split sum. Each call queued
+    the dW + dx MFMA launch over them, the dx split sum with the label terms. Each call queued
     behind a GPU spin (HIP events). phases_ms: the forward part (the same call without dx and dW) and the rest. Beside it the
     reference's arrangement on this GPU (library_chunk_loop_ms: hipBLASLt logits GEMM, the HIP row pass writing G over
     the logits, hipBLASLt dx and dW GEMMs; chunks of 1 GiB of logits), the design this pass replaces.

@@ -13,20 +13,21 @@
 //      the chunk the second way (also fp16's, whose exponent range is too small for the first): against m_t, the row's
 //      maximum over one 128-column half of a vocabulary tile, kept in a (2 * tiles, N) table. The loss rows are bitwise
 //      those of sisa_lmce_fwd either way;
-//   2. first way: lmce_xscale_kernel writes x s_n / Z_n, rounded; one launch of lmce_grad_kernel runs plain products of
-//      the stored exponentials, dW tiles (256 vocabulary x 256 hidden, all rows of the chunk as K) first, then dx tiles
-//      (256 rows x 256 hidden, K = a range of the vocabulary: dx is split so that both kinds of workgroup run about
-//      equally long), both operands by buffer loads straight into LDS (plain_tile); lmce_label_dw_kernel and the dx
-//      reduction add the label terms s_n (p - 1) in fp32 (the combine took the label's p~ out of the buffer and formed
-//      p - 1 there) and the latter applies s_n / Z_n;
+//   2. first way: the combine has taken the label's p~ out of the buffer and formed s_n (1 - p) in fp32. One launch of
+//      lmce_grad_kernel runs dW tiles (256 vocabulary x 256 hidden, all rows of the chunk as K) first, G = p~ s_n / Z_n
+//      formed while staging it into LDS (grad_tile), then dx tiles (256 rows x 256 hidden, K = a range of the vocabulary: dx
+//      is split so that both kinds of workgroup run about equally long), plain products of the stored exponentials by
+//      buffer loads straight into LDS (plain_tile); the dx reduction applies s_n / Z_n and adds the label terms in fp32;
 //   3. second way: lmce_scale_kernel turns the m_t table into c = exp2(m_t - lse2) * s_n in place, so that
 //      G[n, v] = p~[n, v] * c[n, tile half of v] - s_n [v == label_n], and writes each row's label entry of G; the same
 //      launch of lmce_grad_kernel then forms G from p~ and c while staging it into LDS (grad_tile: 16-byte loads, 8
 //      multiplies, the rare label subtraction, one rounding and one 16-byte LDS store per 8 values);
 //   4. lmce_dx_reduce_kernel adds the dx splits in split order.
-// Rounding: p~ once; then x s_n / Z_n (dW) or nothing (dx) the first way, G the second; the label terms are exact to fp32
-// the first way (rows with 1 - p near 0.008: dW off by 1e-4 of its norm; 0.29 with the label's p~ left in the products). At 16,384 rows of 768 (V 50,277) the gradient launch takes 2,399 us the first way (1.06 PFLOP/s) and
-// 3,209 the second; 157 and 204 us at 1,023 rows of 512.
+// Rounding: p~ once, then G; the first way's dx only p~, its label terms exact to fp32. A label's G, p - 1 times s_n, keeps
+// its relative precision where p is near 1 (taken from the products of two rounded numbers, dx was off by 20 % of its
+// norm and dW by 29 % for rows with 1 - p near 0.008).
+// At 16,384 rows of 768 (V 50,277) the gradient launch takes 2,737 us the first way (0.93 PFLOP/s) and 3,209 the second;
+// 175 and 204 us at 1,023 rows of 512.
 // G and the logits are never written to memory; the only large buffer is the chunk's exponentials (read once per
 // output column tile). Deterministic: no atomics.
 //
@@ -70,7 +71,8 @@ struct __attribute__((aligned(16))) GradLds {
 struct GradArgs {
     const void* probs;              // (N, Vp) exponentials p~ in the compute dtype, row stride Vp
     const float* cs;                // (2 * tiles, N): c = exp2(m_t - lse2) * s_n
-    const float2* rinfo;            // (N,) per row: s_n (first way: s_n (1 - p_label)), and the label (bit pattern of an int; -1 if none)
+    const float2* rinfo;            // (N,) per row: s_n (first way: s_n (1 - p_label)), and the label (bit pattern of an int;
+                                    // -1 if none)
     const float* glab;              // (N,) per row: G at the label, p~ * c - s_n rounded once to the compute dtype
     const int64_t* labels;
     const void* x;
@@ -83,7 +85,7 @@ struct GradArgs {
     int n_dw, n_dw_pad, n_dx;       // dW items (blocks padded to a multiple of 8), dx items
     int accumulate;
     const int* flag;                // device: nonzero = exponentials against tile-half maxima (null: always so)
-    const void* xs;                 // (N, D) x * s_n / Z_n in the compute dtype, row stride D (per-row references)
+    const float* cn;                // (N,) s_n / Z_n (per-row references)
 };
 
 SISA_DEV int64_t clamp_bytes(int64_t b) {
@@ -141,8 +143,9 @@ SISA_DEV void store_tile(const GradArgs& a, f32x4 (&acc)[IB][JB], int vt, int sp
 }
 
 // One output tile: DW (dW tile u = vocabulary tile * dts + hidden tile) or dx (u = (row block * dx_splits + split)
-// * dts + hidden tile).
-template <class T, bool DW>
+// * dts + hidden tile). ROW (dW only): the exponentials are relative to one reference per row, c = s_n / Z_n and G at the
+// label -s_n (1 - p_label).
+template <class T, bool DW, bool ROW>
 SISA_DEV void grad_tile(const GradArgs& a, GradLds<T>& sm, int u) {
     const int tid = threadIdx.x, lane = tid & 63, grp = lane >> 4, lc = lane & 15;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -197,9 +200,10 @@ SISA_DEV void grad_tile(const GradArgs& a, GradLds<T>& sm, int u) {
             for (int p = 0; p < GL; ++p) {
                 raw[p] = load16<T>(rs, (int)((rr[p] * Vp + (int64_t)vt * TV + 8 * gc) * (int64_t)sizeof(T)));
                 const int64_t n = m0 + rr[p] < N ? m0 + rr[p] : N - 1;   // rows past N: their p~ read as 0
-                cv[p] = a.cs[(int64_t)(2 * vt + h) * N + n];
-                lab[p] = m0 + rr[p] < N ? __float_as_int(a.rinfo[n].y) : -1;
-                gl[p] = a.glab[n];
+                cv[p] = ROW ? a.cn[n] : a.cs[(int64_t)(2 * vt + h) * N + n];
+                const float2 ri = a.rinfo[n];
+                lab[p] = m0 + rr[p] < N ? __float_as_int(ri.y) : -1;
+                gl[p] = ROW ? -ri.x : a.glab[n];
             }
         } else {
             const int64_t v0 = (int64_t)(k0 + g) * TK;
@@ -228,7 +232,7 @@ SISA_DEV void grad_tile(const GradArgs& a, GradLds<T>& sm, int u) {
     };
     auto issue_dense = [&](int g, int buf) {
         const int64_t k = (int64_t)(k0 + g) * TK;
-        if constexpr (DW) dma_issue<7>(dma, dsrc, dbytes, (int)(k * dld * (int64_t)sizeof(T)), sm.dense[buf], w);
+        if constexpr (DW) dma_issue<ROW ? 10 : 7>(dma, dsrc, dbytes, (int)(k * dld * (int64_t)sizeof(T)), sm.dense[buf], w);
         else dma_issue<6>(dma, dsrc, dbytes, (int)(k * dld * (int64_t)sizeof(T)), sm.dense[buf], w);
     };
 
@@ -277,46 +281,43 @@ SISA_DEV void grad_tile(const GradArgs& a, GradLds<T>& sm, int u) {
     store_tile<DW>(a, acc, vt, sp, n0, d0, wd, wo, grp, lc);
 }
 
-// One output tile when the exponentials are relative to one reference per row, G = p~ cn - s_n [label]: plain products of
-// the stored exponentials, dW = p~^T (x cn) and dx / cn = p~ W (the scale and the label terms are applied where dx is
-// reduced and by lmce_label_dw_kernel). Both operands go straight into LDS, so a stage's MFMAs have nothing beside them
-// but their fragment reads: forming G while staging it (16-byte loads to registers, 32 multiplies, packing and label
-// checks a thread and stage) kept the matrix pipe idle for a third of the launch.
-template <class T, bool DW>
+// One dx tile when the exponentials are relative to one reference per row: the plain product dx / cn = p~ W of the stored
+// exponentials (the scale and the label terms are applied where dx is reduced). Both operands go straight into LDS, so a
+// stage's MFMAs have nothing beside them but their fragment reads: forming G while staging it (16-byte loads to registers,
+// 32 multiplies, packing and label checks a thread and stage) kept the matrix pipe idle for a third of the launch. dW
+// forms G all the same (grad_tile<ROW>): a plain product needs the label terms added in fp32 by another kernel, whose chains
+// are as long as a label is frequent (a training pass of 16,384 rows: 4,124 us with uniform labels, 9,558 with labels as
+// frequent as words, 27,657 with one; 4,349, 4,319 and 4,309 this way), or rounds them twice.
+template <class T>
 SISA_DEV void plain_tile(const GradArgs& a, GradLds<T>& sm, int u) {
     const int lane = threadIdx.x & 63, grp = lane >> 4, lc = lane & 15;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int64_t N = a.N, Vp = a.Vp;
     const int dt = u % a.dts, rest = u / a.dts;
     const int d0 = dt * TD;
-    const int vt = rest, sp = rest % a.dx_splits, rb = rest / a.dx_splits;
-    const int64_t n0 = DW ? 0 : (int64_t)rb * TO;
-    const int k0 = DW ? 0 : sp * a.dx_per;
-    const int kstages = DW ? (int)((N + TK - 1) / TK) : (int)(Vp / TK);
-    const int k1 = DW ? kstages : (k0 + a.dx_per < kstages ? k0 + a.dx_per : kstages);
+    const int sp = rest % a.dx_splits, rb = rest / a.dx_splits;
+    const int64_t n0 = (int64_t)rb * TO;
+    const int k0 = sp * a.dx_per, kstages = (int)(Vp / TK);
+    const int k1 = k0 + a.dx_per < kstages ? k0 + a.dx_per : kstages;
     const int total = k1 > k0 ? k1 - k0 : 0;
     const int wd = WD * (w & 1), wo = WO * (w >> 1);
 
     DmaStage<T, TD, NWG> dma;                        // dense: 64 K-rows x 256 hidden columns
-    const T* dsrc = DW ? (const T*)a.xs + d0 : (const T*)a.w + d0;
-    const int64_t dld = DW ? a.D : a.ldw;
-    const int64_t drows = DW ? N : Vp;
-    const int64_t dbytes = ((drows - 1) * dld + a.D - d0) * (int64_t)sizeof(T);
-    dma.init(dld, w, lane);
-    // exponentials: 64 rows x 256 vocabulary columns (dW), 256 rows x 64 columns as four groups of 64 rows (dx); rows past
-    // the data read as zero, columns past Vp belong to outputs that are not stored
-    constexpr int GC = DW ? TO : TK, GG = DW ? 1 : TO / 64;
-    DmaStage<T, GC, NWG> dmg;
+    const T* dsrc = (const T*)a.w + d0;
+    const int64_t dbytes = ((Vp - 1) * a.ldw + a.D - d0) * (int64_t)sizeof(T);
+    dma.init(a.ldw, w, lane);
+    // exponentials: 256 rows x 64 columns as four groups of 64 rows; rows past the data read as zero
+    DmaStage<T, TK, NWG> dmg;
     dmg.init(Vp, w, lane);
     const T* P = (const T*)a.probs;
     auto issue = [&](int g, int buf) {
         const int64_t k = (int64_t)(k0 + g) * TK;
-        dma_issue<DW ? 10 : 11>(dma, dsrc, dbytes, (int)(k * dld * (int64_t)sizeof(T)), sm.dense[buf], w);
+        dma_issue<11>(dma, dsrc, dbytes, (int)(k * a.ldw * (int64_t)sizeof(T)), sm.dense[buf], w);
 #pragma unroll
-        for (int h = 0; h < GG; ++h) {
-            const int64_t row = DW ? k : n0 + 64 * h, col = DW ? (int64_t)vt * TV : k;
-            dma_issue<DW ? 12 : 13>(dmg, P + row * Vp + col, clamp_bytes(((N - row) * Vp - col) * (int64_t)sizeof(T)), 0,
-                                    sm.g[buf] + 64 * h * GC, w);
+        for (int h = 0; h < TO / 64; ++h) {
+            const int64_t row = n0 + 64 * h;
+            dma_issue<13>(dmg, P + row * Vp + k, clamp_bytes(((N - row) * Vp - k) * (int64_t)sizeof(T)), 0,
+                          sm.g[buf] + 64 * h * TK, w);
         }
     };
 
@@ -335,13 +336,9 @@ SISA_DEV void plain_tile(const GradArgs& a, GradLds<T>& sm, int u) {
         for (int step = 0; step < TK / 32; ++step) {
             frag8<T> af[IB], bf[JB];
 #pragma unroll
-            for (int j = 0; j < JB; ++j)
-                bf[j] = DW ? frag_tr<T, TO>(sm.g[buf], wo + 16 * j, step, lane)
-                           : frag_rows<T, TK>(sm.g[buf], wo + 16 * j, step, lane);
+            for (int j = 0; j < JB; ++j) bf[j] = frag_rows<T, TK>(sm.g[buf], wo + 16 * j, step, lane);
 #pragma unroll
-            for (int i = 0; i < IB; ++i)
-                af[i] = DW ? frag_tr<T, TD>(sm.dense[buf], wd + 16 * i, step, lane)
-                           : frag_trf<T, TD>(sm.dense[buf], wd + 16 * i, step, lane);
+            for (int i = 0; i < IB; ++i) af[i] = frag_trf<T, TD>(sm.dense[buf], wd + 16 * i, step, lane);
 #pragma unroll
             for (int i = 0; i < IB; ++i)
 #pragma unroll
@@ -349,7 +346,7 @@ SISA_DEV void plain_tile(const GradArgs& a, GradLds<T>& sm, int u) {
         }
         __syncthreads();
     }
-    store_tile<DW>(a, acc, vt, sp, n0, d0, wd, wo, grp, lc);
+    store_tile<false>(a, acc, 0, sp, n0, d0, wd, wo, grp, lc);
 }
 
 template <class T>
@@ -361,95 +358,13 @@ __global__ __launch_bounds__(64 * NWG) void lmce_grad_kernel(GradArgs a) {
     if (u < 0) return;
     if constexpr (__is_same(T, __bf16)) {
         if (a.flag && *a.flag == 0) {
-            if (dw) plain_tile<T, true>(a, sm, u);
-            else plain_tile<T, false>(a, sm, u);
+            if (dw) grad_tile<T, true, true>(a, sm, u);
+            else plain_tile<T>(a, sm, u);
             return;
         }
     }
-    if (dw) grad_tile<T, true>(a, sm, u);
-    else grad_tile<T, false>(a, sm, u);
-}
-
-// xs[n, :] = x[n, :] * cn[n], rounded once (the dense operand of dW; the other one is the rounded exponential, as G was
-// the rounded product of the two)
-template <class T>
-__global__ __launch_bounds__(256) void lmce_xscale_kernel(const T* x, int64_t ldx, const float* cn, T* xs, int64_t N,
-                                                          int D, const int* flag) {
-    if (*flag) return;
-    const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    const int q = D / 8;
-    if (idx >= N * q) return;
-    const int64_t n = idx / q;
-    const int d = 8 * (int)(idx % q);
-    const f32x8 v = load_f32x8<T>(x + n * ldx + d) * cn[n];
-    store_f32x8<T>(xs + n * D + d, v);
-}
-
-// dW[label_n, :] -= s_n (1 - p_n) x[n, :] (rinfo's first value) in row order, for rows with a valid label. A workgroup owns 64 vocabulary rows and
-// collects, LBATCH rows of the chunk at a time, the rows whose label is among them (in order, by ballots); wave w then adds
-// those of vocabulary rows 16 w .. 16 w + 15, each lane always the same columns, so that sums run in row order without
-// atomics. 16,384 labels over 50,304 vocabulary rows: 66 us (32 and 128 rows a workgroup: 82, 78).
-constexpr int LROWS = 64, LBATCH = 4096;
-template <class T>
-__global__ __launch_bounds__(256) void lmce_label_dw_kernel(const float2* rinfo, const T* x, int64_t ldx, float* dw,
-                                                            int64_t lddw, int64_t N, int D, const int* flag) {
-    if (*flag) return;
-    __shared__ int list[LBATCH], lrow[LBATCH];
-    __shared__ int count[4], base[4];
-    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-    const int v0 = blockIdx.x * LROWS;
-    constexpr int PW = LBATCH / 4;                   // consecutive rows scanned by a wave
-    for (int64_t b0 = 0; b0 < N; b0 += LBATCH) {
-        const int64_t n0 = b0 + w * PW;
-        int lab[PW / 64];
-        int cnt = 0;
-#pragma unroll
-        for (int k = 0; k < PW / 64; ++k) {
-            const int64_t n = n0 + 64 * k + lane;
-            lab[k] = n < N ? __float_as_int(rinfo[n].y) - v0 : -1;
-        }
-#pragma unroll
-        for (int k = 0; k < PW / 64; ++k) cnt += __popcll(__builtin_amdgcn_ballot_w64((unsigned)lab[k] < (unsigned)LROWS));
-        if (lane == 0) count[w] = cnt;
-        __syncthreads();
-        if (tid == 0) {
-            int s = 0;
-            for (int k = 0; k < 4; ++k) {
-                base[k] = s;
-                s += count[k];
-            }
-        }
-        __syncthreads();
-        const int total = base[3] + count[3];
-        int at = base[w];
-#pragma unroll
-        for (int k = 0; k < PW / 64; ++k) {
-            const bool hit = (unsigned)lab[k] < (unsigned)LROWS;
-            const uint64_t m = __builtin_amdgcn_ballot_w64(hit);
-            if (hit) {
-                const int p = at + __popcll(m & (((uint64_t)1 << lane) - 1));
-                list[p] = (int)(n0 - b0) + 64 * k + lane;
-                lrow[p] = lab[k];
-            }
-            at += __popcll(m);
-        }
-        __syncthreads();
-        for (int e = 0; e < total; ++e) {
-            const int r = lrow[e];
-            if (r / (LROWS / 4) != w) continue;      // wave-uniform
-            const int64_t n = b0 + list[e];
-            const float sn = rinfo[n].x;
-            float* out = dw + (int64_t)(v0 + r) * lddw;
-            for (int d = 4 * lane; d < D; d += 256) {
-                const vec4<T> xv = load4<T>(x + n * ldx + d);
-                f32x4 o = lds4f(out + d);
-#pragma unroll
-                for (int i = 0; i < 4; ++i) o[i] = fmaf(-sn, (float)xv[i], o[i]);
-                *reinterpret_cast<f32x4*>(out + d) = o;
-            }
-        }
-        __syncthreads();
-    }
+    if (dw) grad_tile<T, true, false>(a, sm, u);
+    else grad_tile<T, false, false>(a, sm, u);
 }
 
 // c[k, n] = exp2(m_t[k, n] - lse2[n]) * s_n, in place over the (2 * tiles, N) table; the entry k that holds the
@@ -497,7 +412,7 @@ __global__ __launch_bounds__(256) void lmce_dx_reduce_kernel(const float* part, 
 }
 
 struct Layout {
-    int64_t probs, cs, part, lse2, srow, glab, cn, xs, dxp, total;
+    int64_t probs, cs, part, lse2, srow, glab, cn, dxp, total;
 };
 
 int64_t align256(int64_t b) { return (b + 255) / 256 * 256; }
@@ -519,8 +434,7 @@ Layout layout(int64_t N, int64_t Vp, int D, int dx_splits) {
     l.srow = l.lse2 + align256(N * 4);
     l.glab = l.srow + align256(N * 8);
     l.cn = l.glab + align256(N * 4);
-    l.xs = l.cn + align256(N * 4);
-    l.dxp = l.xs + align256(N * D * 2);
+    l.dxp = l.cn + align256(N * 4);
     l.total = l.dxp + align256((int64_t)dx_splits * N * D * 4);
     return l;
 }
@@ -582,12 +496,6 @@ extern "C" int sisa_lmce_train(const sisa_lmce_train_args* a, void* stream) {
                                                            a->N, flag);
     rc = sisa::launch_status("sisa_lmce_train (scale)");
     if (rc) return rc;
-    if (flag && a->dw) {
-        lmce_xscale_kernel<__bf16><<<(unsigned)sisa::cdiv(a->N * (a->D / 8), 256), 256, 0, st>>>(
-            (const __bf16*)a->x, a->ldx, cn, (__bf16*)(ws + l.xs), a->N, a->D, flag);
-        rc = sisa::launch_status("sisa_lmce_train (scaled rows)");
-        if (rc) return rc;
-    }
 
     GradArgs g{};
     g.probs = ws + l.probs;
@@ -613,7 +521,7 @@ extern "C" int sisa_lmce_train(const sisa_lmce_train_args* a, void* stream) {
     g.lddw = a->lddw;
     g.accumulate = a->dw_accumulate != 0;
     g.flag = flag;
-    g.xs = ws + l.xs;
+    g.cn = cn;
     const bool reduce = S > 1 || flag;
     if (reduce) {
         g.dxo = (float*)(ws + l.dxp);
@@ -629,12 +537,6 @@ extern "C" int sisa_lmce_train(const sisa_lmce_train_args* a, void* stream) {
     else lmce_grad_kernel<_Float16><<<grid, 64 * NWG, 0, st>>>(g);
     rc = sisa::launch_status("sisa_lmce_train (gradients)");
     if (rc) return rc;
-    if (flag && a->dw) {
-        lmce_label_dw_kernel<__bf16><<<(unsigned)(a->Vp / LROWS), 256, 0, st>>>(rinfo, (const __bf16*)a->x, a->ldx, a->dw,
-                                                                              a->lddw, a->N, a->D, flag);
-        rc = sisa::launch_status("sisa_lmce_train (label rows)");
-        if (rc) return rc;
-    }
     if (a->dx == nullptr || !reduce) return SISA_OK;
     const unsigned rgrid = (unsigned)sisa::cdiv(a->N * (a->D / 4), 256);
     if (a->dtype == SISA_BF16)
