@@ -309,7 +309,7 @@ __global__ __launch_bounds__(64 * NWC) void lmce_fwd_kernel(sisa_lmce_fwd_args a
 struct CeTrainRows {
     float* lse2;                  // (N,) or nullptr (the no-gradient pass)
     float2* rinfo;                // (N,): s_n (REF with cn: s_n (1 - p_label), what G holds at the label, negated), and
-                                  // the label as the bit pattern of an int (-1 outside [0, V))
+                                  // the label as the bit pattern of an int (-1 outside [0, V) or ignored)
     const float* inv_n;           // device scalar 1 / N_valid
     float gscale;
     const float* ref;             // REF: (N,) the reference of the row's exponentials, log2 units
@@ -373,7 +373,7 @@ __global__ __launch_bounds__(CRW * CSP) void lmce_combine_kernel(sisa_lmce_fwd_a
     if (a.lse) a.lse[n] = lse;
     if (tr.lse2) {
         tr.lse2[n] = l2;
-        const int lab = (y >= 0 && y < a.V) ? (int)y : -1;
+        const int lab = (y != a.ignore_index && y >= 0 && y < a.V) ? (int)y : -1;   // its logit exists only then
         const float sn = y == a.ignore_index ? 0.f : tr.inv_n[0] * tr.gscale;
         float gl = sn;
         if (REF && tr.cn) {

@@ -126,3 +126,43 @@ def test_scalars(N):
         assert abs(float(mean) - float(want)) <= 2 * 2.0 ** -24 * abs(float(want))
     else:
         assert not bool(torch.isfinite(mean))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("fill", [0x45, 0xff, 0x7f])          # large finite numbers, NaNs, and the largest finite ones
+def test_ignored_label_inside_the_vocabulary(dtype, fill):
+    """A padding id as ignore_index: its rows have no label term at all, whatever the workspace held before."""
+    from sisa_amd.kernels import linear_ce as LC
+    x, w, lab = _case(300, 256, 1003, 11)
+    x, w = x.to(dtype), w.to(dtype)
+    lab[lab < 0] = 0
+    lab[::3] = 0
+    valid = lab != 0
+    wpad = LC.padded_weight(w, dtype)
+    inv_n = torch.reciprocal(valid.sum().float()).reshape(1)
+    ws = LC.train_workspace([300], wpad.shape[0], 256, DEV)
+    ws.fill_(fill)
+    rows, dx = torch.empty(300, device=DEV), torch.empty(300, 256, device=DEV)
+    dw = torch.empty(wpad.shape[0], 256, device=DEV)
+    LC.lmce_train_chunk(x, wpad, lab, 1003, 0, inv_n, 256.0, rows, dx, dw, False, ws)   # 256: G above fp16's subnormals
+    assert torch.equal(rows[~valid], torch.zeros_like(rows[~valid]))
+    assert torch.equal(dx[~valid], torch.zeros_like(dx[~valid]))
+    ref = _truth(x, w, torch.where(valid, lab, -100))
+    assert _rel(dx, 256 * ref[1]) <= 3 * 2 ** -8 and _rel(dw[:1003], 256 * ref[2]) <= 3 * 2 ** -8
+
+
+@pytest.mark.gpu
+def test_ignored_label_inside_the_vocabulary_over_short_chunks():
+    """The same through the public call, the last chunk shorter, so that its slots hold the previous one's exponentials.
+    Logits spread over 35 make those large; the truth takes the logits as the kernels round them."""
+    x, w, lab = _case(500, 256, 1003, 12)
+    w = (8 * w.float()).to(torch.bfloat16)
+    lab[lab < 0] = 0
+    lab[::3] = 0
+    valid = lab != 0
+    logits = (x.double() @ w.double().t()).to(torch.bfloat16).double()
+    G = torch.softmax(logits, 1).scatter_add(1, lab[:, None], -torch.ones(500, 1, dtype=torch.float64, device=DEV))
+    G = G * valid[:, None] / valid.sum()
+    got = _run(x, w, lab, ignore_index=0, chunk_tokens=192)
+    assert _rel(got[1], G @ w.double()) <= 3 * 2 ** -8 and _rel(got[2], G.t() @ x.double()) <= 3 * 2 ** -8
