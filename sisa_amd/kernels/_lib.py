@@ -242,15 +242,23 @@ def ptr(t: torch.Tensor | None):
     return None if t is None else t.data_ptr()
 
 
+def device_index(t: torch.Tensor) -> int:
+    """The index of the GPU that holds ``t``; ``ValueError`` for a tensor elsewhere (entering its device, -1, would do
+    nothing, and a kernel would read host addresses)."""
+    if not t.is_cuda:
+        raise ValueError(f"the HIP kernels take tensors on a GPU, got one on {t.device}")
+    return t.get_device()
+
+
 def stream_of(t: torch.Tensor) -> int:
     """The raw handle of the current stream on ``t``'s device."""
-    return torch._C._cuda_getCurrentRawStream(t.get_device())
+    return torch._C._cuda_getCurrentRawStream(device_index(t))
 
 
 def launch(fn, tensor: torch.Tensor, *args) -> int:
     """``fn(*args, stream)`` on ``tensor``'s device and its current stream. The device is entered only when it is not
     the current one: the context manager and a Stream object cost as much host time as the launch itself."""
-    index = tensor.get_device()
+    index = device_index(tensor)
     if index == torch._C._cuda_getDevice():
         return fn(*args, torch._C._cuda_getCurrentRawStream(index))
     with torch.cuda.device(index):

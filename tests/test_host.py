@@ -342,3 +342,16 @@ def test_wgrad_row_pieces():
     assert all((r1 - r0) * lda * 2 < OPERAND_LIMIT and (r1 - r0) % 64 == 0 for r0, r1 in pieces[:-1])
     assert (pieces[-1][1] - pieces[-1][0]) * lda * 2 < OPERAND_LIMIT
     assert row_pieces(0, 8, 8) == []
+
+
+def test_launch_refuses_cpu_tensors(monkeypatch):
+    """A tensor that is not on a GPU raises before its entry point is called: the kernels would read host addresses."""
+    from sisa_amd.kernels import _lib
+    monkeypatch.setattr(torch._C, "_cuda_getDevice", lambda: 0, raising=False)
+    monkeypatch.setattr(torch._C, "_cuda_getCurrentRawStream", lambda index: 0, raising=False)
+    reached = []
+    with pytest.raises(ValueError, match="GPU"):
+        _lib.launch(lambda *a: reached.append(a) or 0, torch.zeros(2))
+    with pytest.raises(ValueError, match="GPU"):
+        _lib.stream_of(torch.zeros(2))
+    assert not reached
