@@ -250,7 +250,7 @@ int sisa_lmce_fwd(const sisa_lmce_fwd_args* a, void* stream);
  * (src/sisa/kernels/linear_ce.py:138-217: the logits GEMM, `_lmce_row_kernel` (linear_ce.py:60-96) and the dx and
  * dW GEMMs of linear_ce.py:171-191). Deterministic: no atomics. */
 typedef struct {
-    int64_t N;                 /* rows of the chunk (0 is a no-op) */
+    int64_t N;                 /* rows of the chunk (0 is a no-op); 2 N Vp at most 0x7fffff00 */
     int64_t V;                 /* real vocabulary rows of w, >= 1 */
     int64_t Vp;                /* rows of w, a multiple of 128, >= V (rows >= V never enter a sum) */
     int32_t D;                 /* hidden size, a positive multiple of 64 */

@@ -150,7 +150,8 @@ __global__ __launch_bounds__(64 * NWC) void lmce_fwd_kernel(sisa_lmce_fwd_args a
 #pragma unroll
         for (int j = 0; j < JB; ++j) acc[i][j] = zero4();
 
-    // STORE: the exponentials go out through one buffer resource over (N, Vp) (below 2 GiB, checked by the host)
+    // STORE: the exponentials go out through one buffer resource over (N, Vp) (at most 0x7fffff00 bytes, checked by
+    // sisa_lmce_train)
     const __amdgpu_buffer_rsrc_t prs =
         make_rsrc(STORE ? (const void*)out.probs : (const void*)a.x, STORE ? N * a.Vp * (int64_t)sizeof(T) : 0);
     const int total = ntiles * nks;

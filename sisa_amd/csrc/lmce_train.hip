@@ -471,6 +471,10 @@ extern "C" int sisa_lmce_train(const sisa_lmce_train_args* a, void* stream) {
     SISA_REQUIRE(((sisa::cdiv(a->N, 256) * 256 - 1) * a->ldx + a->D) * 2 < ((int64_t)1 << 31) &&
                      ((sisa::cdiv(a->Vp, 256) * 256 - 1) * a->ldw + a->D) * 2 < ((int64_t)1 << 31),
                  "sisa_lmce_train: x or w spans 2 GiB or more");
+    // the exponentials go out by 32-bit offsets into one resource, with positions past the data at 0x7ffffff0
+    SISA_REQUIRE(a->N <= (int64_t)0x7fffff00 / (a->Vp * 2),
+                 "sisa_lmce_train: the exponentials of %lld rows of %lld span 2 GiB or more", (long long)a->N,
+                 (long long)a->Vp);
     hipStream_t st = (hipStream_t)stream;
     const int S = a->dx_splits > 0 ? a->dx_splits : default_dx_splits(a->N, a->Vp);
     const Layout l = layout(a->N, a->Vp, a->D, S);

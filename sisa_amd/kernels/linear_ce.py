@@ -45,7 +45,9 @@ __all__ = ["linear_cross_entropy", "reference_linear_cross_entropy", "lmce_rows"
 
 VOCAB_MULTIPLE = 128
 HIDDEN_MULTIPLE = 64             # the CE kernels stream the hidden size in 64-wide stages
-PROBS_BUDGET = 2 << 30           # bytes of one chunk of stored exponentials
+PROBS_LIMIT = 0x7fffff00         # bytes that a chunk's stored exponentials may take: the kernels address them by 32-bit
+                                 # offsets and drop what lies at 0x7ffffff0
+PROBS_BUDGET = 2 << 30           # bytes of one chunk of stored exponentials, within that
 SCALAR_ROWS = 1 << 17            # rows up to which one workgroup counts the valid ones and averages the loss: 16 and
                                  # 8 loads a thread deep there, still less than the launches of the general sums
 
@@ -70,15 +72,16 @@ def chunk_rows(n_rows: int, vocab_rows: int, chunk_tokens: int | None, itemsize:
                budget: int = PROBS_BUDGET) -> int:
     """Token rows per chunk of the gradient pass: ``chunk_tokens`` if given (within [1, n_rows]); otherwise the
     smallest number of equal chunks whose stored exponentials fit ``budget`` bytes, each rounded up to whole 128-row
-    GEMM tiles."""
+    GEMM tiles. Either way at most what ``PROBS_LIMIT`` holds."""
     if n_rows <= 0:
         return 1
+    most = max(1, PROBS_LIMIT // (vocab_rows * itemsize))
     if chunk_tokens:
-        return min(n_rows, max(1, int(chunk_tokens)))
-    fit = max(VOCAB_MULTIPLE, budget // (vocab_rows * itemsize))
+        return min(n_rows, most, max(1, int(chunk_tokens)))
+    fit = min(most, max(VOCAB_MULTIPLE, budget // (vocab_rows * itemsize)))
     pieces = -(-n_rows // fit)
     per = -(-n_rows // pieces)
-    return min(n_rows, -(-per // VOCAB_MULTIPLE) * VOCAB_MULTIPLE)
+    return min(n_rows, most, -(-per // VOCAB_MULTIPLE) * VOCAB_MULTIPLE)
 
 
 def lmce_rows(logits: torch.Tensor, labels: torch.Tensor, loss_rows: torch.Tensor, V: int, ignore_index: int,
@@ -247,8 +250,8 @@ def linear_cross_entropy(hidden: torch.Tensor, weight: torch.Tensor, labels: tor
 
     hidden ``(..., D)``; weight ``(V, D)`` (the tied embedding; fp32 master or 16-bit); labels ``(...)`` integer
     targets, one per hidden row, not shifted; rows equal to ``ignore_index`` add neither loss nor gradient (the loss
-    is NaN when all are ignored). ``chunk_tokens``: token rows per chunk of the gradient pass (default: chunks of at
-    most 1 GiB of logits). ``grad_scale``: promise that the backward seed is exactly this value (G is scaled in the
+    is NaN when all are ignored). ``chunk_tokens``: token rows per chunk of the gradient pass (default, and at
+    most: what 2 GiB of stored exponentials hold). ``grad_scale``: promise that the backward seed is exactly this value (G is scaled in the
     forward pass; a different seed trips a device-side assert). The compute dtype is the autocast dtype when autocast
     is on, else ``hidden.dtype``; CPU tensors and fp32 use the eager formula.
     """

@@ -355,3 +355,20 @@ def test_launch_refuses_cpu_tensors(monkeypatch):
     with pytest.raises(ValueError, match="GPU"):
         _lib.stream_of(torch.zeros(2))
     assert not reached
+
+
+def test_linear_ce_chunks_stay_addressable(lib):
+    """The stored exponentials of a chunk end below the offset that stands for "past the data", however many rows there
+    are and whatever chunk is asked for, in as many chunks as the limit allows; the entry point refuses a larger one."""
+    from sisa_amd.kernels import _lib
+    from sisa_amd.kernels import linear_ce as LC
+    for Vp in (128, 1024, 32000, 50304, 128256, 1 << 23, (1 << 23) + 128):
+        most = 0x7ffffff0 // (2 * Vp)
+        for n in [*range(1, 70000, 97), 64000, 65536, 131072, 1 << 20, (1 << 24) + 5]:
+            for tokens in (None, 50000, 1 << 30):
+                rows = LC.chunk_rows(n, Vp, tokens, 2)
+                assert 1 <= rows <= n and rows * Vp * 2 <= 0x7ffffff0, (n, Vp, tokens, rows)
+                assert tokens or -(-n // rows) <= -(-n // max(1, most)), (n, Vp, rows)
+    a = _lib.LmceTrainArgs(21376, 50277, 50304, 64, _lib.BF16, 256, 64, 256, 64, 256, -100, 256, 1.0, 256, None, 256, 64,
+                           256, 64, 0, 0, 256)
+    assert lib.sisa_lmce_train(ctypes.byref(a), None) != 0 and "21376 rows" in lib.sisa_last_error().decode()
