@@ -179,10 +179,15 @@ def _unmet(impl: str, x: torch.Tensor, cfg: SISAConfig | None) -> list[str]:
     return unmet
 
 
+def meets(impl: str, x: torch.Tensor, cfg: SISAConfig | None) -> bool:
+    """Whether HIP implementation ``impl`` can run for layer input ``x`` and config ``cfg``."""
+    return not _unmet(impl, x, cfg)
+
+
 def fused_eligible(x: torch.Tensor) -> bool:
     """Whether ``hip_fused`` can run for layer input ``x`` as far as device and dtype go (the head/state sizes are
     :func:`select_impl`'s part)."""
-    return not _unmet("hip_fused", x, None)
+    return meets("hip_fused", x, None)
 
 
 _warned: set = set()

@@ -310,15 +310,17 @@ class SISABlock(nn.Module):
         self._init_ffn_and_norms()
         self.attn.reset_parameters()
 
-    def _fused_norm_ok(self, x: Tensor) -> bool:
-        """The HIP block path applies: GPU input, the fused HIP attention selected for it, and rows the norm
-        kernels take."""
+    def _norm_rows_ok(self, x: Tensor) -> bool:
+        """GPU input with rows the norm kernels take, and the block's HIP path not switched off."""
         if not self.fuse_norm or x.device.type != "cuda" or x.dim() != 3 or x.numel() == 0:
             return False
         d, h = x.shape[-1], self.config.n_head
-        if d % 8 or d > 4096 or h > 64 or x.dtype not in (torch.float32, torch.bfloat16, torch.float16):
-            return False
-        return backends.select_impl(self.config.attn_impl, x, self.config) == "hip_fused"
+        return not (d % 8 or d > 4096 or h > 64) and x.dtype in (torch.float32, torch.bfloat16, torch.float16)
+
+    def _fused_norm_ok(self, x: Tensor) -> bool:
+        """The HIP block path applies: GPU input, the fused HIP attention selected for it, and rows the norm
+        kernels take."""
+        return self._norm_rows_ok(x) and backends.select_impl(self.config.attn_impl, x, self.config) == "hip_fused"
 
     def _forward_cached_hip(self, x: Tensor, res: Tensor | None, cache: "SISACache"):
         """Generation on HIP kernels, or None where it does not apply. A prompt (empty cache entry) takes
@@ -329,8 +331,11 @@ class SISABlock(nn.Module):
         from .generation import SISACache
         from .kernels import step
 
-        if x.device.type != "cuda" or type(cache) is not SISACache or not step.unobserved(x) \
-                or not self._fused_norm_ok(x) or not step.plain(self, SISABlock):
+        # A forced implementation that x does not meet raises in the module path, or not at all: a cached fp32 call runs
+        # the unfused kernels in place of "hip_fused", and a decode step selects nothing.
+        if type(cache) is not SISACache or not self._norm_rows_ok(x) or not step.unobserved(x) \
+                or self.config.attn_impl not in ("auto", "hip_fused") \
+                or not backends.meets("hip_fused", x, self.config) or not step.plain(self, SISABlock):
             return None
         mods = self._modules
         at, ffn, n1, n2 = mods["attn"], mods["ffn"], mods["attn_norm"], mods["ffn_norm"]

@@ -166,3 +166,14 @@ def test_step_struct_layout_matches_c(tmp_path):
                    check=True)
     got = subprocess.run([str(exe)], capture_output=True, text=True, check=True).stdout.split()
     assert [int(v) for v in got] == expect
+
+
+@pytest.mark.gpu
+def test_fp32_generation_with_the_fused_implementation_requested():
+    """Cached fp32 calls under attn_impl="hip_fused" run the unfused kernels, as a call without a cache cannot."""
+    ids = token_ids(2, 9, seed=4).to(DEV)
+    model = tiny_model(seed=4, theta_scale=0.25, attn_impl="hip_fused").to(DEV).eval()
+    got, _ = _decode(model, ids, 6)
+    model.set_attn_impl("hip")
+    want, _ = _decode(model, ids, 6)
+    assert torch.equal(got, want)
