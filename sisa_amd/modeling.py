@@ -481,7 +481,8 @@ class SISAModel(nn.Module):
             if DEFER_RESIDUAL and not recompute and cache is None and block._fused_norm_ok(x):
                 x, pending = block._forward_hip(x, pending, defer=True)
                 continue
-            done = None if cache is None else block._forward_cached_hip(x, pending, cache)
+            # other modules in place of a block are only called
+            done = block._forward_cached_hip(x, pending, cache) if cache is not None and type(block) is SISABlock else None
             if done is not None:
                 x, pending = done
                 continue

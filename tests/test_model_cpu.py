@@ -223,3 +223,20 @@ def test_loss_conventions():
     with pytest.raises(ValueError, match="GPU"):
         model(ids, labels=labels, fused_ce=True)
     assert math.isfinite(out.loss.item())
+
+
+def test_generation_through_a_wrapped_block():
+    """``layers`` may hold any module that takes ``(x, cache=...)``, as a wrapper around a block does."""
+    class Wrapped(torch.nn.Module):
+        def __init__(self, block):
+            super().__init__()
+            self.block = block
+
+        def forward(self, x, cache=None):
+            return self.block(x, cache=cache)
+
+    model = tiny_model(seed=2).eval()
+    ids = token_ids(2, 5, seed=2)
+    want = model.generate(ids, 4)
+    model.layers[1] = Wrapped(model.layers[1])
+    assert torch.equal(model.generate(ids, 4), want)
