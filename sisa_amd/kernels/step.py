@@ -117,6 +117,15 @@ def layer_step(x: Tensor, res: Tensor | None, weights: list[int], d_ff: int, lam
     return h, ffn, phi_out
 
 
+def _fill(cache, layer_idx: int, name: str, args, x: Tensor) -> None:
+    """The call that fills a layer's new cache entry; if it fails there is no entry again, not one of no positions."""
+    try:
+        _lib.call(name, args, x)
+    except Exception:
+        cache._slabs.pop(layer_idx, None)
+        raise
+
+
 def layer_prefill(x: Tensor, res: Tensor | None, weights: list[int], d_ff: int, lambda_raw: Tensor, w_down: Tensor,
                   eps: tuple[float, float], cache, layer_idx: int, checked: bool) -> tuple[Tensor, Tensor]:
     """A prompt ``x`` ``(B, L, D)`` (contiguous; plus ``res``, added first) through a layer whose cache entry is empty,
@@ -140,11 +149,7 @@ def layer_prefill(x: Tensor, res: Tensor | None, weights: list[int], d_ff: int, 
                             *weights, lambda_raw.data_ptr(),
                             *(_lib.view(buf[n]) for n in ("k", "v", "b", "g", "fgate")), phi.data_ptr(), h.data_ptr(),
                             act.data_ptr(), _lib.ptr(f), ld, _lib.ptr(ok), ws.data_ptr())
-    try:
-        _lib.call("sisa_prefill", args, x)
-    except RuntimeError:
-        cache._slabs.pop(layer_idx, None)          # still an empty entry
-        raise
+    _fill(cache, layer_idx, "sisa_prefill", args, x)
     if ok is not None:
         torch._assert_async(ok, "sisa_attention_hip: the cumulative log-decay g increases along the sequence")
     slab.filled = L
@@ -164,7 +169,7 @@ def prefill(proj: Tensor, z: Tensor, lam: Tensor, n_head: int, cache, layer_idx:
     phi = torch.empty((B, n_head, HIP_D_STATE // 2), device=proj.device, dtype=torch.float32)
     slab = cache.room(layer_idx, L, dict(k=k, v=v, b=b, g=pp.g, fgate=pp.f), phi)
     buf = slab.buffers
-    _lib.call("sisa_cache_fill", _lib.CacheFillArgs(
+    _fill(cache, layer_idx, "sisa_cache_fill", _lib.CacheFillArgs(
         B, n_head, L, _lib.dtype_code(proj.dtype), proj.data_ptr(), proj.stride(0), proj.stride(1), lay["K"], lay["V"],
         pp.br.data_ptr(), pp.g.data_ptr(), pp.f.data_ptr(), pp.totals.data_ptr(),
         *(_lib.view(buf[n]) for n in ("k", "v", "b", "g", "fgate")), phi.data_ptr()), proj)

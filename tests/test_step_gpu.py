@@ -177,3 +177,25 @@ def test_fp32_generation_with_the_fused_implementation_requested():
     model.set_attn_impl("hip")
     want, _ = _decode(model, ids, 6)
     assert torch.equal(got, want)
+
+
+def test_failed_cache_fill_leaves_no_entry(monkeypatch):
+    """A prefill on the fused route whose last launch fails leaves the layer's entry empty, to be filled again."""
+    from types import SimpleNamespace
+
+    from sisa_amd import SISACache
+    from sisa_amd.kernels import _lib, step
+    B, L, H = 1, 3, 2
+    proj = torch.zeros(B, L, step.P.fused_layout(H)["NPAD"], dtype=torch.bfloat16)
+    rows, gates = torch.zeros(B, L, H, 32, dtype=torch.bfloat16), torch.zeros(B, H, L)
+    prepped = step.P.Prepped(rows, rows, gates, gates, gates, gates, torch.zeros(B * H, 1, 18))
+    monkeypatch.setattr(step.P, "prep_forward", lambda *a: prepped)
+    monkeypatch.setattr(step.A, "attn_forward", lambda *a: SimpleNamespace(o=torch.zeros(B, H, L, 64)))
+
+    def fail(*a):
+        raise RuntimeError("no launch")
+    monkeypatch.setattr(_lib, "call", fail)
+    cache = SISACache()
+    with pytest.raises(RuntimeError, match="no launch"):
+        step.prefill(proj, torch.zeros(B, L, H), torch.ones(H), H, cache, 0)
+    assert len(cache) == 0 and cache.get(0) is None
