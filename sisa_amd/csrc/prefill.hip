@@ -398,7 +398,9 @@ extern "C" int sisa_prefill(const sisa_prefill_args* a, void* stream) {
                  "sisa_prefill: act_ld %lld must be FF = %d rounded up to a multiple of 64", (long long)a->act_ld, a->FF);
     SISA_REQUIRE(a->ffn == nullptr || (sisa::aligned16(a->ffn) && a->w_down && sisa::aligned16(a->w_down) && a->FF % 8 == 0),
                  "sisa_prefill: the down projection needs FF %% 8 == 0 and aligned w_down, ffn");
-    SISA_REQUIRE((int64_t)a->FF * a->H * DH * 2 < ((int64_t)1 << 31), "sisa_prefill: a weight spans 2 GiB or more");
+    SISA_REQUIRE((int64_t)a->FF * a->H * DH * 2 < ((int64_t)1 << 31) &&
+                     (int64_t)a->B * a->L * a->act_ld * 2 < ((int64_t)1 << 31),
+                 "sisa_prefill: a weight or the activation spans 2 GiB or more");
     SISA_REQUIRE(a->b_alpha && a->b_forget && a->lambda_raw && a->phi && a->workspace &&
                      ((uintptr_t)a->workspace & 255) == 0,
                  "sisa_prefill: null pointer, or workspace not 256-byte aligned");

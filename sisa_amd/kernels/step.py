@@ -19,13 +19,19 @@ from . import _lib
 from . import attention as A
 from . import fused_prep as P
 
-__all__ = ["unobserved", "plain", "plain_linears", "rows_ok", "whole", "step_weights", "layer_step", "layer_prefill", "prefill", "MAX_ROWS", "MAX_WIDTH", "PREFILL_ROWS"]
+__all__ = ["unobserved", "plain", "plain_linears", "rows_ok", "whole", "prefill_fits", "step_weights",
+           "layer_step", "layer_prefill", "prefill", "MAX_ROWS", "MAX_WIDTH", "PREFILL_ROWS"]
 
 MAX_ROWS, MAX_WIDTH = 64, 1024          # SISA_STEP_MAX_ROWS, SISA_STEP_MAX_D
 #: Prompts of at most this many tokens (all rows together) take ``sisa_prefill``: as far as it was measured ahead of the
 #: launch-by-launch route, whose library GEMMs gain on it with size (whole model, ms: 800 tokens at width 768 2.0 against
 #: 5.1, 8,192 tokens as 8 x 1,024 4.6 against 5.5; width 1,024 3.6 against 10.3 and 10.3 against 12.9).
 PREFILL_ROWS = 8192
+
+
+def prefill_fits(rows: int, width: int, d_ff: int) -> bool:
+    """``sisa_prefill`` reads activations and weights by 32-bit offsets: each must end below 2 GiB."""
+    return max(rows, width) * (-(-d_ff // 64) * 64) * 2 < 1 << 31
 
 
 def unobserved(x: Tensor) -> bool:

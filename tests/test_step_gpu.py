@@ -199,3 +199,17 @@ def test_failed_cache_fill_leaves_no_entry(monkeypatch):
     with pytest.raises(RuntimeError, match="no launch"):
         step.prefill(proj, torch.zeros(B, L, H), torch.ones(H), H, cache, 0)
     assert len(cache) == 0 and cache.get(0) is None
+
+
+def test_prefill_refuses_what_its_offsets_cannot_reach():
+    """The products read their operands by 32-bit offsets: activations or weights of 2 GiB keep the fused route, and the
+    entry point refuses them."""
+    from sisa_amd.kernels import _lib, step
+    assert step.prefill_fits(8192, 4096, 11008) and step.prefill_fits(8192, 64, 130_000)
+    assert not step.prefill_fits(8192, 64, 131_072) and not step.prefill_fits(1, 4096, 262_144)
+    lib = _lib.load()
+    for L, H, ff in ((8192, 1, 131_072), (1, 64, 262_144)):
+        pointers = {n: 256 for n, t in _lib.PrefillArgs._fields_ if t is ctypes.c_void_p and n != "res"}
+        args = _lib.PrefillArgs(B=1, L=L, H=H, FF=ff, dtype=_lib.BF16, act_ld=ff, **pointers)
+        assert lib.sisa_prefill(ctypes.byref(args), None) != 0
+        assert "2 GiB" in lib.sisa_last_error().decode()
