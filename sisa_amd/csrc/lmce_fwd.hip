@@ -326,6 +326,12 @@ struct CeTrainRows {
 constexpr int CRW = 16, CSP = 16;
 constexpr float Z_MAX = 0x1p60f, Z_MIN = 0x1p-20f;   // sums whose exponentials and products stay far inside fp32 / bf16
 
+// An ignored row adds nothing: unless its log-sum-exp is asked for it takes a reference above any logit, so that its
+// exponentials are 0 and products with them finite, and has no say in the flag. (No column's logit represents such a row, and
+// one prompt token that the loss masks would send a whole chunk the second way.)
+constexpr float REF_IGNORED = 0x1p126f;
+SISA_DEV bool left_out(const sisa_lmce_fwd_args& a, int64_t y) { return y == a.ignore_index && !a.lse; }
+
 template <bool REF>
 __global__ __launch_bounds__(CRW * CSP) void lmce_combine_kernel(sisa_lmce_fwd_args a, int S, CeTrainRows tr) {
     __shared__ float pm[CSP][CRW], ps[CSP][CRW];
@@ -355,7 +361,7 @@ __global__ __launch_bounds__(CRW * CSP) void lmce_combine_kernel(sisa_lmce_fwd_a
         ss = 0.f;
 #pragma unroll
         for (int p = 0; p < CSP; ++p) ss += ps[p][lr];
-        if (!(ss >= Z_MIN && ss <= Z_MAX)) *tr.flag = 1;   // NaN too; every writer stores the same value
+        if (!(ss >= Z_MIN && ss <= Z_MAX) && !left_out(a, a.labels[n])) *tr.flag = 1;   // NaN too; all store the same value
     } else {
 #pragma unroll
         for (int p = 1; p < CSP; ++p) mm = fmaxf(mm, pm[p][lr]);
@@ -378,7 +384,7 @@ __global__ __launch_bounds__(CRW * CSP) void lmce_combine_kernel(sisa_lmce_fwd_a
         const float sn = y == a.ignore_index ? 0.f : tr.inv_n[0] * tr.gscale;
         float gl = sn;
         if (REF && tr.cn) {
-            tr.cn[n] = sn / ss;
+            tr.cn[n] = left_out(a, y) ? 0.f : sn / ss;
             if (lab >= 0) {   // p - 1 is formed here in fp32: taken apart, the two roundings of p would outweigh it near p = 1
                 gl = sn * (1.f - fast_exp2(fmaf(a.workspace[2 * (int64_t)S * N + n], LOG2E, -mm)) / ss);
                 tr.probs[n * a.Vp + lab] = (__bf16)0.f;
@@ -389,8 +395,8 @@ __global__ __launch_bounds__(CRW * CSP) void lmce_combine_kernel(sisa_lmce_fwd_a
 }
 
 // The reference of a row's exponentials: the logit of its label (of column 0 without a valid one), in log2 units. Any
-// column's logit bounds the row's sum below by 1; the label's is near the largest wherever the loss is small. One wave
-// per row; also clears the flag.
+// column's logit bounds the row's sum below by 1; the label's is near the largest wherever the loss is small. Rows left
+// out: REF_IGNORED. One wave per row; also clears the flag.
 template <class T>
 __global__ __launch_bounds__(256) void lmce_ref_kernel(sisa_lmce_fwd_args a, float* ref, int* flag) {
     const int64_t n = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
@@ -398,6 +404,10 @@ __global__ __launch_bounds__(256) void lmce_ref_kernel(sisa_lmce_fwd_args a, flo
     if (blockIdx.x == 0 && threadIdx.x == 0) *flag = 0;
     if (n >= a.N) return;
     const int64_t y = a.labels[n];
+    if (left_out(a, y)) {
+        if (lane == 0) ref[n] = REF_IGNORED;
+        return;
+    }
     const T* x = (const T*)a.x + n * a.ldx;
     const T* w = (const T*)a.w + (y >= 0 && y < a.V ? y : 0) * a.ldw;
     float d = 0.f;
@@ -411,7 +421,7 @@ __global__ __launch_bounds__(256) void lmce_ref_kernel(sisa_lmce_fwd_args a, flo
     if (lane == 0) ref[n] = d * LOG2E;
 }
 
-// Logits GEMM and combine. bf16: against the label logits (REF), then, gated on the flag of a row whose sum left
+// Logits GEMM and combine. bf16: against the label logits (REF), then, gated on the flag of a row that counts whose sum left
 // [Z_MIN, Z_MAX] (its label's logit more than 41 below the row's largest, or non-finite values), again against the
 // tile-half maxima; the gated launches of an unflagged call end at once. That spares each logit the running maximum,
 // and lets the gradient products of the training pass take the stored exponentials as they are. fp16 has too little

@@ -1,6 +1,6 @@
 """The linear cross-entropy's two ways of keeping a row's exponentials: against one reference per row (its label's
 logit; plain gradient products) and, where a row's sum leaves that reference's range, against the maxima over half
-vocabulary tiles. A chunk takes the second way as soon as one of its rows needs it."""
+vocabulary tiles. A chunk takes the second way as soon as one of its rows that count needs it."""
 import pytest
 import torch
 
@@ -17,10 +17,10 @@ def _case(N, D, V, seed, one_label=False):
 
 
 def _poison(x, w, lab):
-    """One more row, ignored, that no single reference of column 0 fits: its logits spread over hundreds."""
+    """One more row that no single reference fits: its logits spread over hundreds, and its label has the lowest."""
     row = (w[1] - w[0]).float()
     row = (row * (300.0 / row.norm() ** 2)).to(torch.bfloat16)
-    return torch.cat([x, row[None]]), w, torch.cat([lab, lab.new_tensor([-100])])
+    return torch.cat([x, row[None]]), w, torch.cat([lab, lab.new_tensor([0])])
 
 
 def _run(x, w, lab, **kw):
@@ -50,23 +50,17 @@ def test_row_references_match_tile_maxima(N, D, V, one_label):
     x, w, lab = _case(N, D, V, N + D, one_label)
     if N == 1:
         lab[0] = 3
-    ref = _truth(x, w, lab)
-    fast = _run(x, w, lab)
-    loss, dx, dw = _run(*_poison(x, w, lab))
-    slow = (loss, dx[:N], dw)
-    assert torch.equal(dx[N], torch.zeros_like(dx[N]))
-    assert N == 1 or not torch.equal(fast[1], slow[1])      # two computations, not one
-    for got in (fast, slow):
+    for case in ((x, w, lab), _poison(x, w, lab)):
+        ref, got = _truth(*case), _run(*case)
         # logits rounded to 8 bits shift the loss by the mean of their errors; gradients: three 8-bit roundings
         assert abs(float(got[0] - ref[0])) <= 2 ** -8 * (1 + abs(float(ref[0])))
         assert _rel(got[1], ref[1]) <= 3 * 2 ** -8 and _rel(got[2], ref[2]) <= 3 * 2 ** -8
-    assert abs(float(fast[0] - slow[0])) <= 1e-5 * abs(float(slow[0]))
-    again = _run(x, w, lab)
-    assert all(torch.equal(a, b) for a, b in zip(fast, again))
-    with torch.no_grad():
-        from sisa_amd.kernels.linear_ce import linear_cross_entropy
-        assert torch.equal(linear_cross_entropy(x, w.float(), lab), fast[0])
-        assert torch.equal(linear_cross_entropy(*_poison(x, w, lab)[:2], _poison(x, w, lab)[2]), slow[0])
+        assert _rel(got[1][:N], ref[1][:N]) <= 3 * 2 ** -8      # the poison row's gradient outweighs the others'
+        again = _run(*case)
+        assert all(torch.equal(a, b) for a, b in zip(got, again))
+        with torch.no_grad():
+            from sisa_amd.kernels.linear_ce import linear_cross_entropy
+            assert torch.equal(linear_cross_entropy(case[0], case[1].float(), case[2]), got[0])
 
 
 @pytest.mark.gpu
@@ -81,11 +75,14 @@ def test_confident_rows(top):
     logits = (x.double() @ w.double().t()).to(torch.bfloat16).double()
     G = torch.softmax(logits, 1)
     rest = G.scatter(1, lab[:, None], 0.0)
-    G = rest.scatter(1, lab[:, None], -rest.sum(1, keepdim=True)) / len(lab)
-    for args in ((x, w, lab), _poison(x, w, lab)):
-        _, dx, dw = _run(*args)
-        assert _rel(dx[:300], G @ w.double()) <= 3 * 2 ** -8
-        assert _rel(dw, G.t() @ x.double()) <= 3 * 2 ** -8
+    G = rest.scatter(1, lab[:, None], -rest.sum(1, keepdim=True))
+    _, dx, dw = _run(x, w, lab)
+    assert _rel(dx, G / 300 @ w.double()) <= 3 * 2 ** -8
+    assert _rel(dw, G.t() / 300 @ x.double()) <= 3 * 2 ** -8
+    px, _, plab = _poison(x, w, lab)
+    _, dx, dw = _run(px, w, plab)
+    assert _rel(dx[:300], G / 301 @ w.double()) <= 3 * 2 ** -8
+    assert _rel(dw[2:], G.t()[2:] / 301 @ x.double()) <= 3 * 2 ** -8     # the poison row reaches rows 0 and 1 only
 
 
 @pytest.mark.gpu
@@ -95,14 +92,13 @@ def test_chunks_of_both_kinds_and_a_hopeless_label():
     x, w, lab = _poison(*_case(500, 256, 2000, 9))
     order = torch.randperm(501, generator=torch.Generator().manual_seed(1)).to(DEV)
     x, lab = x[order], lab[order]
+    rest = order != 500
     ref = _truth(x, w, lab)
-    got = _run(x, w, lab, chunk_tokens=128)
-    assert _rel(got[1], ref[1]) <= 3 * 2 ** -8 and _rel(got[2], ref[2]) <= 3 * 2 ** -8
-    hard = lab.clone()
-    hard[int((order == 500).nonzero())] = 0                 # the poison row's lowest logit as its label
-    ref, got = _truth(x, w, hard), _run(x, w, hard)
-    assert float(ref[0]) > 0.25 and abs(float(got[0] - ref[0])) <= 2 ** -8 * float(ref[0])
-    assert _rel(got[1], ref[1]) <= 3 * 2 ** -8 and _rel(got[2], ref[2]) <= 3 * 2 ** -8
+    for kw in (dict(chunk_tokens=128), {}):
+        got = _run(x, w, lab, **kw)
+        assert float(ref[0]) > 0.25 and abs(float(got[0] - ref[0])) <= 2 ** -8 * float(ref[0])
+        assert _rel(got[1], ref[1]) <= 3 * 2 ** -8 and _rel(got[2], ref[2]) <= 3 * 2 ** -8
+        assert _rel(got[1][rest], ref[1][rest]) <= 3 * 2 ** -8
     bad = lab.clone()
     bad[7] = 2000                                           # outside the vocabulary: NaN loss, as without it
     assert not bool(torch.isfinite(_run(x, w, bad)[0]))
@@ -166,3 +162,27 @@ def test_ignored_label_inside_the_vocabulary_over_short_chunks():
     G = G * valid[:, None] / valid.sum()
     got = _run(x, w, lab, ignore_index=0, chunk_tokens=192)
     assert _rel(got[1], G @ w.double()) <= 3 * 2 ** -8 and _rel(got[2], G.t() @ x.double()) <= 3 * 2 ** -8
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("N", [300, 1500])
+def test_ignored_rows_are_never_outliers(N):
+    """Masked rows whose logits no column's logit represents leave the other rows on the fast way: the same bits as with
+    ordinary masked rows, in both passes, and their own gradient is zero. Asked for, their log-sum-exp is exact."""
+    from sisa_amd.kernels import linear_ce as LC
+    x, w, lab = _case(N, 256, 1003, N)
+    far = (w[1] - w[0]).float()
+    far = (far * (300.0 / far.norm() ** 2)).to(torch.bfloat16)
+    masked = torch.arange(N, device=DEV) % 7 == 0
+    lab[masked] = -100
+    for sign in (1, -1):                                    # column 0 far below the row's largest logit, and above all
+        xo = torch.where(masked[:, None], sign * far, x)
+        (loss, dx, dw), (lo, dxo, dwo) = _run(x, w, lab), _run(xo, w, lab)
+        assert torch.equal(loss, lo) and torch.equal(dx, dxo) and torch.equal(dw, dwo)
+        assert not dx[masked].any()
+        with torch.no_grad():
+            assert torch.equal(LC.linear_cross_entropy(xo, w, lab), loss)
+        lse = torch.empty(N, device=DEV)
+        LC.lmce_fused_loss_rows(xo, LC.padded_weight(w, torch.bfloat16), lab, 1003, -100, lse)
+        logits = (xo.double() @ w.double().t()).to(torch.bfloat16).double()
+        assert float((lse.double() - torch.logsumexp(logits, 1)).abs().max()) <= 1e-4
