@@ -241,11 +241,11 @@ int sisa_lmce_fwd(const sisa_lmce_fwd_args* a, void* stream);
 /* Training pass of the linear cross-entropy over one chunk of rows, on MFMA kernels only: the loss rows and, as
  * requested, dL/dx and dL/dW_pad in fp32 for G = (softmax - onehot) * (*inv_n) * gscale, i.e. for a backward seed of
  * gscale. The logits GEMM is sisa_lmce_fwd's kernel, which here also stores every exponential (compute dtype, in the
- * workspace): bf16 relative to the row's label logit, or, for a chunk with a row which that does not suit, and in fp16,
- * to its maximum over a 128-column half of a 256-column vocabulary tile; the loss rows are bitwise those of
- * sisa_lmce_fwd. One launch then runs the dW tiles (dW = G^T x, all rows of the chunk) and the dx tiles (dx = G W_pad,
- * split over the vocabulary, the splits added in a fixed order), from G formed while staging it, or dx from the stored
- * exponentials themselves (the normaliser applied to the sum, the label term added in fp32). No logits
+ * workspace): bf16 relative to the row's label logit, or, in blocks of 256 rows with a row which that does not suit, to
+ * its log-sum-exp; fp16 relative to its maximum over a 128-column half of a 256-column vocabulary tile. The loss rows are
+ * bitwise those of sisa_lmce_fwd. One launch then runs the dW tiles (dW = G^T x, all rows of the chunk) and the dx tiles
+ * (dx = G W_pad, split over the vocabulary, the splits added in a fixed order), from G formed while staging it, or bf16's dx
+ * from the stored exponentials themselves (the normaliser applied to the sum, the label term added in fp32). No logits
  * and no G are ever written. Replaces the chunk loop of `_LinearCrossEntropyFn.forward`
  * (src/sisa/kernels/linear_ce.py:138-217: the logits GEMM, `_lmce_row_kernel` (linear_ce.py:60-96) and the dx and
  * dW GEMMs of linear_ce.py:171-191). Deterministic: no atomics. */

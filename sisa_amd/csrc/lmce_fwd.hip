@@ -17,9 +17,9 @@
 // when the tile holds a row's label it keeps that logit. At the end the lane groups and the two waves sharing rows
 // combine their partials; a second launch combines the S splits of each row in a fixed order.
 //
-// bf16 takes the exponentials against one reference per row, its label's logit (REF; lmce_ref_kernel), and falls back,
-// for a call with a row that reference does not suit, to the maxima described above; see launch_logits. At 4,094 rows of
-// 1,024 (V 50,277) the launch takes 427 us with REF, 458 without.
+// bf16 takes the exponentials against one reference per row, its label's logit (REF; lmce_ref_kernel), and goes over the
+// 256-row blocks with a row that reference does not suit again, against the maxima described above; see launch_logits. At
+// 4,094 rows of 1,024 (V 50,277) the launch takes 427 us with REF, 458 without.
 //
 // The training pass (sisa_lmce_train, lmce_train.hip) runs the same kernel with STORE: each exponential is also stored in
 // the compute dtype into a (N, Vp) buffer, and without REF the maxima m_t it is relative to into a (2 * tiles, N) table.
@@ -53,34 +53,66 @@ struct __attribute__((aligned(16))) CeLds {
 // What a launch stores and against what it takes its exponentials.
 //   STORE: the exponentials go to probs. REF: they are relative to one given reference per row (ref, log2 units)
 //   instead of the row's maxima over the tile halves, which go to mtab.
-//   gate: run only if *gate is nonzero (null: always).
+//   marks: only the row blocks that it marks (null: all).
 template <class T>
 struct CeStore {
     T* probs;                     // (N, Vp) in the compute dtype, row stride Vp; columns >= V hold 0
     float* mtab;                  // (2 * tiles, N): m_t of (tile t, half h) at row (2 t + h) * N + n, log2 units
     const float* ref;             // (N,)
-    const int* gate;
+    float* zlab;                  // (N,) the label's logit, natural units; left alone without a label that counts
+    const int* marks;
 };
 
-// The vocabulary splits of one problem: S splits of `per` consecutive tiles (the last ones may be shorter or empty).
+// The vocabulary splits of `nrb` row blocks: S splits of `per` consecutive tiles (the last ones may be shorter or empty).
+constexpr int CE_WGS = 512;                      // about as many workgroups: two rounds of one per CU
 struct Split {
-    int64_t tiles, S, per;
+    int S, per;
 };
-inline Split ce_split(int64_t N, int64_t Vp) {
-    const int64_t nrb = sisa::cdiv(N, TR), tiles = sisa::cdiv(Vp, TV);
-    int64_t S = sisa::cdiv(512, nrb);            // about 512 workgroups: two rounds of one per CU
-    S = S < 1 ? 1 : (S > tiles ? tiles : S);
-    return {tiles, S, sisa::cdiv(tiles, S)};
+__host__ __device__ inline Split ce_split(int nrb, int tiles) {
+    int S = (CE_WGS + nrb - 1) / nrb;
+    S = S > tiles ? tiles : S;
+    return {S, (tiles + S - 1) / S};
+}
+// The most (row block, split) items that some of `nrb` row blocks make.
+inline int64_t ce_items(int64_t nrb, int64_t tiles) {
+    return tiles * nrb < CE_WGS - 1 + nrb ? tiles * nrb : CE_WGS - 1 + nrb;
+}
+
+// Marks over the row blocks: word 0 tells whether there are any, word 1 + rb marks block rb. The slot of a marked block is
+// the number of marked ones before it; the marked blocks are split as a problem of that many. (Whole waves call these.)
+SISA_DEV int marks_before(const int* marks, int rb, int lane) {
+    int c = 0;
+    for (int b = 0; b < rb; b += 64) c += __popcll(__builtin_amdgcn_ballot_w64(b + lane < rb && marks[1 + b + lane] != 0));
+    return c;
+}
+SISA_DEV int marked_block(const int* marks, int nrb, int slot, int lane) {
+    for (int b = 0; b < nrb; b += 64) {
+        uint64_t m = __builtin_amdgcn_ballot_w64(b + lane < nrb && marks[1 + b + lane] != 0);
+        const int c = __popcll(m);
+        if (slot < c) {
+            for (; slot > 0; --slot) m &= m - 1;
+            return b + __builtin_ctzll(m);
+        }
+        slot -= c;
+    }
+    return 0;                                    // not reached for a slot below their number
 }
 
 template <class T, bool STORE, bool REF>
 __global__ __launch_bounds__(64 * NWC) void lmce_fwd_kernel(sisa_lmce_fwd_args a, int S, int per, CeStore<T> out) {
     __shared__ CeLds<T> sm;
-    if (out.gate && *out.gate == 0) return;
+    if (out.marks && out.marks[0] == 0) return;
     const int tid = threadIdx.x, lane = tid & 63, grp = lane >> 4, lc = lane & 15;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int64_t N = a.N, V = a.V;
-    const int nrb = (int)((N + TR - 1) / TR);
+    const int blocks = (int)((N + TR - 1) / TR), tiles = (int)((a.Vp + TV - 1) / TV);
+    int nrb = blocks;
+    if (out.marks) {
+        nrb = marks_before(out.marks, blocks, lane);
+        const Split sp = ce_split(nrb, tiles);
+        S = sp.S;
+        per = sp.per;
+    }
     const int item = xcd_item(blockIdx.x, nrb * S);
     if (item < 0) return;
     // Items (row block, split) in groups of RGRP row blocks, row blocks fastest: the 32 workgroups an XCD runs at a time
@@ -88,8 +120,8 @@ __global__ __launch_bounds__(64 * NWC) void lmce_fwd_kernel(sisa_lmce_fwd_args a
     // splits reads 33.
     const int grp_items = RGRP * S, g0 = item / grp_items * RGRP, in_grp = item % grp_items;
     const int rg = nrb - g0 < RGRP ? nrb - g0 : RGRP;
-    const int split = in_grp / rg, rb = g0 + in_grp % rg;
-    const int tiles = (int)((a.Vp + TV - 1) / TV);
+    const int split = in_grp / rg, slot = g0 + in_grp % rg;
+    const int rb = out.marks ? marked_block(out.marks, blocks, slot, lane) : slot;
     const int t_begin = split * per;
     const int t_end = t_begin + per < tiles ? t_begin + per : tiles;
     const int ntiles = t_end > t_begin ? t_end - t_begin : 0;
@@ -273,12 +305,14 @@ __global__ __launch_bounds__(64 * NWC) void lmce_fwd_kernel(sisa_lmce_fwd_args a
     }
 
     // combine the four lane groups of each row, then the two waves sharing the rows (w and w ^ 1)
+    const int64_t np = (int64_t)nrb * TR;
+    float* part = a.workspace + (int64_t)slot * TR;
     float rm[JB], rsum[JB];
 #pragma unroll
     for (int j = 0; j < JB; ++j) {
         rm[j] = REF ? m[j] : group_max(m[j]);
         rsum[j] = group_sum(REF ? s[j] : s[j] * fast_exp2(m[j] - rm[j]));
-        if (got[j]) a.workspace[2 * (int64_t)S * N + row0 + wn + 16 * j + lc] = zlab[j];
+        if (got[j]) out.zlab[row0 + wn + 16 * j + lc] = zlab[j];
     }
     if ((w & 1) && grp == 0) {
 #pragma unroll
@@ -291,61 +325,79 @@ __global__ __launch_bounds__(64 * NWC) void lmce_fwd_kernel(sisa_lmce_fwd_args a
     if ((w & 1) == 0 && grp == 0) {
 #pragma unroll
         for (int j = 0; j < JB; ++j) {
-            const int64_t n = row0 + wn + 16 * j + lc;
-            if (n >= N) continue;
-            const float m2 = sm.red_m[wn + 16 * j + lc], s2 = sm.red_s[wn + 16 * j + lc];
+            const int r = wn + 16 * j + lc;
+            if (row0 + r >= N) continue;
+            const float m2 = sm.red_m[r], s2 = sm.red_s[r];
             if constexpr (REF) {
-                a.workspace[(int64_t)(S + split) * N + n] = rsum[j] + s2;
+                part[(S + split) * np + r] = rsum[j] + s2;
                 continue;
             }
             const float mm = fmaxf(rm[j], m2);
-            a.workspace[(int64_t)split * N + n] = mm;
-            a.workspace[(int64_t)(S + split) * N + n] = rsum[j] * fast_exp2(rm[j] - mm) + s2 * fast_exp2(m2 - mm);
+            part[split * np + r] = mm;
+            part[(S + split) * np + r] = rsum[j] * fast_exp2(rm[j] - mm) + s2 * fast_exp2(m2 - mm);
         }
     }
 }
 
-// Per row: the S split partials combined in split order; lse (natural log) and the loss row. The training pass also
-// keeps lse in log2 units and the row's gradient scale (0 for an ignored row, else inv_n * gscale).
+// Per row: the S split partials combined in split order; lse (natural log) and the loss row, and what the training pass
+// keeps of them. The partials of a row lie at its block's slot (256 rows each) plus its place in the block.
+//   LABEL: of exponentials against the rows' references, all rows; marks the row blocks that must be gone over again.
+//   TOP: of exponentials against maxima: fp16's only pass, or bf16's marked row blocks.
+//   AGAIN: of exponentials stored again against the log-sum-exp, bf16's marked row blocks; the loss stays.
+enum CombineMode { LABEL, TOP, AGAIN };
 struct CeTrainRows {
-    float* lse2;                  // (N,) or nullptr (the no-gradient pass)
-    float2* rinfo;                // (N,): s_n (REF with cn: s_n (1 - p_label), what G holds at the label, negated), and
-                                  // the label as the bit pattern of an int (-1 outside [0, V) or ignored)
+    float* lse2;                  // fp16: (N,) lse in log2 units, or nullptr (the no-gradient pass)
+    float2* rinfo;                // (N,): s_n (bf16: s_n (1 - p_label), what G holds at the label, negated), and the
+                                  // label as the bit pattern of an int (-1 outside [0, V) or ignored)
     const float* inv_n;           // device scalar 1 / N_valid
     float gscale;
-    const float* ref;             // REF: (N,) the reference of the row's exponentials, log2 units
-    float* cn;                    // REF: (N,) s_n / Z_n, or nullptr
-    __bf16* probs;                // REF with cn: the stored exponentials (N, Vp); the label's is zeroed here
-    int* flag;                    // REF: set when a row's sum is not one the reference was good for
-    const int* gate;              // run only if *gate is nonzero (null: always)
+    float* ref;                   // bf16: (N,) the reference of the row's exponentials, log2 units
+    float* cn;                    // bf16: (N,) s_n / Z_n, or nullptr (the no-gradient pass)
+    __bf16* probs;                // bf16 with cn: the stored exponentials (N, Vp); the label's is zeroed here
+    int* marks;                   // LABEL: marks a block with a row that its reference did not suit; else: the blocks to run
+                                  // on (null: all)
 };
 
 // 16 rows per workgroup, 16 threads per row: each folds every sixteenth split, and the row's first thread the sixteen
 // partial results in order. (One thread per row walks S splits in dependent loads: with the 128 splits of 1,023 rows
 // that took 66 us.)
 constexpr int CRW = 16, CSP = 16;
-constexpr float Z_MAX = 0x1p60f, Z_MIN = 0x1p-20f;   // sums whose exponentials and products stay far inside fp32 / bf16
+// Sums of exponentials that a reference is good for: an actual logit's term is 1, and products of up to 2^90 with weights
+// stay far inside fp32, as s_n / 2^90 does.
+constexpr float Z_MIN = 0x1p-20f, Z_MAX = 0x1p90f;
 
 // An ignored row adds nothing: unless its log-sum-exp is asked for it takes a reference above any logit, so that its
-// exponentials are 0 and products with them finite, and has no say in the flag. (No column's logit represents such a row, and
-// one prompt token that the loss masks would send a whole chunk the second way.)
+// exponentials are 0 and products with them finite, and marks no row block. (No column's logit represents such a row, and
+// one prompt token that the loss masks would have a block gone over again.)
 constexpr float REF_IGNORED = 0x1p126f;
 SISA_DEV bool left_out(const sisa_lmce_fwd_args& a, int64_t y) { return y == a.ignore_index && !a.lse; }
 
-template <bool REF>
-__global__ __launch_bounds__(CRW * CSP) void lmce_combine_kernel(sisa_lmce_fwd_args a, int S, CeTrainRows tr) {
+template <CombineMode MODE>
+__global__ __launch_bounds__(CRW * CSP) void lmce_combine_kernel(sisa_lmce_fwd_args a, int S, const float* zlab,
+                                                                 CeTrainRows tr) {
+    constexpr bool REF = MODE != TOP;
     __shared__ float pm[CSP][CRW], ps[CSP][CRW];
-    if (tr.gate && *tr.gate == 0) return;
+    const int lane = threadIdx.x & 63;
+    const int64_t N = a.N;
+    const int rb = (int)((int64_t)blockIdx.x * CRW / TR), blocks = (int)((N + TR - 1) / TR);
+    int nrb = blocks, slot = rb;
+    if (MODE != LABEL && tr.marks) {
+        if (tr.marks[0] == 0 || tr.marks[1 + rb] == 0) return;
+        nrb = marks_before(tr.marks, blocks, lane);
+        slot = marks_before(tr.marks, rb, lane);
+        S = ce_split(nrb, (int)((a.Vp + TV - 1) / TV)).S;
+    }
     const int lr = threadIdx.x % CRW, part = threadIdx.x / CRW;
-    const int64_t n = (int64_t)blockIdx.x * CRW + lr, N = a.N;
+    const int64_t n = (int64_t)blockIdx.x * CRW + lr, np = (int64_t)nrb * TR;
+    const float* in = a.workspace + (int64_t)slot * TR + (n - (int64_t)rb * TR);
     float mm = M_FLOOR_CE, ss = 0.f;
     if (n < N) {
         for (int sp = part; sp < S; sp += CSP) {
-            const float s = a.workspace[(int64_t)(S + sp) * N + n];
+            const float s = in[(S + sp) * np];
             if constexpr (REF) {
                 ss += s;
             } else {
-                const float m = a.workspace[(int64_t)sp * N + n];
+                const float m = in[sp * np];
                 const float mn = fmaxf(mm, m);
                 ss = fmaf(ss, fast_exp2(mm - mn), s * fast_exp2(m - mn));
                 mm = mn;
@@ -356,12 +408,13 @@ __global__ __launch_bounds__(CRW * CSP) void lmce_combine_kernel(sisa_lmce_fwd_a
     ps[part][lr] = ss;
     __syncthreads();
     if (part != 0 || n >= N) return;
+    const int64_t y = a.labels[n];
+    const bool out = left_out(a, y);
     if constexpr (REF) {
         mm = tr.ref[n];
         ss = 0.f;
 #pragma unroll
         for (int p = 0; p < CSP; ++p) ss += ps[p][lr];
-        if (!(ss >= Z_MIN && ss <= Z_MAX) && !left_out(a, a.labels[n])) *tr.flag = 1;   // NaN too; all store the same value
     } else {
 #pragma unroll
         for (int p = 1; p < CSP; ++p) mm = fmaxf(mm, pm[p][lr]);
@@ -369,39 +422,48 @@ __global__ __launch_bounds__(CRW * CSP) void lmce_combine_kernel(sisa_lmce_fwd_a
 #pragma unroll
         for (int p = 0; p < CSP; ++p) ss = fmaf(ps[p][lr], fast_exp2(pm[p][lr] - mm), ss);
     }
+    if constexpr (MODE == LABEL)         // NaN too; all who mark store the same value
+        if (!out && !(ss >= Z_MIN && ss <= Z_MAX)) tr.marks[0] = tr.marks[1 + rb] = 1;
     const float l2 = mm + __builtin_amdgcn_logf(ss);
-    const float lse = l2 * LN2;
-    const int64_t y = a.labels[n];
-    float loss;
-    if (y == a.ignore_index) loss = 0.f;
-    else if (y < 0 || y >= a.V) loss = __builtin_nanf("");
-    else loss = lse - a.workspace[2 * (int64_t)S * N + n];
-    a.loss_rows[n] = loss;
-    if (a.lse) a.lse[n] = lse;
-    if (tr.lse2) {
-        tr.lse2[n] = l2;
-        const int lab = (y != a.ignore_index && y >= 0 && y < a.V) ? (int)y : -1;   // its logit exists only then
-        const float sn = y == a.ignore_index ? 0.f : tr.inv_n[0] * tr.gscale;
+    if constexpr (MODE != AGAIN) {
+        const float lse = l2 * LN2;
+        float loss;
+        if (y == a.ignore_index) loss = 0.f;
+        else if (y < 0 || y >= a.V) loss = __builtin_nanf("");
+        else loss = lse - zlab[n];
+        a.loss_rows[n] = loss;
+        if (a.lse) a.lse[n] = lse;
+        if (MODE == TOP && tr.cn && !out) tr.ref[n] = l2;
+    }
+    const int lab = (y != a.ignore_index && y >= 0 && y < a.V) ? (int)y : -1;   // its logit exists only then
+    const float sn = y == a.ignore_index || !tr.inv_n ? 0.f : tr.inv_n[0] * tr.gscale;
+    if constexpr (REF) {
+        if (!tr.cn) return;
         float gl = sn;
-        if (REF && tr.cn) {
-            tr.cn[n] = left_out(a, y) ? 0.f : sn / ss;
-            if (lab >= 0) {   // p - 1 is formed here in fp32: taken apart, the two roundings of p would outweigh it near p = 1
-                gl = sn * (1.f - fast_exp2(fmaf(a.workspace[2 * (int64_t)S * N + n], LOG2E, -mm)) / ss);
-                tr.probs[n * a.Vp + lab] = (__bf16)0.f;
-            }
+        tr.cn[n] = out ? 0.f : sn / ss;
+        if (lab >= 0) {   // p - 1 is formed here in fp32: taken apart, the two roundings of p would outweigh it near p = 1
+            gl = sn * (1.f - fast_exp2(fmaf(zlab[n], LOG2E, -mm)) / ss);
+            tr.probs[n * a.Vp + lab] = (__bf16)0.f;
         }
         tr.rinfo[n] = float2{gl, __int_as_float(lab)};
+    } else if (tr.lse2) {
+        tr.lse2[n] = l2;
+        tr.rinfo[n] = float2{sn, __int_as_float(lab)};
     }
 }
 
 // The reference of a row's exponentials: the logit of its label (of column 0 without a valid one), in log2 units. Any
 // column's logit bounds the row's sum below by 1; the label's is near the largest wherever the loss is small. Rows left
-// out: REF_IGNORED. One wave per row; also clears the flag.
+// out: REF_IGNORED. One wave per row; also clears the marks.
 template <class T>
-__global__ __launch_bounds__(256) void lmce_ref_kernel(sisa_lmce_fwd_args a, float* ref, int* flag) {
+__global__ __launch_bounds__(256) void lmce_ref_kernel(sisa_lmce_fwd_args a, float* ref, int* marks) {
     const int64_t n = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
-    if (blockIdx.x == 0 && threadIdx.x == 0) *flag = 0;
+    if (threadIdx.x == 0 && blockIdx.x % (TR / 4) == 0) {
+        const int rb = blockIdx.x / (TR / 4);
+        marks[1 + rb] = 0;
+        if (rb == 0) marks[0] = 0;
+    }
     if (n >= a.N) return;
     const int64_t y = a.labels[n];
     if (left_out(a, y)) {
@@ -421,47 +483,74 @@ __global__ __launch_bounds__(256) void lmce_ref_kernel(sisa_lmce_fwd_args a, flo
     if (lane == 0) ref[n] = d * LOG2E;
 }
 
-// Logits GEMM and combine. bf16: against the label logits (REF), then, gated on the flag of a row that counts whose sum left
-// [Z_MIN, Z_MAX] (its label's logit more than 41 below the row's largest, or non-finite values), again against the
-// tile-half maxima; the gated launches of an unflagged call end at once. That spares each logit the running maximum,
-// and lets the gradient products of the training pass take the stored exponentials as they are. fp16 has too little
-// exponent range for a reference per row and always takes the maxima.
-template <class T, bool STORE>
-int launch_logits(const sisa_lmce_fwd_args* a, T* probs, float* mtab, const CeTrainRows& rows, float* ref, int* flag,
-                  hipStream_t st) {
-    const Split sp = ce_split(a->N, a->Vp);
-    const unsigned grid = (unsigned)(8 * sisa::cdiv(sisa::cdiv(a->N, TR) * sp.S, 8));
-    const unsigned cgrid = (unsigned)sisa::cdiv(a->N, CRW);
-    const int S = (int)sp.S, per = (int)sp.per;
-    CeTrainRows r = rows;
-    if constexpr (__is_same(T, __bf16)) {
-        lmce_ref_kernel<T><<<(unsigned)sisa::cdiv(a->N, 4), 256, 0, st>>>(*a, ref, flag);
-        int rc = sisa::launch_status("linear CE (reference)");
-        if (rc) return rc;
-        lmce_fwd_kernel<T, STORE, true><<<grid, 64 * NWC, 0, st>>>(*a, S, per, CeStore<T>{probs, nullptr, ref, nullptr});
-        rc = sisa::launch_status("linear CE (logits)");
-        if (rc) return rc;
-        r.ref = ref;
-        r.flag = flag;
-        lmce_combine_kernel<true><<<cgrid, CRW * CSP, 0, st>>>(*a, S, r);
-        rc = sisa::launch_status("linear CE (combine)");
-        if (rc) return rc;
-        r.gate = flag;
-    }
-    lmce_fwd_kernel<T, STORE, false><<<grid, 64 * NWC, 0, st>>>(*a, S, per, CeStore<T>{probs, mtab, nullptr, r.gate});
-    const int rc = sisa::launch_status("linear CE (logits)");
-    if (rc) return rc;
-    lmce_combine_kernel<false><<<cgrid, CRW * CSP, 0, st>>>(*a, S, r);
-    return sisa::launch_status("linear CE (combine)");
+// The workspace of the logits pass: the split partials (max and sum rows), label logits, the rows' references, the marks.
+struct CeWs {
+    float *zlab, *ref;
+    int* marks;
+    int64_t bytes;
+};
+CeWs ce_ws(float* base, int64_t N, int64_t Vp) {
+    const int64_t nrb = sisa::cdiv(N, TR);
+    CeWs w;
+    w.zlab = base + 2 * TR * ce_items(nrb, sisa::cdiv(Vp, TV));
+    w.ref = w.zlab + N;
+    w.marks = (int*)(w.ref + N);
+    w.bytes = (char*)(w.marks + 1 + nrb) - (char*)base;
+    return w;
 }
 
-// The split partials (max and sum rows, label logits), then the rows' references and the flag.
-float* ws_ref(const sisa_lmce_fwd_args* a) { return a->workspace + (2 * ce_split(a->N, a->Vp).S + 1) * a->N; }
-int* ws_flag(const sisa_lmce_fwd_args* a) { return (int*)(ws_ref(a) + a->N); }
+// Logits GEMM and combine. bf16: against the label logits (REF). That spares each logit the running maximum, and lets the
+// gradient products of the training pass take the stored exponentials as they are. A row that counts may have a sum its
+// reference was not good for: its label's logit more than 62 below its largest, or non-finite values. Its block of 256
+// rows is then gone over again, for the loss against the maxima, and in the training pass once more, storing exponentials
+// against the log-sum-exp. Those launches split the marked blocks over the whole chip and end at once without any. (16,384
+// rows of 768: 4,340 us, 4,400 with one such row, 6,830 with one in every block; taking the whole chunk through maxima
+// and forming G for dx as fp16 does took 6,090 with any.) fp16 has too little exponent range for a reference per row and
+// always takes the maxima.
+template <class T, bool STORE>
+int launch_logits(const sisa_lmce_fwd_args* a, T* probs, float* mtab, CeTrainRows r, hipStream_t st) {
+    const int64_t nrb = sisa::cdiv(a->N, TR), tiles = sisa::cdiv(a->Vp, TV);
+    const Split sp = ce_split((int)nrb, (int)tiles);
+    const CeWs ws = ce_ws(a->workspace, a->N, a->Vp);
+    const unsigned grid = (unsigned)(8 * sisa::cdiv(nrb * sp.S, 8)), again = (unsigned)(8 * sisa::cdiv(ce_items(nrb, tiles), 8));
+    const unsigned cgrid = (unsigned)sisa::cdiv(a->N, CRW);
+    CeStore<T> out{probs, mtab, nullptr, ws.zlab, nullptr};
+    if constexpr (__is_same(T, __bf16)) {
+        out.ref = r.ref = ws.ref;
+        r.marks = ws.marks;
+        lmce_ref_kernel<T><<<(unsigned)sisa::cdiv(a->N, 4), 256, 0, st>>>(*a, ws.ref, ws.marks);
+        int rc = sisa::launch_status("linear CE (reference)");
+        if (rc) return rc;
+        lmce_fwd_kernel<T, STORE, true><<<grid, 64 * NWC, 0, st>>>(*a, sp.S, sp.per, out);
+        rc = sisa::launch_status("linear CE (logits)");
+        if (rc) return rc;
+        lmce_combine_kernel<LABEL><<<cgrid, CRW * CSP, 0, st>>>(*a, sp.S, ws.zlab, r);
+        rc = sisa::launch_status("linear CE (combine)");
+        if (rc) return rc;
+        out.marks = ws.marks;
+        lmce_fwd_kernel<T, false, false><<<again, 64 * NWC, 0, st>>>(*a, 0, 0, out);
+        rc = sisa::launch_status("linear CE (logits again)");
+        if (rc) return rc;
+        lmce_combine_kernel<TOP><<<cgrid, CRW * CSP, 0, st>>>(*a, 0, ws.zlab, r);
+        rc = sisa::launch_status("linear CE (combine again)");
+        if (rc || !STORE) return rc;
+        lmce_fwd_kernel<T, true, true><<<again, 64 * NWC, 0, st>>>(*a, 0, 0, out);
+        rc = sisa::launch_status("linear CE (exponentials again)");
+        if (rc) return rc;
+        lmce_combine_kernel<AGAIN><<<cgrid, CRW * CSP, 0, st>>>(*a, 0, ws.zlab, r);
+        return sisa::launch_status("linear CE (scales again)");
+    } else {
+        lmce_fwd_kernel<T, STORE, false><<<grid, 64 * NWC, 0, st>>>(*a, sp.S, sp.per, out);
+        const int rc = sisa::launch_status("linear CE (logits)");
+        if (rc) return rc;
+        lmce_combine_kernel<TOP><<<cgrid, CRW * CSP, 0, st>>>(*a, sp.S, ws.zlab, r);
+        return sisa::launch_status("linear CE (combine)");
+    }
+}
 
 template <class T>
 int launch_lmce_fwd(const sisa_lmce_fwd_args* a, hipStream_t st) {
-    return launch_logits<T, false>(a, nullptr, nullptr, CeTrainRows{}, ws_ref(a), ws_flag(a), st);
+    return launch_logits<T, false>(a, nullptr, nullptr, CeTrainRows{}, st);
 }
 
 }  // namespace
@@ -469,29 +558,25 @@ int launch_lmce_fwd(const sisa_lmce_fwd_args* a, hipStream_t st) {
 namespace sisa {
 namespace detail {
 
-// Bytes of the logits pass's workspace (partials, references, flag).
-int64_t lmce_fwd_ws_bytes(int64_t N, int64_t Vp) {
-    return (2 * ce_split(N, Vp).S + 2) * N * (int64_t)sizeof(float) + 16;
-}
+int64_t lmce_fwd_ws_bytes(int64_t N, int64_t Vp) { return ce_ws(nullptr, N, Vp).bytes; }
 
 // The training pass's forward: the logits GEMM storing the exponentials (probs: (N, Vp) in the compute dtype), then the
-// split combine writing the loss rows, lse in log2 units and each row's gradient scale, for bf16 also s_n / Z_n (cn).
-// Afterwards *flag (returned; null for fp16) tells on the device which exponentials probs holds: zero, those against
-// one reference per row, G = probs * cn off the label, whose entry of probs is zero, and -rinfo.x at it; nonzero or null,
-// those against the tile-half maxima in mtab ((2 * ceil(Vp / 256), N) fp32). a->workspace: lmce_fwd_ws_bytes.
+// split combine writing the loss rows and each row's gradient scale. bf16: exponentials against one reference per row,
+// G = probs * cn off the label, whose entry of probs is zero, and -rinfo.x at it. fp16: exponentials against the tile-half
+// maxima in mtab ((2 * ceil(Vp / 256), N) fp32), lse in log2 units, rinfo.x = s_n. a->workspace: lmce_fwd_ws_bytes.
 int lmce_train_forward(const sisa_lmce_fwd_args* a, void* probs, float* mtab, float* lse2, float2* rinfo, float* cn,
-                       const float* inv_n, float gscale, const int** flag, hipStream_t st) {
+                       const float* inv_n, float gscale, hipStream_t st) {
     CeTrainRows r{};
-    r.lse2 = lse2;
     r.rinfo = rinfo;
     r.inv_n = inv_n;
     r.gscale = gscale;
-    r.cn = cn;
-    r.probs = (__bf16*)probs;
-    *flag = a->dtype == SISA_BF16 ? ws_flag(a) : nullptr;
-    if (a->dtype == SISA_BF16)
-        return launch_logits<__bf16, true>(a, (__bf16*)probs, mtab, r, ws_ref(a), ws_flag(a), st);
-    return launch_logits<_Float16, true>(a, (_Float16*)probs, mtab, r, nullptr, nullptr, st);
+    if (a->dtype == SISA_BF16) {
+        r.cn = cn;
+        r.probs = (__bf16*)probs;
+        return launch_logits<__bf16, true>(a, (__bf16*)probs, nullptr, r, st);
+    }
+    r.lse2 = lse2;
+    return launch_logits<_Float16, true>(a, (_Float16*)probs, mtab, r, st);
 }
 
 }  // namespace detail

@@ -9,32 +9,32 @@
 //   1. the logits GEMM of sisa_lmce_fwd (lmce_fwd.hip) with its STORE epilogue: each row's exponentials go to a (N, Vp)
 //      buffer in the compute dtype. bf16: p~ = exp2(logit * log2e - r_n) against one reference per row, its label's
 //      logit, so that G = p~ s_n / Z_n - s_n [v == label_n] with Z_n = sum_v p~ and the row's scale s_n = inv_n * gscale
-//      (0 for ignored rows). A row whose Z_n leaves [2^-20, 2^60] raises the chunk's flag, and launches gated on it redo
-//      the chunk the second way (also fp16's, whose exponent range is too small for the first): against m_t, the row's
-//      maximum over one 128-column half of a vocabulary tile, kept in a (2 * tiles, N) table. The loss rows are bitwise
-//      those of sisa_lmce_fwd either way;
-//   2. first way: the combine has taken the label's p~ out of the buffer and formed s_n (1 - p) in fp32. One launch of
+//      (0 for ignored rows). Blocks of 256 rows with a row whose Z_n leaves [2^-20, 2^90] are stored again, against
+//      the rows' log-sum-exps. fp16, whose exponent range is too small for that: against m_t, the row's maximum over one
+//      128-column half of a vocabulary tile, kept in a (2 * tiles, N) table. The loss rows are bitwise those of
+//      sisa_lmce_fwd either way;
+//   2. bf16: the combine has taken the label's p~ out of the buffer and formed s_n (1 - p) in fp32. One launch of
 //      lmce_grad_kernel runs dW tiles (256 vocabulary x 256 hidden, all rows of the chunk as K) first, G = p~ s_n / Z_n
 //      formed while staging it into LDS (grad_tile), then dx tiles (256 rows x 256 hidden, K = a range of the vocabulary: dx
 //      is split so that both kinds of workgroup run about equally long), plain products of the stored exponentials by
 //      buffer loads straight into LDS (plain_tile); the dx reduction applies s_n / Z_n and adds the label terms in fp32;
-//   3. second way: lmce_scale_kernel turns the m_t table into c = exp2(m_t - lse2) * s_n in place, so that
+//   3. fp16: lmce_scale_kernel turns the m_t table into c = exp2(m_t - lse2) * s_n in place, so that
 //      G[n, v] = p~[n, v] * c[n, tile half of v] - s_n [v == label_n], and writes each row's label entry of G; the same
 //      launch of lmce_grad_kernel then forms G from p~ and c while staging it into LDS (grad_tile: 16-byte loads, 8
 //      multiplies, the rare label subtraction, one rounding and one 16-byte LDS store per 8 values);
 //   4. lmce_dx_reduce_kernel adds the dx splits in split order.
-// Rounding: p~ once, then G; the first way's dx only p~, its label terms exact to fp32. A label's G, p - 1 times s_n, keeps
+// Rounding: p~ once, then G; bf16's dx only p~, its label terms exact to fp32. A label's G, p - 1 times s_n, keeps
 // its relative precision where p is near 1 (taken from the products of two rounded numbers, dx was off by 20 % of its
 // norm and dW by 29 % for rows with 1 - p near 0.008).
-// At 16,384 rows of 768 (V 50,277) the gradient launch takes 2,737 us the first way (0.93 PFLOP/s) and 3,209 the second;
-// 175 and 204 us at 1,023 rows of 512.
+// At 16,384 rows of 768 (V 50,277) the gradient launch takes 2,737 us in bf16 (0.93 PFLOP/s) and took 3,209 formed as
+// fp16's is; 175 and 204 us at 1,023 rows of 512.
 // G and the logits are never written to memory; the only large buffer is the chunk's exponentials (read once per
 // output column tile). Deterministic: no atomics.
 //
 // Tile arithmetic: a workgroup of 2 x 4 waves, two waves per SIMD (249 VGPRs); a wave owns 128 hidden x 64 rows
 // (dx) or 128 hidden x 64 vocabulary (dW) as 8 x 4 blocks of v_mfma_f32_16x16x32 (128 accumulators; all 12 operand
 // fragments of a 32-deep step are read before its 32 MFMAs), hidden on the A side so that a lane's 4 results are 4
-// consecutive hidden values (16-byte stores). The second way's next exponentials are loaded into registers before a
+// consecutive hidden values (16-byte stores). Exponentials to form G from are loaded into registers before a
 // stage's MFMAs and formed into G in LDS after them. dx reads W_pad as A with the feature-map transpose read (K = vocabulary, W_pad
 // rows) and G as B with direct 16-byte fragment reads (K = vocabulary along G rows); dW reads x and G both with the
 // sequence-map transpose read (K = rows). Workgroup i runs on XCD i % 8; each XCD takes consecutive work items, so
@@ -46,7 +46,7 @@ namespace sisa {
 namespace detail {
 int64_t lmce_fwd_ws_bytes(int64_t N, int64_t Vp);
 int lmce_train_forward(const sisa_lmce_fwd_args* a, void* probs, float* mtab, float* lse2, float2* rinfo, float* cn,
-                       const float* inv_n, float gscale, const int** flag, hipStream_t st);
+                       const float* inv_n, float gscale, hipStream_t st);
 }  // namespace detail
 }  // namespace sisa
 
@@ -70,10 +70,10 @@ struct __attribute__((aligned(16))) GradLds {
 
 struct GradArgs {
     const void* probs;              // (N, Vp) exponentials p~ in the compute dtype, row stride Vp
-    const float* cs;                // (2 * tiles, N): c = exp2(m_t - lse2) * s_n
-    const float2* rinfo;            // (N,) per row: s_n (first way: s_n (1 - p_label)), and the label (bit pattern of an int;
-                                    // -1 if none)
-    const float* glab;              // (N,) per row: G at the label, p~ * c - s_n rounded once to the compute dtype
+    const float* cs;                // fp16: (2 * tiles, N): c = exp2(m_t - lse2) * s_n
+    const float2* rinfo;            // (N,) per row: s_n (bf16: s_n (1 - p_label)), and the label (bit pattern of an int; -1 if
+                                    // none)
+    const float* glab;              // fp16: (N,) per row: G at the label, p~ * c - s_n rounded once to the compute dtype
     const int64_t* labels;
     const void* x;
     const void* w;
@@ -84,8 +84,7 @@ struct GradArgs {
     int dx_splits, dx_per;          // vocabulary splits of dx, 64-column stages per split
     int n_dw, n_dw_pad, n_dx;       // dW items (blocks padded to a multiple of 8), dx items
     int accumulate;
-    const int* flag;                // device: nonzero = exponentials against tile-half maxima (null: always so)
-    const float* cn;                // (N,) s_n / Z_n (per-row references)
+    const float* cn;                // bf16: (N,) s_n / Z_n
 };
 
 SISA_DEV int64_t clamp_bytes(int64_t b) {
@@ -143,8 +142,8 @@ SISA_DEV void store_tile(const GradArgs& a, f32x4 (&acc)[IB][JB], int vt, int sp
 }
 
 // One output tile: DW (dW tile u = vocabulary tile * dts + hidden tile) or dx (u = (row block * dx_splits + split)
-// * dts + hidden tile). ROW (dW only): the exponentials are relative to one reference per row, c = s_n / Z_n and G at the
-// label -s_n (1 - p_label).
+// * dts + hidden tile). ROW (bf16's dW): the exponentials are relative to one reference per row, c = s_n / Z_n and G at
+// the label -s_n (1 - p_label).
 template <class T, bool DW, bool ROW>
 SISA_DEV void grad_tile(const GradArgs& a, GradLds<T>& sm, int u) {
     const int tid = threadIdx.x, lane = tid & 63, grp = lane >> 4, lc = lane & 15;
@@ -356,14 +355,9 @@ __global__ __launch_bounds__(64 * NWG) void lmce_grad_kernel(GradArgs a) {
     const bool dw = i < a.n_dw_pad;
     const int u = dw ? xcd_item(i, a.n_dw) : xcd_item(i - a.n_dw_pad, a.n_dx);
     if (u < 0) return;
-    if constexpr (__is_same(T, __bf16)) {
-        if (a.flag && *a.flag == 0) {
-            if (dw) grad_tile<T, true, true>(a, sm, u);
-            else plain_tile<T>(a, sm, u);
-            return;
-        }
-    }
-    if (dw) grad_tile<T, true, false>(a, sm, u);
+    constexpr bool ROW = __is_same(T, __bf16);
+    if (dw) grad_tile<T, true, ROW>(a, sm, u);
+    else if constexpr (ROW) plain_tile<T>(a, sm, u);
     else grad_tile<T, false, false>(a, sm, u);
 }
 
@@ -371,9 +365,7 @@ __global__ __launch_bounds__(64 * NWG) void lmce_grad_kernel(GradArgs a) {
 // row's label also writes G at the label, p~ * c - s_n, rounded once to T (glab, kept in fp32)
 template <class T>
 __global__ __launch_bounds__(256) void lmce_scale_kernel(float* cs, const float* lse2, const float2* rinfo,
-                                                         const T* probs, int64_t Vp, float* glab, int64_t N,
-                                                         const int* gate) {
-    if (gate && *gate == 0) return;
+                                                         const T* probs, int64_t Vp, float* glab, int64_t N) {
     const int64_t n = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (n >= N) return;
     const int k = blockIdx.y;
@@ -386,11 +378,11 @@ __global__ __launch_bounds__(256) void lmce_scale_kernel(float* cs, const float*
         glab[n] = (float)cvt<T>(fmaf((float)probs[n * Vp + lab], c, -ri.x));
 }
 
-// dx[n, :] = sum over the splits, in split order, of the partial rows; with per-row references (flag given and zero) that
-// sum is scaled by cn[n], and the label's term s_n (1 - p_n) W[label_n] subtracted
+// dx[n, :] = sum over the splits, in split order, of the partial rows; bf16: that sum is scaled by cn[n], and the label's
+// term s_n (1 - p_n) W[label_n] subtracted
 template <class T>
 __global__ __launch_bounds__(256) void lmce_dx_reduce_kernel(const float* part, float* dx, int64_t N, int D, int S,
-                                                             int64_t lddx, const int* flag, const float* cn,
+                                                             int64_t lddx, const float* cn,
                                                              const float2* rinfo, const T* w, int64_t ldw) {
     const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
     const int q = D / 4;
@@ -398,7 +390,7 @@ __global__ __launch_bounds__(256) void lmce_dx_reduce_kernel(const float* part, 
     const int64_t n = idx / q, d = 4 * (idx % q);
     f32x4 s = lds4f(part + n * D + d);
     for (int sp = 1; sp < S; ++sp) s += lds4f(part + ((int64_t)sp * N + n) * D + d);
-    if (flag && *flag == 0) {
+    if constexpr (__is_same(T, __bf16)) {
         s *= cn[n];
         const float2 ri = rinfo[n];
         const int lab = __float_as_int(ri.y);
@@ -486,20 +478,17 @@ extern "C" int sisa_lmce_train(const sisa_lmce_train_args* a, void* stream) {
     sisa_lmce_fwd_args f{a->N, a->V, a->Vp, a->D, a->dtype, a->x, a->ldx, a->w, a->ldw, a->labels, a->ignore_index,
                          a->lse, a->loss_rows, (float*)(ws + l.part)};
     float* cn = (float*)(ws + l.cn);
-    const int* flag = nullptr;       // bf16: which exponentials the logits pass left (lmce_train_forward)
-    int rc = sisa::detail::lmce_train_forward(&f, ws + l.probs, cs, lse2, rinfo, cn, a->inv_n, a->gscale, &flag, st);
+    int rc = sisa::detail::lmce_train_forward(&f, ws + l.probs, cs, lse2, rinfo, cn, a->inv_n, a->gscale, st);
     if (rc || (a->dx == nullptr && a->dw == nullptr)) return rc;
 
     const int64_t tiles = sisa::cdiv(a->Vp, TV);
-    const dim3 sgrid((unsigned)sisa::cdiv(a->N, 256), (unsigned)(2 * tiles));
-    if (a->dtype == SISA_BF16)
-        lmce_scale_kernel<__bf16><<<sgrid, 256, 0, st>>>(cs, lse2, rinfo, (const __bf16*)(ws + l.probs), a->Vp, glab, a->N,
-                                                         flag);
-    else
+    if (a->dtype == SISA_F16) {
+        const dim3 sgrid((unsigned)sisa::cdiv(a->N, 256), (unsigned)(2 * tiles));
         lmce_scale_kernel<_Float16><<<sgrid, 256, 0, st>>>(cs, lse2, rinfo, (const _Float16*)(ws + l.probs), a->Vp, glab,
-                                                           a->N, flag);
-    rc = sisa::launch_status("sisa_lmce_train (scale)");
-    if (rc) return rc;
+                                                           a->N);
+        rc = sisa::launch_status("sisa_lmce_train (scale)");
+        if (rc) return rc;
+    }
 
     GradArgs g{};
     g.probs = ws + l.probs;
@@ -524,9 +513,8 @@ extern "C" int sisa_lmce_train(const sisa_lmce_train_args* a, void* stream) {
     g.dw = a->dw;
     g.lddw = a->lddw;
     g.accumulate = a->dw_accumulate != 0;
-    g.flag = flag;
     g.cn = cn;
-    const bool reduce = S > 1 || flag;
+    const bool reduce = S > 1 || a->dtype == SISA_BF16;
     if (reduce) {
         g.dxo = (float*)(ws + l.dxp);
         g.lddxo = a->D;
@@ -544,10 +532,10 @@ extern "C" int sisa_lmce_train(const sisa_lmce_train_args* a, void* stream) {
     if (a->dx == nullptr || !reduce) return SISA_OK;
     const unsigned rgrid = (unsigned)sisa::cdiv(a->N * (a->D / 4), 256);
     if (a->dtype == SISA_BF16)
-        lmce_dx_reduce_kernel<__bf16><<<rgrid, 256, 0, st>>>(g.dxo, a->dx, a->N, a->D, S, a->lddx, flag, cn, rinfo,
+        lmce_dx_reduce_kernel<__bf16><<<rgrid, 256, 0, st>>>(g.dxo, a->dx, a->N, a->D, S, a->lddx, cn, rinfo,
                                                              (const __bf16*)a->w, a->ldw);
     else
-        lmce_dx_reduce_kernel<_Float16><<<rgrid, 256, 0, st>>>(g.dxo, a->dx, a->N, a->D, S, a->lddx, flag, cn, rinfo,
+        lmce_dx_reduce_kernel<_Float16><<<rgrid, 256, 0, st>>>(g.dxo, a->dx, a->N, a->D, S, a->lddx, cn, rinfo,
                                                                (const _Float16*)a->w, a->ldw);
     return sisa::launch_status("sisa_lmce_train (dx splits)");
 }

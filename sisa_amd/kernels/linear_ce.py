@@ -13,15 +13,14 @@ How the work is arranged here (every kernel is HIP, ``libsisa_hip.so``; no libra
   ``sisa_lmce_fwd`` (csrc/lmce_fwd.hip). An MFMA GEMM whose tiles are reduced on the fly to each row's log-sum-exp
   and label logit; no logits are stored anywhere.
 * Gradients wanted: ``sisa_lmce_train`` (csrc/lmce_train.hip) per chunk of rows. The same logits GEMM also stores
-  each exponential in the compute dtype, bf16 against one reference per row (its label's logit); then one launch of MFMA
-  tiles computes dW from G = (softmax - onehot) / N_valid * gscale formed while staging it into LDS, and dx as the plain
-  product of the stored exponentials, with the softmax normaliser and the label term applied to the sum in fp32. Chunks
-  with a row that reference does not suit, and fp16, take the exponentials against maxima over half vocabulary tiles and
-  form G for dx, too, while
-  staging it into LDS. Neither the logits nor G are ever written. The reference's chunk loop (linear_ce.py:160-191:
-  logits GEMM, row kernel, dx and dW GEMMs) has the same contract; its chunk budget is 1 GiB of logits, this one 2 GiB
-  of exponentials (one chunk at N = 16,384, V = 50,277), because every chunk after the first re-reads and adds the
-  fp32 dW.
+  each exponential in the compute dtype, bf16 against one reference per row: its label's logit, or, in blocks of 256 rows
+  with a row which that does not suit, its log-sum-exp. Then one launch of MFMA tiles computes dW from
+  G = (softmax - onehot) / N_valid * gscale formed while staging it into LDS, and dx as the plain product of the stored
+  exponentials, with the softmax normaliser and the label term applied to the sum in fp32. fp16 takes the exponentials
+  against maxima over half vocabulary tiles and forms G for dx, too, while staging it into LDS. Neither the logits nor G
+  are ever written. The reference's chunk loop (linear_ce.py:160-191: logits GEMM, row kernel, dx and dW GEMMs) has the
+  same contract; its chunk budget is 1 GiB of logits, this one 2 GiB of exponentials (one chunk at N = 16,384,
+  V = 50,277), because every chunk after the first re-reads and adds the fp32 dW.
 
 Both paths round each logit, accumulated in fp32 by the MFMAs, once to the compute dtype before the log-sum-exp, as
 the reference's row kernel reads bf16/fp16 logits (linear_ce.py:166-170), so the loss has the reference's rounding

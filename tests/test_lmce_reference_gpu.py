@@ -1,6 +1,5 @@
-"""The linear cross-entropy's two ways of keeping a row's exponentials: against one reference per row (its label's
-logit; plain gradient products) and, where a row's sum leaves that reference's range, against the maxima over half
-vocabulary tiles. A chunk takes the second way as soon as one of its rows that count needs it."""
+"""The linear cross-entropy's references of a row's exponentials: its label's logit, and for blocks of 256 rows with a row
+whose sum that does not suit, the log-sum-exp, found against the maxima over half vocabulary tiles."""
 import pytest
 import torch
 
@@ -186,3 +185,51 @@ def test_ignored_rows_are_never_outliers(N):
         LC.lmce_fused_loss_rows(xo, LC.padded_weight(w, torch.bfloat16), lab, 1003, -100, lse)
         logits = (xo.double() @ w.double().t()).to(torch.bfloat16).double()
         assert float((lse.double() - torch.logsumexp(logits, 1)).abs().max()) <= 1e-4
+
+
+def _outliers(x, w, lab, gaps):
+    """``gaps``: row -> how far the row's label lies below its largest logit."""
+    x, lab = x.clone(), lab.clone()
+    d = (w[1] - w[0]).double()
+    for n, gap in gaps.items():
+        x[n], lab[n] = (d * (gap / d.norm() ** 2)).to(torch.bfloat16), 0
+    return x, w, lab
+
+
+# a label's logit up to 62 below the largest suits; 63 is the first that does not, from 89 the exponentials overflow; blocks 0,
+# 1, the last and a partial one, past the 64 blocks that a wave looks at together, every block, and fewer splits than tiles
+@pytest.mark.gpu
+@pytest.mark.parametrize("N,D,V,gaps", [(700, 128, 1003, {3: 64.0}), (700, 128, 1003, {300: 100.0}),
+                                        (700, 128, 1003, {3: 61.0, 300: 64.0}),
+                                        (700, 128, 50277, {0: 70.0, 699: 100.0}), (513, 64, 1003, {512: 300.0}),
+                                        (16900, 64, 130, {100: 70.0, 16400: 64.0, 16899: 100.0}),
+                                        (16900, 64, 130, {256 * i + 7: 64.0 + i for i in range(66)})])
+def test_outliers_reach_their_row_block_alone(N, D, V, gaps):
+    x, w, lab = _case(N, D, V, N + V)
+    lab[list(gaps)] = 0
+    case = _outliers(x, w, lab, gaps)
+    base, got, ref = _run(x, w, lab), _run(*case), _truth(*case)
+    block = torch.arange(N, device=DEV) // 256
+    hit = torch.isin(block, torch.tensor([n // 256 for n, gap in gaps.items() if gap > 62], device=DEV))
+    same = ~hit & ~torch.isin(torch.arange(N, device=DEV), torch.tensor(list(gaps), device=DEV))
+    assert torch.equal(got[1][same], base[1][same])
+    rest = torch.ones(N, dtype=torch.bool, device=DEV)
+    rest[list(gaps)] = False
+    assert abs(float(got[0] - ref[0])) <= 2 ** -8 * (1 + abs(float(ref[0])))
+    assert _rel(got[1], ref[1]) <= 3 * 2 ** -8 and _rel(got[1][rest], ref[1][rest]) <= 3 * 2 ** -8
+    assert _rel(got[2], ref[2]) <= 3 * 2 ** -8 and _rel(got[2][2:], ref[2][2:]) <= 3 * 2 ** -8
+    with torch.no_grad():
+        from sisa_amd.kernels.linear_ce import linear_cross_entropy
+        assert torch.equal(linear_cross_entropy(*case), got[0])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("bad", [float("nan"), float("inf")])
+def test_a_row_that_is_not_finite(bad):
+    x, w, lab = _case(700, 128, 1003, 21)
+    x2 = x.clone()
+    x2[300, 5] = bad
+    base, got = _run(x, w, lab), _run(x2, w, lab)
+    assert not torch.isfinite(got[0]) and torch.isnan(got[1][300]).all() and torch.isnan(got[2]).any()
+    keep = torch.arange(700, device=DEV) // 256 != 1
+    assert torch.equal(got[1][keep], base[1][keep]) and torch.isfinite(got[1][torch.arange(700) != 300]).all()
