@@ -38,10 +38,12 @@ SISA_DEV float wave_sum(float x) {
 }
 
 // The cached rows are read once per step. A cache larger than the 256 MB last-level cache cannot be found there at the
-// next step, so from that size its rows are loaded with the non-temporal hint and displace nothing on their way.
+// next step, so from that size 16-bit rows are loaded with the non-temporal hint and displace nothing on their way.
 // Measured with 8 x 12 heads in bf16: 516 MB 108.9 -> 99.0 us (4.7 -> 5.2 TB/s), and 108.6 -> 100.5 with several such
-// caches in turn. Below the line it depends on the caller: 258 MB read again and again 51.1 -> 53.2, in turn with
-// others 58.6 -> 54.2; 16 MB 9.3 -> 10.3 and 11.2 -> 11.2.
+// caches in turn. Below the line it depends on the caller, which this call does not know: 258 MB read again and again
+// 51.1 -> 53.2, in turn with others 58.6 -> 54.2; 16 MB 9.3 -> 10.3 and 11.2 -> 11.2. The plain loads stay there. They stay
+// for fp32, too, whose lanes read 32 bytes of a row in two loads: 8 x 12 heads, 516 MB 198 -> 206 us, 1 GB 355 -> 377; 16 x
+// 16 heads, 2.7 GB 864 -> 949.
 constexpr int64_t STREAM_BYTES = (int64_t)256 << 20;
 template <class T, bool STREAM> SISA_DEV frag8<T> row8(const T* p) {
     if constexpr (STREAM) return __builtin_nontemporal_load(reinterpret_cast<const frag8<T>*>(p));
@@ -224,7 +226,8 @@ int launch_decode(const sisa_decode_args* a, TO* out, hipStream_t st) {
     const dim3 grid((unsigned)nchunk, (unsigned)rows);
     // M > 1: the rows of a head share its cache, which the caches then serve
     const int64_t bytes = (int64_t)a->B * a->H * a->N * ((2 * DH + DS) * (int64_t)sizeof(T) + 8);
-    if (a->M == 1 && bytes >= STREAM_BYTES) decode_chunk_kernel<T, true><<<grid, 64 * DW, 0, st>>>(*a);
+    const bool stream = sizeof(T) == 2 && a->M == 1 && bytes >= STREAM_BYTES;
+    if (stream) decode_chunk_kernel<T, sizeof(T) == 2><<<grid, 64 * DW, 0, st>>>(*a);
     else decode_chunk_kernel<T, false><<<grid, 64 * DW, 0, st>>>(*a);
     const int rc = sisa::launch_status("sisa_decode_attn");
     if (rc) return rc;

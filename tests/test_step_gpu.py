@@ -115,7 +115,7 @@ def test_calls_that_keep_the_module_path(monkeypatch):
 @pytest.mark.parametrize("dtype,N", [(torch.bfloat16, 54560), (torch.bfloat16, 54561), (torch.float32, 27617)])
 def test_decode_at_the_streaming_line(dtype, N):
     """Caches just below and above 256 MiB (15 heads: 4,920 or 9,720 bytes a position) give each row what its head alone,
-    far below it, gives: the loads' cache policy is all that changes."""
+    far below it, gives: the loads' cache policy is all that changes, in 16 bits, and nothing in fp32."""
     from sisa_amd.kernels.decode import sisa_decode_hip
     gen = torch.Generator(device=DEV).manual_seed(3)
 
