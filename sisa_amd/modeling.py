@@ -331,25 +331,34 @@ class SISABlock(nn.Module):
         from .generation import SISACache
         from .kernels import step
 
-        # A forced implementation that x does not meet raises in the module path, or not at all: a cached fp32 call runs
-        # the unfused kernels in place of "hip_fused", and a decode step selects nothing.
-        if type(cache) is not SISACache or not self._norm_rows_ok(x) or not step.unobserved(x) \
-                or self.config.attn_impl not in ("auto", "hip_fused") \
-                or not backends.meets("hip_fused", x, self.config) or not step.plain(self, SISABlock):
+        # Cheap conditions first: a call that keeps the module path pays for them in every layer. A forced implementation
+        # that x does not meet raises in the module path, or not at all: a cached fp32 call runs the unfused kernels in
+        # place of "hip_fused", and a decode step selects nothing.
+        if type(cache) is not SISACache or not self._norm_rows_ok(x) or backends.compute_dtype(x) not in _LOW_PRECISION \
+                or self.config.attn_impl not in ("auto", "hip_fused"):
             return None
         mods = self._modules
         at, ffn, n1, n2 = mods["attn"], mods["ffn"], mods["attn_norm"], mods["ffn_norm"]
-        if not (step.plain(at, SISAAttention) and step.plain(ffn, SwiGLU) and step.plain(n1, RMSNorm)
-                and step.plain(n2, RMSNorm)):
-            return None
-        linears = step.plain_linears(at._modules, ffn._modules)
-        if linears is None:
+        if not step.plain(at, SISAAttention):
             return None
         slab, mode = cache._slabs.get(at.layer_idx), backends.get_check_mode()
-        B, L, D = x.shape
-        H, lam = self.config.n_head, at.lambda_raw
+        (B, L, D), H = x.shape, self.config.n_head
+        if slab is not None and (L != 1 or B > step.MAX_ROWS or D > step.MAX_WIDTH or x.dtype not in _LOW_PRECISION):
+            return None
+        if not (step.unobserved(x) and step.plain(self, SISABlock) and step.plain(ffn, SwiGLU) and step.plain(n1, RMSNorm)
+                and step.plain(n2, RMSNorm)):
+            return None
+        lam = at.lambda_raw
         native = (x.dtype in _LOW_PRECISION and not torch.is_autocast_enabled("cuda") and lam.dtype == torch.float32
                   and lam.shape == (H,) and lam.get_device() == x.get_device() and lam.is_contiguous())
+        if slab is not None:
+            buf = slab.buffers
+            if not native or slab.filled < 1 or not step.rows_ok(x) or not step.whole(res) or buf["k"].dtype != x.dtype \
+                    or buf["k"].shape[:2] != (B, H) or buf["k"].get_device() != x.get_device():
+                return None
+        linears = step.plain_linears(at._modules, ffn._modules)
+        if linears is None or not backends.meets("hip_fused", x, self.config):
+            return None
         if slab is None:
             native = native and B * L <= step.PREFILL_ROWS and mode != "sync" and step.whole(x) and step.whole(res)
             weights = native and step.step_weights(linears, n1._parameters["weight"], n2._parameters["weight"], H, x)
@@ -357,12 +366,6 @@ class SISABlock(nn.Module):
                 return self._forward_hip(x, res, defer=True, cache=cache)
             return step.layer_prefill(x, res, *weights, lam, ffn.w_down.weight, (n1.eps, n2.eps), cache, at.layer_idx,
                                       mode == "async")
-        buf = slab.buffers
-        if not native or L != 1 or B > step.MAX_ROWS or D > step.MAX_WIDTH or slab.filled < 1 or not step.rows_ok(x) \
-                or not step.whole(res):
-            return None
-        if buf["k"].dtype != x.dtype or buf["k"].shape[:2] != (B, H) or buf["k"].get_device() != x.get_device():
-            return None
         weights = step.step_weights(linears, n1._parameters["weight"], n2._parameters["weight"], H, x)
         if weights is None:
             return None

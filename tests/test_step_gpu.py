@@ -213,3 +213,20 @@ def test_prefill_refuses_what_its_offsets_cannot_reach():
         args = _lib.PrefillArgs(B=1, L=L, H=H, FF=ff, dtype=_lib.BF16, act_ld=ff, **pointers)
         assert lib.sisa_prefill(ctypes.byref(args), None) != 0
         assert "2 GiB" in lib.sisa_last_error().decode()
+
+
+@pytest.mark.gpu
+def test_calls_refused_by_size_or_type_cost_nothing_more(monkeypatch):
+    """Steps that the kernels do not take for their size or type keep the module path before the modules are looked at."""
+    from sisa_amd import SISACache
+    from sisa_amd.kernels import step
+    ids = token_ids(65, 12, seed=1).to(DEV)
+    for rows, n, dtype in ((65, 1, torch.bfloat16), (3, 2, torch.bfloat16), (3, 1, torch.float32)):
+        model, cache = tiny_model(seed=1, attn_impl="auto").to(DEV).to(dtype).eval(), SISACache()
+        with torch.no_grad():
+            model(ids[:rows, :8], cache=cache)
+            looked = []
+            monkeypatch.setattr(step, "plain_linears", lambda *a: looked.append(a))
+            model(ids[:rows, 8:8 + n], cache=cache)
+            monkeypatch.undo()
+        assert not looked, (rows, n, dtype)
