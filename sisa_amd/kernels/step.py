@@ -19,19 +19,24 @@ from . import _lib
 from . import attention as A
 from . import fused_prep as P
 
-__all__ = ["unobserved", "plain", "plain_linears", "rows_ok", "whole", "prefill_fits", "step_weights",
-           "layer_step", "layer_prefill", "prefill", "MAX_ROWS", "MAX_WIDTH", "PREFILL_ROWS"]
+__all__ = ["unobserved", "plain", "plain_linears", "rows_ok", "whole", "prefill_takes", "step_weights",
+           "layer_step", "layer_prefill", "prefill", "MAX_ROWS", "MAX_WIDTH", "PREFILL_ROWS", "PREFILL_WORK"]
 
 MAX_ROWS, MAX_WIDTH = 64, 1024          # SISA_STEP_MAX_ROWS, SISA_STEP_MAX_D
-#: Prompts of at most this many tokens (all rows together) take ``sisa_prefill``: as far as it was measured ahead of the
-#: launch-by-launch route, whose library GEMMs gain on it with size (whole model, ms: 800 tokens at width 768 2.0 against
-#: 5.1, 8,192 tokens as 8 x 1,024 4.6 against 5.5; width 1,024 3.6 against 10.3 and 10.3 against 12.9).
-PREFILL_ROWS = 8192
+#: Prompts of at most this many tokens (all rows together) take ``sisa_prefill``, and at most PREFILL_WORK / width of them
+#: in a model wider than 1,024: as far as it was measured no slower than the launch-by-launch route, whose library GEMMs
+#: gain on it with size. Two layers of hidden width 2.7 D, us, native against launch by launch: width 768 318 and 990 for
+#: 1,024 tokens, 664 and 1,015 for 8 x 1,024; 1,024 976 and 1,095; 1,536 647 and 982 for 2,048 tokens, 1,711 and 1,625 for
+#: 8,192; 2,048 1,042 and 1,072, 2,865 and 2,477; 4,096 1,821 and 1,895 for 1,024, 4,017 and 3,656 for 3,072, 10,307 and
+#: 8,009 for 8,192.
+PREFILL_ROWS, PREFILL_WORK = 8192, 1 << 22
 
 
-def prefill_fits(rows: int, width: int, d_ff: int) -> bool:
-    """``sisa_prefill`` reads activations and weights by 32-bit offsets: each must end below 2 GiB."""
-    return max(rows, width) * (-(-d_ff // 64) * 64) * 2 < 1 << 31
+def prefill_takes(rows: int, width: int, d_ff: int) -> bool:
+    """Whether a prompt is for ``sisa_prefill``: small enough (above), and its activations and weights, which the kernels
+    read by 32-bit offsets, each ending below 2 GiB."""
+    return (rows <= PREFILL_ROWS and (width <= 1024 or rows * width <= PREFILL_WORK)
+            and max(rows, width) * (-(-d_ff // 64) * 64) * 2 < 1 << 31)
 
 
 def unobserved(x: Tensor) -> bool:

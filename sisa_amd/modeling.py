@@ -360,9 +360,10 @@ class SISABlock(nn.Module):
         if linears is None or not backends.meets("hip_fused", x, self.config):
             return None
         if slab is None:
-            native = native and B * L <= step.PREFILL_ROWS and mode != "sync" and step.whole(x) and step.whole(res)
+            native = (native and step.prefill_takes(B * L, D, ffn.w_gate.out_features) and mode != "sync"
+                      and step.whole(x) and step.whole(res))
             weights = native and step.step_weights(linears, n1._parameters["weight"], n2._parameters["weight"], H, x)
-            if not weights or not step.prefill_fits(B * L, D, weights[1]):
+            if not weights:
                 return self._forward_hip(x, res, defer=True, cache=cache)
             return step.layer_prefill(x, res, *weights, lam, ffn.w_down.weight, (n1.eps, n2.eps), cache, at.layer_idx,
                                       mode == "async")

@@ -201,12 +201,15 @@ def test_failed_cache_fill_leaves_no_entry(monkeypatch):
     assert len(cache) == 0 and cache.get(0) is None
 
 
-def test_prefill_refuses_what_its_offsets_cannot_reach():
-    """The products read their operands by 32-bit offsets: activations or weights of 2 GiB keep the fused route, and the
-    entry point refuses them."""
+def test_prefill_takes_what_it_is_faster_at_and_can_reach():
+    """Wide models hand over to the library's GEMMs at fewer tokens. The products read their operands by 32-bit offsets:
+    activations or weights of 2 GiB keep the fused route, and the entry point refuses them."""
     from sisa_amd.kernels import _lib, step
-    assert step.prefill_fits(8192, 4096, 11008) and step.prefill_fits(8192, 64, 130_000)
-    assert not step.prefill_fits(8192, 64, 131_072) and not step.prefill_fits(1, 4096, 262_144)
+    for width, most in ((64, 8192), (1024, 8192), (1088, 3855), (1536, 2730), (2048, 2048), (4096, 1024)):
+        assert step.prefill_takes(1, width, 2736) and step.prefill_takes(most, width, 2736)
+        assert not step.prefill_takes(most + 1, width, 2736)
+    assert step.prefill_takes(8192, 64, 130_000)
+    assert not step.prefill_takes(8192, 64, 131_072) and not step.prefill_takes(1, 4096, 262_144)
     lib = _lib.load()
     for L, H, ff in ((8192, 1, 131_072), (1, 64, 262_144)):
         pointers = {n: 256 for n, t in _lib.PrefillArgs._fields_ if t is ctypes.c_void_p and n != "res"}
