@@ -14,7 +14,7 @@
 //
 // Work decomposition: a wave holds RB = 64 / HP rows (HP = the projection width padded to 16, 32 or 64) with NVL =
 // HP / 8 eight-element vectors per lane (lane l holds elements 8 c .. 8 c + 7, c = l + 64 i), so RB * NVL = 8 and
-// the row length is at most 512 NVL. For up to 16 outputs and rows of at most 1024 (a multiple of 64) the projection
+// the row length is at most 512 NVL. For up to 16 outputs and rows of at most 1024 (a multiple of 64; see norm_on_mfma) the projection
 // and its adjoint run on the matrix cores: the workgroup's sixteen rows of n (of dz W_f) pass through LDS and each
 // wave forms a quarter of the columns with v_mfma_f32_16x16x4_f32 (norm_fwd_mfma_kernel, norm_bwd_mfma_kernel).
 // Otherwise a lane's RB * HP projection partial sums are reduced over the 64 lanes with a halving exchange (63
@@ -198,6 +198,14 @@ __global__ __launch_bounds__(64 * NORM_WAVES) void norm_fwd_kernel(sisa_norm_arg
 // 42 us, 55 before this and the batched tails of the reductions.
 constexpr int MFMA_DMAX = 1024;
 constexpr int NQ_SMALL = 12, NQ_LARGE = MFMA_DMAX / 64;
+// The matrix-core kernels take up to 16 outputs. Their cost does not depend on the number, that of the vector units does: of
+// many rows longer than 768 with few outputs, which are bound by memory, the larger register set and the LDS trip cost
+// more than they save. 65,536 rows of 832, forward, vector and matrix, us: 69.7 and 75.0 with 1 output, 74.3 and 77.7 with 4,
+// 81.8 and 79.4 with 8; backward 199.9 and 206.4, 202.6 and 207.2, 206.5 and 209.4, and 213.0 and 212.1 with 12. Below 16,384
+// rows the matrix kernels are the faster ones with any.
+inline bool norm_on_mfma(const sisa_norm_args* a) {
+    return a->H > 0 && a->D % 64 == 0 && a->D <= MFMA_DMAX && (a->D <= 64 * NQ_SMALL || a->H >= 12 || a->N < 16384);
+}
 constexpr int NL_PAD = 4;                       // row padding of the staged n: conflict-free 16-byte reads
 inline int64_t norm_mfma_lds_bytes(int D) { return (int64_t)16 * (D + NL_PAD) * (int64_t)sizeof(float); }
 template <class TX, class TY, int NQ>
@@ -754,7 +762,7 @@ template <class TX, class TY, int HP>
 int launch_norm_hp(const sisa_norm_args* a, int bwd, hipStream_t st) {
     constexpr int RB = 64 / HP;
     if (!bwd) {
-        if (HP == 16 && a->H > 0 && a->D % 64 == 0 && a->D <= MFMA_DMAX) {
+        if (HP == 16 && norm_on_mfma(a)) {
             const unsigned grid = (unsigned)sisa::cdiv(a->N, 16);
             const size_t lds = (size_t)norm_mfma_lds_bytes(a->D);
             if (a->D <= 64 * NQ_SMALL) norm_fwd_mfma_kernel<TX, TY, NQ_SMALL><<<grid, 64 * NORM_WAVES, lds, st>>>(*a);
@@ -769,7 +777,7 @@ int launch_norm_hp(const sisa_norm_args* a, int bwd, hipStream_t st) {
     const int64_t np = sisa::cdiv(a->N, NORM_RPW);
     const unsigned grid = (unsigned)sisa::cdiv(np, NORM_WAVES);
     const size_t lds = (size_t)norm_mfma_lds_bytes(a->D);
-    const bool mfma = HP == 16 && a->H > 0 && a->D % 64 == 0 && a->D <= MFMA_DMAX;
+    const bool mfma = HP == 16 && norm_on_mfma(a);
     if (mfma && a->D <= 64 * NQ_SMALL)
         norm_bwd_mfma_kernel<TX, TY, NQ_SMALL><<<grid, 64 * NORM_WAVES, lds, st>>>(*a, ws.dw_part);
     else if (mfma)
