@@ -454,13 +454,15 @@ __global__ __launch_bounds__(CRW * CSP) void lmce_combine_kernel(sisa_lmce_fwd_a
 
 // The reference of a row's exponentials: the logit of its label (of column 0 without a valid one), in log2 units. Any
 // column's logit bounds the row's sum below by 1; the label's is near the largest wherever the loss is small. Rows left
-// out: REF_IGNORED. One wave per row; also clears the marks.
-template <class T>
+// out: REF_IGNORED. LPR lanes a row, 8 elements each at a time (a whole wave for a row of 64
+// elements keeps 8 lanes busy: 140,000 such rows took 30 us). Also clears the marks.
+template <class T, int LPR>
 __global__ __launch_bounds__(256) void lmce_ref_kernel(sisa_lmce_fwd_args a, float* ref, int* marks) {
-    const int64_t n = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-    const int lane = threadIdx.x & 63;
-    if (threadIdx.x == 0 && blockIdx.x % (TR / 4) == 0) {
-        const int rb = blockIdx.x / (TR / 4);
+    constexpr int RPB = 256 / LPR;                        // rows of a workgroup; 256 = TR is a multiple of it
+    const int64_t n = (int64_t)blockIdx.x * RPB + threadIdx.x / LPR;
+    const int lane = threadIdx.x % LPR;
+    if (threadIdx.x == 0 && blockIdx.x % (TR / RPB) == 0) {
+        const int rb = blockIdx.x / (TR / RPB);
         marks[1 + rb] = 0;
         if (rb == 0) marks[0] = 0;
     }
@@ -473,14 +475,21 @@ __global__ __launch_bounds__(256) void lmce_ref_kernel(sisa_lmce_fwd_args a, flo
     const T* x = (const T*)a.x + n * a.ldx;
     const T* w = (const T*)a.w + (y >= 0 && y < a.V ? y : 0) * a.ldw;
     float d = 0.f;
-    for (int c = 8 * lane; c < a.D; c += 512) {
+    for (int c = 8 * lane; c < a.D; c += 8 * LPR) {
         const f32x8 xv = load_f32x8<T>(x + c), wv = load_f32x8<T>(w + c);
 #pragma unroll
         for (int e = 0; e < 8; ++e) d = fmaf(xv[e], wv[e], d);
     }
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) d += __shfl_xor(d, o);
+    for (int o = LPR / 2; o > 0; o >>= 1) d += __shfl_xor(d, o);
     if (lane == 0) ref[n] = d * LOG2E;
+}
+
+template <class T>
+void launch_ref(const sisa_lmce_fwd_args* a, float* ref, int* marks, hipStream_t st) {
+    if (a->D <= 64) lmce_ref_kernel<T, 8><<<(unsigned)sisa::cdiv(a->N, 32), 256, 0, st>>>(*a, ref, marks);
+    else if (a->D <= 256) lmce_ref_kernel<T, 32><<<(unsigned)sisa::cdiv(a->N, 8), 256, 0, st>>>(*a, ref, marks);
+    else lmce_ref_kernel<T, 64><<<(unsigned)sisa::cdiv(a->N, 4), 256, 0, st>>>(*a, ref, marks);
 }
 
 // The workspace of the logits pass: the split partials (max and sum rows), label logits, the rows' references, the marks.
@@ -518,7 +527,7 @@ int launch_logits(const sisa_lmce_fwd_args* a, T* probs, float* mtab, CeTrainRow
     if constexpr (__is_same(T, __bf16)) {
         out.ref = r.ref = ws.ref;
         r.marks = ws.marks;
-        lmce_ref_kernel<T><<<(unsigned)sisa::cdiv(a->N, 4), 256, 0, st>>>(*a, ws.ref, ws.marks);
+        launch_ref<T>(a, ws.ref, ws.marks, st);
         int rc = sisa::launch_status("linear CE (reference)");
         if (rc) return rc;
         lmce_fwd_kernel<T, STORE, true><<<grid, 64 * NWC, 0, st>>>(*a, sp.S, sp.per, out);
