@@ -200,9 +200,15 @@ SISA_DEV void grad_tile(const GradArgs& a, GradLds<T>& sm, int u) {
                 raw[p] = load16<T>(rs, (int)((rr[p] * Vp + (int64_t)vt * TV + 8 * gc) * (int64_t)sizeof(T)));
                 const int64_t n = m0 + rr[p] < N ? m0 + rr[p] : N - 1;   // rows past N: their p~ read as 0
                 cv[p] = ROW ? a.cn[n] : a.cs[(int64_t)(2 * vt + h) * N + n];
-                const float2 ri = a.rinfo[n];
-                lab[p] = m0 + rr[p] < N ? __float_as_int(ri.y) : -1;
-                gl[p] = ROW ? -ri.x : a.glab[n];
+                // nothing is computed from these before the stage's MFMAs: it would wait for all loads of the stage there
+                if constexpr (ROW) {
+                    const float2 ri = a.rinfo[n];
+                    gl[p] = ri.x;
+                    lab[p] = __float_as_int(ri.y);
+                } else {
+                    gl[p] = a.glab[n];
+                    lab[p] = __float_as_int(a.rinfo[n].y);
+                }
             }
         } else {
             const int64_t v0 = (int64_t)(k0 + g) * TK;
@@ -219,9 +225,11 @@ SISA_DEV void grad_tile(const GradArgs& a, GradLds<T>& sm, int u) {
     auto store_g = [&](int g, int buf) {
         if constexpr (DW) {
             const int vc = vt * TV + 8 * gc;
+            const int64_t m0 = (int64_t)(k0 + g) * TK;
 #pragma unroll
             for (int p = 0; p < GL; ++p)
-                g_store<T>(sm.g[buf] + toff<T, TO>(rr[p], gc), raw[p], cv[p], lab[p] < 0 ? -1 : lab[p] - vc, gl[p]);
+                g_store<T>(sm.g[buf] + toff<T, TO>(rr[p], gc), raw[p], cv[p],
+                           lab[p] < 0 || m0 + rr[p] >= N ? -1 : lab[p] - vc, ROW ? -gl[p] : gl[p]);
         } else {
             const int vc = (k0 + g) * TK + 8 * gc;
 #pragma unroll
