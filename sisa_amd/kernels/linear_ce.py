@@ -145,7 +145,7 @@ def train_workspace(chunk_sizes, Vp: int, D: int, device, dx_splits: int = 0) ->
 
 class _Problem:
     """One call's operands in the compute dtype: x (N, D) contiguous, the padded weight, int64 labels, and the
-    device scalars N_valid and 1/N_valid (fp32)."""
+    device scalars N_valid and 1/N_valid."""
 
     def __init__(self, hidden: torch.Tensor, weight: torch.Tensor, labels: torch.Tensor, ignore_index: int,
                  cdtype: torch.dtype):
@@ -161,11 +161,11 @@ class _Problem:
         self.N, self.D = self.x.shape[0], D
         self.n_valid, self.inv_n = self._count()
 
-    def _count(self) -> tuple[torch.Tensor, torch.Tensor]:
-        """The number of valid rows and its reciprocal, fp32 device scalars of one element."""
+    def _count(self) -> tuple[torch.Tensor, torch.Tensor | None]:
+        """The number of valid rows and its reciprocal, fp32 device scalars of one element; of more rows than one
+        workgroup counts, the int64 number alone (an evaluation needs no more)."""
         if self.N > SCALAR_ROWS:
-            n_valid = (self.labels != self.ignore_index).sum().to(torch.float32).reshape(1)
-            return n_valid, torch.reciprocal(n_valid)
+            return (self.labels != self.ignore_index).sum(), None
         n_valid, inv_n = torch.empty(2, dtype=torch.float32, device=self.x.device).split(1)
         _lib.call_values("sisa_ce_count", self.labels, self.labels.data_ptr(), self.N, self.ignore_index,
                          n_valid.data_ptr(), inv_n.data_ptr())
@@ -173,7 +173,7 @@ class _Problem:
 
     def _mean(self, rows: torch.Tensor) -> torch.Tensor:
         if self.N > SCALAR_ROWS:
-            return rows.sum() / self.n_valid[0]
+            return rows.sum() / self.n_valid
         mean = torch.empty((), dtype=torch.float32, device=rows.device)
         _lib.call_values("sisa_ce_mean", rows, rows.data_ptr(), self.N, self.n_valid.data_ptr(), mean.data_ptr())
         return mean
@@ -190,11 +190,12 @@ class _Problem:
         dx = torch.empty((N, Dp), dtype=torch.float32, device=dev) if want_dx else None
         dw = (torch.zeros if N == 0 else torch.empty)((Vp, Dp), dtype=torch.float32, device=dev) if want_dw else None
         step = chunk_rows(N, Vp, chunk_tokens, self.wpad.element_size())
+        inv_n = torch.reciprocal(self.n_valid.to(torch.float32)).reshape(1) if self.inv_n is None else self.inv_n
         if N:
             ws = train_workspace({min(step, N), N - (N - 1) // step * step}, Vp, Dp, dev)   # this loop's chunk sizes
             for r0 in range(0, N, step):
                 r1 = min(N, r0 + step)
-                lmce_train_chunk(self.x[r0:r1], self.wpad, self.labels[r0:r1], self.V, self.ignore_index, self.inv_n,
+                lmce_train_chunk(self.x[r0:r1], self.wpad, self.labels[r0:r1], self.V, self.ignore_index, inv_n,
                                  gscale, rows[r0:r1], None if dx is None else dx[r0:r1], dw, r0 > 0, ws)
         if dx is not None and Dp != self.D:
             dx = dx[:, :self.D]

@@ -233,3 +233,17 @@ def test_a_row_that_is_not_finite(bad):
     assert not torch.isfinite(got[0]) and torch.isnan(got[1][300]).all() and torch.isnan(got[2]).any()
     keep = torch.arange(700, device=DEV) // 256 != 1
     assert torch.equal(got[1][keep], base[1][keep]) and torch.isfinite(got[1][torch.arange(700) != 300]).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("N", [1 << 17, (1 << 17) + 1])
+def test_rows_at_the_line_of_the_scalar_kernels(N):
+    """One workgroup counts and averages up to 131,072 rows; beyond, the general sums do. Both against float64."""
+    from sisa_amd.kernels.linear_ce import linear_cross_entropy
+    x, w, lab = _case(N, 64, 130, 3)
+    got, ref = _run(x, w, lab), _truth(x, w, lab)
+    # logits rounded to 8 bits shift the loss by the mean of their errors; gradients: three 8-bit roundings
+    assert abs(float(got[0] - ref[0])) <= 2 ** -8 * (1 + abs(float(ref[0])))
+    assert _rel(got[1], ref[1]) <= 3 * 2 ** -8 and _rel(got[2], ref[2]) <= 3 * 2 ** -8
+    with torch.no_grad():
+        assert torch.equal(linear_cross_entropy(x, w.float(), lab), got[0])
