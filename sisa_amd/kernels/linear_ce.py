@@ -47,8 +47,10 @@ HIDDEN_MULTIPLE = 64             # the CE kernels stream the hidden size in 64-w
 PROBS_LIMIT = 0x7fffff00         # bytes that a chunk's stored exponentials may take: the kernels address them by 32-bit
                                  # offsets and drop what lies at 0x7ffffff0
 PROBS_BUDGET = 2 << 30           # bytes of one chunk of stored exponentials, within that
-SCALAR_ROWS = 1 << 17            # rows up to which one workgroup counts the valid ones and averages the loss: 16 and
-                                 # 8 loads a thread deep there, still less than the launches of the general sums
+SCALAR_ROWS = 1 << 16            # rows up to which one workgroup counts the valid ones and averages the loss, where the
+                                 # launches of the general sums cost more than its loads (evaluations of rows of 64 at 1,003
+                                 # tokens, us: 32,768 rows 54 and 65, 65,536 79 and 85, 98,304 128 and 115, 131,072 156
+                                 # and 114)
 
 
 # ------------------------------------------------------------------------------------------------ pieces
