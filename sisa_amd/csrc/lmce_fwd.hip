@@ -53,7 +53,8 @@ struct __attribute__((aligned(16))) CeLds {
 // What a launch stores and against what it takes its exponentials.
 //   STORE: the exponentials go to probs. REF: they are relative to one given reference per row (ref, log2 units)
 //   instead of the row's maxima over the tile halves, which go to mtab.
-//   marks: only the row blocks that it marks (null: all).
+//   MARKED: only the row blocks that marks marks. (A kernel of its own: with the choice made in the kernel of all blocks its
+//   main loop, short of scalar registers, took 1.5 % longer.)
 template <class T>
 struct CeStore {
     T* probs;                     // (N, Vp) in the compute dtype, row stride Vp; columns >= V hold 0
@@ -98,16 +99,16 @@ SISA_DEV int marked_block(const int* marks, int nrb, int slot, int lane) {
     return 0;                                    // not reached for a slot below their number
 }
 
-template <class T, bool STORE, bool REF>
+template <class T, bool STORE, bool REF, bool MARKED>
 __global__ __launch_bounds__(64 * NWC) void lmce_fwd_kernel(sisa_lmce_fwd_args a, int S, int per, CeStore<T> out) {
     __shared__ CeLds<T> sm;
-    if (out.marks && out.marks[0] == 0) return;
+    if (MARKED && out.marks[0] == 0) return;
     const int tid = threadIdx.x, lane = tid & 63, grp = lane >> 4, lc = lane & 15;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int64_t N = a.N, V = a.V;
     const int blocks = (int)((N + TR - 1) / TR), tiles = (int)((a.Vp + TV - 1) / TV);
     int nrb = blocks;
-    if (out.marks) {
+    if constexpr (MARKED) {
         nrb = marks_before(out.marks, blocks, lane);
         const Split sp = ce_split(nrb, tiles);
         S = sp.S;
@@ -121,7 +122,7 @@ __global__ __launch_bounds__(64 * NWC) void lmce_fwd_kernel(sisa_lmce_fwd_args a
     const int grp_items = RGRP * S, g0 = item / grp_items * RGRP, in_grp = item % grp_items;
     const int rg = nrb - g0 < RGRP ? nrb - g0 : RGRP;
     const int split = in_grp / rg, slot = g0 + in_grp % rg;
-    const int rb = out.marks ? marked_block(out.marks, blocks, slot, lane) : slot;
+    const int rb = MARKED ? marked_block(out.marks, blocks, slot, lane) : slot;
     const int t_begin = split * per;
     const int t_end = t_begin + per < tiles ? t_begin + per : tiles;
     const int ntiles = t_end > t_begin ? t_end - t_begin : 0;
@@ -142,9 +143,9 @@ __global__ __launch_bounds__(64 * NWC) void lmce_fwd_kernel(sisa_lmce_fwd_args a
         const int k0 = (g % nks) * TK;
 #pragma unroll
         for (int h = 0; h < 4; ++h) {
-            dma_issue<(STORE ? 8 : 4) + (REF ? 16 : 0)>(sx, X, xbytes, (int)(((row0 + 64 * h) * a.ldx + k0) * (int64_t)sizeof(T)),
+            dma_issue<(STORE ? 8 : 4) + (REF ? 16 : 0) + (MARKED ? 32 : 0)>(sx, X, xbytes, (int)(((row0 + 64 * h) * a.ldx + k0) * (int64_t)sizeof(T)),
                          sm.x[buf] + 64 * h * TK, w);
-            dma_issue<(STORE ? 9 : 5) + (REF ? 16 : 0)>(sw, W, wbytes, (int)(((v0 + 64 * h) * a.ldw + k0) * (int64_t)sizeof(T)),
+            dma_issue<(STORE ? 9 : 5) + (REF ? 16 : 0) + (MARKED ? 32 : 0)>(sw, W, wbytes, (int)(((v0 + 64 * h) * a.ldw + k0) * (int64_t)sizeof(T)),
                          sm.w[buf] + 64 * h * TK, w);
         }
     };
@@ -305,8 +306,8 @@ __global__ __launch_bounds__(64 * NWC) void lmce_fwd_kernel(sisa_lmce_fwd_args a
     }
 
     // combine the four lane groups of each row, then the two waves sharing the rows (w and w ^ 1)
-    const int64_t np = (int64_t)nrb * TR;
-    float* part = a.workspace + (int64_t)slot * TR;
+    const int64_t np = MARKED ? (int64_t)nrb * TR : (N + TR - 1) / TR * TR;
+    float* part = a.workspace + (MARKED ? (int64_t)slot * TR : row0);
     float rm[JB], rsum[JB];
 #pragma unroll
     for (int j = 0; j < JB; ++j) {
@@ -530,26 +531,26 @@ int launch_logits(const sisa_lmce_fwd_args* a, T* probs, float* mtab, CeTrainRow
         launch_ref<T>(a, ws.ref, ws.marks, st);
         int rc = sisa::launch_status("linear CE (reference)");
         if (rc) return rc;
-        lmce_fwd_kernel<T, STORE, true><<<grid, 64 * NWC, 0, st>>>(*a, sp.S, sp.per, out);
+        lmce_fwd_kernel<T, STORE, true, false><<<grid, 64 * NWC, 0, st>>>(*a, sp.S, sp.per, out);
         rc = sisa::launch_status("linear CE (logits)");
         if (rc) return rc;
         lmce_combine_kernel<LABEL><<<cgrid, CRW * CSP, 0, st>>>(*a, sp.S, ws.zlab, r);
         rc = sisa::launch_status("linear CE (combine)");
         if (rc) return rc;
         out.marks = ws.marks;
-        lmce_fwd_kernel<T, false, false><<<again, 64 * NWC, 0, st>>>(*a, 0, 0, out);
+        lmce_fwd_kernel<T, false, false, true><<<again, 64 * NWC, 0, st>>>(*a, 0, 0, out);
         rc = sisa::launch_status("linear CE (logits again)");
         if (rc) return rc;
         lmce_combine_kernel<TOP><<<cgrid, CRW * CSP, 0, st>>>(*a, 0, ws.zlab, r);
         rc = sisa::launch_status("linear CE (combine again)");
         if (rc || !STORE) return rc;
-        lmce_fwd_kernel<T, true, true><<<again, 64 * NWC, 0, st>>>(*a, 0, 0, out);
+        lmce_fwd_kernel<T, true, true, true><<<again, 64 * NWC, 0, st>>>(*a, 0, 0, out);
         rc = sisa::launch_status("linear CE (exponentials again)");
         if (rc) return rc;
         lmce_combine_kernel<AGAIN><<<cgrid, CRW * CSP, 0, st>>>(*a, 0, ws.zlab, r);
         return sisa::launch_status("linear CE (scales again)");
     } else {
-        lmce_fwd_kernel<T, STORE, false><<<grid, 64 * NWC, 0, st>>>(*a, sp.S, sp.per, out);
+        lmce_fwd_kernel<T, STORE, false, false><<<grid, 64 * NWC, 0, st>>>(*a, sp.S, sp.per, out);
         const int rc = sisa::launch_status("linear CE (logits)");
         if (rc) return rc;
         lmce_combine_kernel<TOP><<<cgrid, CRW * CSP, 0, st>>>(*a, sp.S, ws.zlab, r);
