@@ -114,7 +114,7 @@ def profiled_mfma_busy(name: str = "counters_ns_ce.txt") -> dict | None:
     t = sum(us for us, _ in rows.values())
     out = {k: v[1] for k, v in rows.items()}
     out["time_weighted"] = round(sum(us * b for us, b in rows.values()) / t, 2)
-    out["source"] = f"profiles/{name} (rocprofv3 counter passes of this build, not measured in this run)"
+    out["source"] = f"profiles/{name} (committed rocprofv3 counter passes, not measured in this run)"
     return out
 
 
@@ -775,8 +775,8 @@ def main():
         "roofline": {"bound": "mfma", "achieved": round(achieved, 3), "peak": PEAK_BF16_TFLOPS, "unit": "TFLOP/s",
                      "frac": round(achieved / PEAK_BF16_TFLOPS, 4),
                      "traffic": profiled_traffic(ATTN_KERNELS) if cfg == "ns" else None,
-                     "traffic_source": "profiles/hbm_traffic_ns_ce.txt (rocprofv3 FETCH_SIZE / WRITE_SIZE passes of this "
-                                       "build, not measured in this run)" if cfg == "ns" else None,
+                     "traffic_source": "profiles/hbm_traffic_ns_ce.txt (committed rocprofv3 FETCH_SIZE / WRITE_SIZE "
+                                       "passes, not measured in this run)" if cfg == "ns" else None,
                      "kernel": "attention fwd + bwd launches (attn_fwd, attn_bwd_dq, attn_bwd_dkv)",
                      "algorithmic": f"1152 flop per causal pair x {fl['pairs']:.4g} pairs per step"},
         "roofline_prep": {"bound": "hbm", "achieved": round(prep_gbs, 1), "peak": PEAK_HBM_GBS, "unit": "GB/s",

@@ -224,8 +224,8 @@ SISA_DEV void fwd_tile(const FwdLds<T>& sm, int qblk, int lane, int n0, int q0, 
             // The weights first, under the offset at hand: a lane's sum of 8 of them at most 2^RESCALE_LOG2 bounds
             // each. With the tile's maximum formed before them (16 max, a reduction over the lane groups and a ballot
             // between the scores and the first exponential) all 64 keys' scores had to be held at once; 32 keys at a
-            // time leave registers for the scheduler. 4 x 4096 x 8 heads 174 -> 170 us, 1 x 16384 x 16 heads
-            // 1082 -> 991, 2 x 3001 x 12 heads 81 -> 77.
+            // time leave registers for the scheduler. 4 x 4096 x 8 heads 161 -> 160 us, 1 x 16384 x 16 heads
+            // 996 -> 941, 2 x 3001 x 12 heads 80.5 -> 77 (kernel traces in turn).
             const bool over = ls > __builtin_exp2f(RESCALE_LOG2);
             if (__builtin_amdgcn_ballot_w64(over) != 0) {
                 rescale(max8(s2, -__builtin_inff()), group_max(over ? 1.f : 0.f) > 0.f);

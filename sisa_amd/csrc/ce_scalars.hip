@@ -1,8 +1,8 @@
 // The two scalars around the linear cross-entropy's kernels: the valid-row count with its reciprocal, and the mean loss.
 // Reference: src/sisa/kernels/linear_ce.py:138-191 (n_valid, the loss sum). One workgroup each: at the row counts a
 // call has, a few thousand 4- or 8-byte values, the six torch launches they replace (compare, sum, cast, reciprocal;
-// sum, divide) cost 4 to 5 us apiece and nothing else: 1,023 rows of 512 366 -> 338 us a
-// training pass, 4,094 rows of 1,024 443 -> 426 us an evaluation.
+// sum, divide) cost 4 to 5 us apiece and nothing else: evaluations of 1,023 rows of 512 120 -> 107 us, of 4,096 258 -> 249,
+// of 16,384 793 -> 784. Callers bring at most 65,536 rows; beyond, one workgroup's loads cost more than the launches.
 #include "common.h"
 #include "host.h"
 #include "sisa_hip_ce.h"

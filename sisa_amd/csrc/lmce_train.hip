@@ -26,12 +26,12 @@
 // Rounding: p~ once, then G; bf16's dx only p~, its label terms exact to fp32. A label's G, p - 1 times s_n, keeps
 // its relative precision where p is near 1 (taken from the products of two rounded numbers, dx was off by 20 % of its
 // norm and dW by 29 % for rows with 1 - p near 0.008).
-// At 16,384 rows of 768 (V 50,277) the gradient launch takes 2,737 us in bf16 (0.93 PFLOP/s) and took 3,209 formed as
-// fp16's is; 175 and 204 us at 1,023 rows of 512.
+// At 16,384 rows of 768 (V 50,277) the gradient launch takes 2,585-2,650 us in bf16 (0.97 PFLOP/s; 2,730 with the row values
+// of a stage waited for ahead of its MFMAs) and took 3,209 formed as fp16's is; 173 us at 1,023 rows of 512, and 204.
 // G and the logits are never written to memory; the only large buffer is the chunk's exponentials (read once per
 // output column tile). Deterministic: no atomics.
 //
-// Tile arithmetic: a workgroup of 2 x 4 waves, two waves per SIMD (249 VGPRs); a wave owns 128 hidden x 64 rows
+// Tile arithmetic: a workgroup of 2 x 4 waves, two waves per SIMD (241 VGPRs); a wave owns 128 hidden x 64 rows
 // (dx) or 128 hidden x 64 vocabulary (dW) as 8 x 4 blocks of v_mfma_f32_16x16x32 (128 accumulators; all 12 operand
 // fragments of a 32-deep step are read before its 32 MFMAs), hidden on the A side so that a lane's 4 results are 4
 // consecutive hidden values (16-byte stores). Exponentials to form G from are loaded into registers before a

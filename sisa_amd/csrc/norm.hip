@@ -14,7 +14,7 @@
 //
 // Work decomposition: a wave holds RB = 64 / HP rows (HP = the projection width padded to 16, 32 or 64) with NVL =
 // HP / 8 eight-element vectors per lane (lane l holds elements 8 c .. 8 c + 7, c = l + 64 i), so RB * NVL = 8 and
-// the row length is at most 512 NVL. For up to 16 outputs and rows of at most 1024 (a multiple of 64; see norm_on_mfma) the projection
+// the row length is at most 512 NVL. For up to 16 outputs and rows of at most 1024 (norm_on_mfma) the projection
 // and its adjoint run on the matrix cores: the workgroup's sixteen rows of n (of dz W_f) pass through LDS and each
 // wave forms a quarter of the columns with v_mfma_f32_16x16x4_f32 (norm_fwd_mfma_kernel, norm_bwd_mfma_kernel).
 // Otherwise a lane's RB * HP projection partial sums are reduced over the 64 lanes with a halving exchange (63

@@ -5,7 +5,7 @@
 // Reference: the block and its cached attention (src/sisa/modeling.py:171-199, 224-238, 288-291) at L = 1, computed
 // there by about seventy torch kernels per layer. With B rows the weights are read once and nothing else is large, so
 // what such a step costs is launches and memory latency, not arithmetic: 11 ms of host time per token for 2.9 ms of
-// kernels in the 152M model, against about 0.06 ms for its bytes; here 0.85 ms of host time for 0.55 ms of kernels. Rounding points are those of the modules: every
+// kernels in the 152M model, against about 0.06 ms for its bytes; here 0.73 ms of host time for 0.48 ms of kernels. Rounding points are those of the modules: every
 // projection is an fp32 sum rounded once to the weights' dtype (biases added before it), the norm's rows, the
 // residual sums and the activation are rounded once, the forget logits stay fp32, the gates and the rotation are fp32.
 //

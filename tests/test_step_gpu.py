@@ -39,9 +39,9 @@ def _watched(model):
     return [blk.attn.W_Q.register_forward_hook(lambda *a: None) for blk in model.layers]
 
 
-# prompts of 1 to 1,105 rows (tiles of 128, remainders of 1 to 127); rows: one, two and four column groups of the products and their edges; widths below and above eight 32-element steps,
-# a head count that is not a multiple of the 16-row groups' 16; hidden widths that are no multiple of 32, 16, 8 or 2;
-# prompts of one position, of a chunk's edge and past it
+# prompts of 1 to 1,105 rows (tiles of 128, remainders of 1 to 127); rows: one, two and four column groups of the products
+# and their edges; widths below and above eight 32-element steps, a head count that is not a multiple of the 16-row groups'
+# 16; hidden widths that are no multiple of 32, 16, 8 or 2; prompts of one position, of a chunk's edge and past it
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("B,H,d_ff,prompt,steps", [(1, 2, 256, 1, 3), (4, 12, 2744, 64, 3), (16, 3, 40, 5, 2),
