@@ -88,8 +88,8 @@ def step_weights(linears: list[dict], attn_norm, ffn_norm, H: int, x: Tensor) ->
     None unless each is a plain contiguous parameter of the block's shape in ``x``'s dtype on its device, 16-byte
     aligned where the kernels load it in vectors, with biases on the two gates only."""
     D, s, dtype, device = x.shape[-1], HIP_D_STATE, x.dtype, x.get_device()
-    q, k, v, b, c, theta, alpha, forget, o, gate, up, down = (p["weight"] for p in linears)
-    biases = [p["bias"] for p in linears]
+    q, k, v, b, c, theta, alpha, forget, o, gate, up, down = (p.get("weight") for p in linears)
+    biases = [p.get("bias") for p in linears]
     if gate is None or any(t is not None for i, t in enumerate(biases) if i not in (6, 7)):
         return None
     ff = gate.shape[0]

@@ -362,12 +362,12 @@ class SISABlock(nn.Module):
         if slab is None:
             native = (native and step.prefill_takes(B * L, D, ffn.w_gate.out_features) and mode != "sync"
                       and step.whole(x) and step.whole(res))
-            weights = native and step.step_weights(linears, n1._parameters["weight"], n2._parameters["weight"], H, x)
+            weights = native and step.step_weights(linears, n1._parameters.get("weight"), n2._parameters.get("weight"), H, x)
             if not weights:
                 return self._forward_hip(x, res, defer=True, cache=cache)
             return step.layer_prefill(x, res, *weights, lam, ffn.w_down.weight, (n1.eps, n2.eps), cache, at.layer_idx,
                                       mode == "async")
-        weights = step.step_weights(linears, n1._parameters["weight"], n2._parameters["weight"], H, x)
+        weights = step.step_weights(linears, n1._parameters.get("weight"), n2._parameters.get("weight"), H, x)
         if weights is None:
             return None
         slab = cache.room(at.layer_idx, 1, buf, slab.phi)

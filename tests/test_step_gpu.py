@@ -233,3 +233,35 @@ def test_calls_refused_by_size_or_type_cost_nothing_more(monkeypatch):
             model(ids[:rows, 8:8 + n], cache=cache)
             monkeypatch.undo()
         assert not looked, (rows, n, dtype)
+
+
+def _unregister(module):
+    """Its weight as a plain attribute, as wrappers that shard or flatten parameters leave it."""
+    w = module._parameters.pop("weight")
+    module.__dict__["weight"] = w.detach()
+    return w
+
+
+def test_step_weights_of_unregistered_parameters():
+    from sisa_amd.kernels import step
+    model = tiny_model(seed=1).to(torch.bfloat16)
+    blk, x = model.layers[0], torch.zeros(1, 1, 128, dtype=torch.bfloat16)
+
+    def parts():
+        return (step.plain_linears(blk.attn._modules, blk.ffn._modules), blk.attn_norm.weight, blk.ffn_norm.weight, 2, x)
+    assert parts()[0] is not None
+    _unregister(blk.ffn.w_down)
+    assert step.step_weights(*parts()) is None
+    _unregister(blk.attn.alpha_proj)
+    assert step.step_weights(*parts()) is None
+
+
+@pytest.mark.gpu
+def test_generation_with_unregistered_parameters():
+    ids = token_ids(2, 5, seed=6).to(DEV)
+    for of in (lambda b: b.ffn.w_gate, lambda b: b.attn_norm, lambda b: b.attn.W_Q):
+        model = tiny_model(seed=6, theta_scale=0.25, attn_impl="auto").to(DEV).to(torch.bfloat16).eval()
+        want, _ = _decode(model, ids, 3)
+        _unregister(of(model.layers[0]))
+        got, _ = _decode(model, ids, 3)
+        assert rel_err(got, want) <= 2.0 ** -5        # another route in 16 bits, not other values
