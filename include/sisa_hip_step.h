@@ -74,7 +74,7 @@ typedef struct {
     sisa_view k, v, b, g, f;           /* cache slabs (B,H,capacity,64|64|32) in dtype, (B,H,capacity) fp32 */
     float* phi;                        /* (B,H,16) contiguous: phase at position L - 1 */
     void *h, *act, *ffn;               /* (B*L, D), (B*L, act_ld), (B*L, D) */
-    int64_t act_ld;                    /* FF rounded up to a multiple of 64 */
+    int64_t act_ld;                    /* FF rounded up to a multiple of 64; act, like each weight, spans less than 2 GiB */
     unsigned char* rise_ok;
     void* workspace;                   /* sisa_prefill_workspace_bytes(B,L,H), 256-byte aligned */
 } sisa_prefill_args;

@@ -265,3 +265,31 @@ def test_generation_with_unregistered_parameters():
         _unregister(of(model.layers[0]))
         got, _ = _decode(model, ids, 3)
         assert rel_err(got, want) <= 2.0 ** -5        # another route in 16 bits, not other values
+
+
+# more heads than the 16 and 32 outputs of the norm kernels' narrower forms, head counts that are no multiple of the four
+# outputs a lane stores at once, the widest model; prompts at the line from which wide models take the library's products
+@pytest.mark.gpu
+@pytest.mark.parametrize("H,d_ff,B,L", [(17, 200, 2, 70), (33, 329, 3, 5), (64, 264, 1, 130), (24, 136, 1, 2730)])
+def test_prompts_of_wide_models(H, d_ff, B, L, monkeypatch):
+    model = tiny_model(seed=H, theta_scale=0.25, attn_impl="auto", n_head=H, d_model=64 * H, d_ff=d_ff).to(DEV).to(
+        torch.bfloat16).eval()
+    ids = token_ids(B, L, seed=H).to(DEV)
+    calls = _count(monkeypatch)
+    got, cache = _decode(model, ids, L)
+    assert calls["sisa_prefill"] == 2
+    hooks = _watched(model)
+    calls.clear()
+    want, kept = _decode(model, ids, L)
+    assert "sisa_prefill" not in calls
+    for h in hooks:
+        h.remove()
+    ref = M64.logits64(model, M64.params64(model, requires_grad=False), ids)
+    # both round the same quantities to bf16: neither is further from fp64 than the other by more than the spread of such
+    # errors
+    assert rel_err(got, ref) <= 1.25 * rel_err(want, ref) + 1e-3
+    for layer in range(2):
+        a, b = cache.get(layer), kept.get(layer)
+        assert a.length == b.length == L
+        # the first layer's entries are projections of the same rows: two roundings to bf16 each side
+        assert layer or all(rel_err(getattr(a, n), getattr(b, n)) <= 4 * 2.0 ** -8 for n in ("k", "v", "g", "fgate", "phi"))
