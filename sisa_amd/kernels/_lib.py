@@ -198,6 +198,9 @@ STEP_SIGNATURES = {
 CE_SIGNATURES = {
     "sisa_ce_count": ([c_void_p, c_int64, c_int64, c_void_p, c_void_p, c_void_p], c_int),
     "sisa_ce_mean": ([c_void_p, c_int64, c_void_p, c_void_p, c_void_p], c_int),
+    "sisa_ce_workspace_bytes": ([c_int64], c_int64),
+    "sisa_ce_count_wide": ([c_void_p, c_int64, c_int64, c_void_p, c_void_p, c_void_p, c_void_p], c_int),
+    "sisa_ce_mean_wide": ([c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_void_p], c_int),
 }
 
 _LOCK = threading.Lock()

@@ -47,10 +47,9 @@ HIDDEN_MULTIPLE = 64             # the CE kernels stream the hidden size in 64-w
 PROBS_LIMIT = 0x7fffff00         # bytes that a chunk's stored exponentials may take: the kernels address them by 32-bit
                                  # offsets and drop what lies at 0x7ffffff0
 PROBS_BUDGET = 2 << 30           # bytes of one chunk of stored exponentials, within that
-SCALAR_ROWS = 1 << 16            # rows up to which one workgroup counts the valid ones and averages the loss, where the
-                                 # launches of the general sums cost more than its loads (evaluations of rows of 64 at 1,003
-                                 # tokens, us: 32,768 rows 54 and 65, 65,536 79 and 85, 98,304 128 and 115, 131,072 156
-                                 # and 114)
+SCALAR_ROWS = 1 << 15            # rows up to which one workgroup counts the valid ones and averages the loss: the second
+                                 # launch of several costs more below (32,768 rows of 64 at 1,003 tokens evaluated 57 and
+                                 # 71 us, 49,152 74 and 71, 65,536 81 and 70, 131,072 155 and 95)
 
 
 # ------------------------------------------------------------------------------------------------ pieces
@@ -163,21 +162,25 @@ class _Problem:
         self.N, self.D = self.x.shape[0], D
         self.n_valid, self.inv_n = self._count()
 
-    def _count(self) -> tuple[torch.Tensor, torch.Tensor | None]:
-        """The number of valid rows and its reciprocal, fp32 device scalars of one element; of more rows than one
-        workgroup counts, the int64 number alone (an evaluation needs no more)."""
-        if self.N > SCALAR_ROWS:
-            return (self.labels != self.ignore_index).sum(), None
+    def _scalar(self, name: str, values: torch.Tensor, *rest) -> None:
+        """``name`` over the call's rows, in its wide form where they are more than one workgroup takes well. (No torch
+        sum on either way: it records a memset, which a captured call must not.)"""
+        if self.N <= SCALAR_ROWS:
+            _lib.call_values(name, values, values.data_ptr(), self.N, *rest)
+            return
+        ws = torch.empty(_lib.workspace_bytes("sisa_ce_workspace_bytes", self.N) // 8, dtype=torch.int64,
+                         device=values.device)
+        _lib.call_values(name + "_wide", values, values.data_ptr(), self.N, *rest, ws.data_ptr())
+
+    def _count(self) -> tuple[torch.Tensor, torch.Tensor]:
+        """The number of valid rows and its reciprocal, fp32 device scalars of one element."""
         n_valid, inv_n = torch.empty(2, dtype=torch.float32, device=self.x.device).split(1)
-        _lib.call_values("sisa_ce_count", self.labels, self.labels.data_ptr(), self.N, self.ignore_index,
-                         n_valid.data_ptr(), inv_n.data_ptr())
+        self._scalar("sisa_ce_count", self.labels, self.ignore_index, n_valid.data_ptr(), inv_n.data_ptr())
         return n_valid, inv_n
 
     def _mean(self, rows: torch.Tensor) -> torch.Tensor:
-        if self.N > SCALAR_ROWS:
-            return rows.sum() / self.n_valid
         mean = torch.empty((), dtype=torch.float32, device=rows.device)
-        _lib.call_values("sisa_ce_mean", rows, rows.data_ptr(), self.N, self.n_valid.data_ptr(), mean.data_ptr())
+        self._scalar("sisa_ce_mean", rows, self.n_valid.data_ptr(), mean.data_ptr())
         return mean
 
     def loss_without_grad(self) -> torch.Tensor:
@@ -192,12 +195,11 @@ class _Problem:
         dx = torch.empty((N, Dp), dtype=torch.float32, device=dev) if want_dx else None
         dw = (torch.zeros if N == 0 else torch.empty)((Vp, Dp), dtype=torch.float32, device=dev) if want_dw else None
         step = chunk_rows(N, Vp, chunk_tokens, self.wpad.element_size())
-        inv_n = torch.reciprocal(self.n_valid.to(torch.float32)).reshape(1) if self.inv_n is None else self.inv_n
         if N:
             ws = train_workspace({min(step, N), N - (N - 1) // step * step}, Vp, Dp, dev)   # this loop's chunk sizes
             for r0 in range(0, N, step):
                 r1 = min(N, r0 + step)
-                lmce_train_chunk(self.x[r0:r1], self.wpad, self.labels[r0:r1], self.V, self.ignore_index, inv_n,
+                lmce_train_chunk(self.x[r0:r1], self.wpad, self.labels[r0:r1], self.V, self.ignore_index, self.inv_n,
                                  gscale, rows[r0:r1], None if dx is None else dx[r0:r1], dw, r0 > 0, ws)
         if dx is not None and Dp != self.D:
             dx = dx[:, :self.D]

@@ -236,9 +236,64 @@ def test_a_row_that_is_not_finite(bad):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("N", [1 << 16, (1 << 16) + 1])
+@pytest.mark.parametrize("N", [1, 63, 8192, 8193, 65537, 131071, 8192 * 256, 8192 * 256 + 1, 5000001])
+def test_wide_scalars(N):
+    """Remainders of the workgroups' 8,192 rows, as many workgroups as there may be, and two batches each."""
+    from sisa_amd.kernels import _lib
+    gen = torch.Generator().manual_seed(N)
+    lab = torch.randint(-1, 3, (N,), generator=gen).to(DEV)
+    rows = (10 + torch.randn(N, generator=gen)).to(DEV)
+    n, inv, mean, one = torch.empty(4, device=DEV).split(1)
+    size = _lib.workspace_bytes("sisa_ce_workspace_bytes", N)
+    assert 8 <= size <= 8 * 256
+    ws = torch.full((size // 8 + 1,), -7, dtype=torch.int64, device=DEV)
+    _lib.call_values("sisa_ce_count_wide", n, lab.data_ptr(), N, -1, n.data_ptr(), inv.data_ptr(), ws.data_ptr())
+    _lib.call_values("sisa_ce_mean_wide", n, rows.data_ptr(), N, n.data_ptr(), mean.data_ptr(), ws.data_ptr())
+    _lib.call_values("sisa_ce_mean", n, rows.data_ptr(), N, n.data_ptr(), one.data_ptr())
+    assert int(ws[-1]) == -7
+    count = int((lab != -1).sum())
+    assert float(n) == count and torch.equal(inv, torch.reciprocal(n))
+    want = rows.double().sum() / count
+    if count:       # one rounding of the sum, one of the quotient
+        assert abs(float(mean) - float(want)) <= 2 * 2.0 ** -24 * abs(float(want))
+        assert torch.equal(mean, one)               # fp64 sums round to fp32 alike in any order
+
+
+@pytest.mark.gpu
+def test_scalars_in_a_captured_call():
+    """Training and evaluation of more rows than one workgroup counts, replayed between eager work, give the eager bits."""
+    from sisa_amd.kernels.linear_ce import linear_cross_entropy
+    x, w, lab = _case((1 << 16) + 77, 64, 130, 5)
+    w, other = w.float(), lab.roll(1)
+
+    def both(labels):
+        xg, wg = x.detach().requires_grad_(True), w.detach().requires_grad_(True)
+        loss = linear_cross_entropy(xg, wg, labels)
+        dx, dw = torch.autograd.grad(loss, (xg, wg))
+        with torch.no_grad():
+            return loss.detach(), dx, dw, linear_cross_entropy(x, w, labels)
+    eager = [t.clone() for t in both(lab)]
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        both(lab)
+    torch.cuda.current_stream().wait_stream(side)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        outs = both(lab)
+    for _ in range(4):
+        both(other)
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip(outs, eager))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("N", [1 << 15, (1 << 15) + 1])
 def test_rows_at_the_line_of_the_scalar_kernels(N):
-    """One workgroup counts and averages up to 65,536 rows; beyond, the general sums do. Both against float64."""
+    """One workgroup counts and averages up to 32,768 rows, several beyond. Both against float64."""
     from sisa_amd.kernels.linear_ce import linear_cross_entropy
     x, w, lab = _case(N, 64, 130, 3)
     got, ref = _run(x, w, lab), _truth(x, w, lab)
