@@ -248,9 +248,10 @@ def ptr(t: torch.Tensor | None):
 def device_index(t: torch.Tensor) -> int:
     """The index of the GPU that holds ``t``; ``ValueError`` for a tensor elsewhere (entering its device, -1, would do
     nothing, and a kernel would read host addresses)."""
-    if not t.is_cuda:
+    index = t.get_device()
+    if index < 0:
         raise ValueError(f"the HIP kernels take tensors on a GPU, got one on {t.device}")
-    return t.get_device()
+    return index
 
 
 def stream_of(t: torch.Tensor) -> int:
