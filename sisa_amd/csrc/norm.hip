@@ -202,9 +202,10 @@ constexpr int NQ_SMALL = 12, NQ_LARGE = MFMA_DMAX / 64;
 // many rows longer than 768 with few outputs, which are bound by memory, the larger register set and the LDS trip cost
 // more than they save. 65,536 rows of 832, forward, vector and matrix, us: 69.7 and 75.0 with 1 output, 74.3 and 77.7 with 4,
 // 81.8 and 79.4 with 8; backward 199.9 and 206.4, 202.6 and 207.2, 206.5 and 209.4, and 213.0 and 212.1 with 12. Below 16,384
-// rows the matrix kernels are the faster ones with any.
-inline bool norm_on_mfma(const sisa_norm_args* a) {
-    return a->H > 0 && a->D % 64 == 0 && a->D <= MFMA_DMAX && (a->D <= 64 * NQ_SMALL || a->H >= 12 || a->N < 16384);
+// rows the matrix kernels are the faster ones with any. Hence at least 8 outputs forward, 12 backward.
+inline bool norm_on_mfma(const sisa_norm_args* a, bool bwd) {
+    return a->H > 0 && a->D % 64 == 0 && a->D <= MFMA_DMAX &&
+           (a->D <= 64 * NQ_SMALL || a->H >= (bwd ? 12 : 8) || a->N < 16384);
 }
 constexpr int NL_PAD = 4;                       // row padding of the staged n: conflict-free 16-byte reads
 inline int64_t norm_mfma_lds_bytes(int D) { return (int64_t)16 * (D + NL_PAD) * (int64_t)sizeof(float); }
@@ -762,7 +763,7 @@ template <class TX, class TY, int HP>
 int launch_norm_hp(const sisa_norm_args* a, int bwd, hipStream_t st) {
     constexpr int RB = 64 / HP;
     if (!bwd) {
-        if (HP == 16 && norm_on_mfma(a)) {
+        if (HP == 16 && norm_on_mfma(a, false)) {
             const unsigned grid = (unsigned)sisa::cdiv(a->N, 16);
             const size_t lds = (size_t)norm_mfma_lds_bytes(a->D);
             if (a->D <= 64 * NQ_SMALL) norm_fwd_mfma_kernel<TX, TY, NQ_SMALL><<<grid, 64 * NORM_WAVES, lds, st>>>(*a);
@@ -777,7 +778,7 @@ int launch_norm_hp(const sisa_norm_args* a, int bwd, hipStream_t st) {
     const int64_t np = sisa::cdiv(a->N, NORM_RPW);
     const unsigned grid = (unsigned)sisa::cdiv(np, NORM_WAVES);
     const size_t lds = (size_t)norm_mfma_lds_bytes(a->D);
-    const bool mfma = HP == 16 && norm_on_mfma(a);
+    const bool mfma = HP == 16 && norm_on_mfma(a, true);
     if (mfma && a->D <= 64 * NQ_SMALL)
         norm_bwd_mfma_kernel<TX, TY, NQ_SMALL><<<grid, 64 * NORM_WAVES, lds, st>>>(*a, ws.dw_part);
     else if (mfma)
