@@ -334,8 +334,10 @@ class SISABlock(nn.Module):
         # Cheap conditions first: a call that keeps the module path pays for them in every layer. A forced implementation
         # that x does not meet raises in the module path, or not at all: a cached fp32 call runs the unfused kernels in
         # place of "hip_fused", and a decode step selects nothing.
-        if type(cache) is not SISACache or not self._norm_rows_ok(x) or backends.compute_dtype(x) not in _LOW_PRECISION \
-                or self.config.attn_impl not in ("auto", "hip_fused"):
+        if type(cache) is not SISACache or not self._norm_rows_ok(x) or self.config.attn_impl not in ("auto", "hip_fused"):
+            return None
+        autocast = torch.is_autocast_enabled("cuda")
+        if (torch.get_autocast_dtype("cuda") if autocast else x.dtype) not in _LOW_PRECISION:
             return None
         mods = self._modules
         at, ffn, n1, n2 = mods["attn"], mods["ffn"], mods["attn_norm"], mods["ffn_norm"]
@@ -343,14 +345,14 @@ class SISABlock(nn.Module):
             return None
         slab, mode = cache._slabs.get(at.layer_idx), backends.get_check_mode()
         (B, L, D), H = x.shape, self.config.n_head
-        if slab is not None and (L != 1 or B > step.MAX_ROWS or D > step.MAX_WIDTH or x.dtype not in _LOW_PRECISION):
+        if slab is not None and (autocast or L != 1 or B > step.MAX_ROWS or D > step.MAX_WIDTH):
             return None
         if not (step.unobserved(x) and step.plain(self, SISABlock) and step.plain(ffn, SwiGLU) and step.plain(n1, RMSNorm)
                 and step.plain(n2, RMSNorm)):
             return None
         lam = at.lambda_raw
-        native = (x.dtype in _LOW_PRECISION and not torch.is_autocast_enabled("cuda") and lam.dtype == torch.float32
-                  and lam.shape == (H,) and lam.get_device() == x.get_device() and lam.is_contiguous())
+        native = (not autocast and lam.dtype == torch.float32 and lam.shape == (H,)
+                  and lam.get_device() == x.get_device() and lam.is_contiguous())
         if slab is not None:
             buf = slab.buffers
             if not native or slab.filled < 1 or not step.rows_ok(x) or not step.whole(res) or buf["k"].dtype != x.dtype \
